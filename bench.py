@@ -166,7 +166,8 @@ def run_prefill(a):
         "data": "synthetic: seeded N(0,0.02) random-init weights, uniform random token ids",
         "config": {"workload": f"{a.workload}: GPT-2 {shape_name}, batch {B}, prefill {T} tokens, full logits",
                    "batch": B, "tokens": T, "weights": "f32"},
-        "roofline": {"bound": "mfma", "kernel": "whole prefill (gemm_lds_kernel dominant)",
+        "roofline": {"bound": "mfma", "kernel": "whole prefill (pair_gemm_kernel dominant: f32 products as three f16 MFMA products; "
+                               "frac is of the f32 MFMA peak)",
                      "achieved": round(achieved, 2), "peak": MFMA_FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / MFMA_FP32_PEAK_TFLOPS, 4), "flops_per_step": flops,
                      "traffic": None},

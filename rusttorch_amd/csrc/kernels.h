@@ -52,6 +52,10 @@ void launch_embed(hipStream_t s, const void* wte, int wtype, const float* wpe, c
 // Row LayerNorm (gpt2.rs:636-666), rows x d.
 void launch_layernorm(hipStream_t s, const float* x, const float* w, const float* b, float eps, int rows, int d,
                       float* out);
+// The same over rows of stride ldx, written as the pair GEMM's input
+// (gemm_pair.h): f16 pairs of LN(x) * scale. d % 32 == 0.
+void launch_layernorm_pair(hipStream_t s, const float* x, long ldx, const float* w, const float* b, float eps,
+                           int rows, int d, const float* scale, uint16_t* out);
 
 // Decode GEMV: y[b][n] = epi(sum_k x[b][k] * W[n][k]) for b < B (any B: more
 // than 16 sequences run as slices of 16).
@@ -77,7 +81,7 @@ void launch_finalize(hipStream_t s, int B, unsigned long long* keys, uint32_t* t
 void launch_keys_to_tokens(hipStream_t s, int B, unsigned long long* keys, uint32_t* token);
 void launch_reset_keys(hipStream_t s, int B, unsigned long long* keys);
 
-// Prefill GEMM on MFMA: C[M][N] = epi(A[M][K] * W[N][K]^T); C row stride ldc.
+// GEMM on f32 MFMA, for the models the pair GEMM (gemm_pair.h) does not take: C[M][N] = epi(A[M][K] * W[N][K]^T); C row stride ldc.
 // ws (ws_floats floats, may be null) holds split-k partial tiles: shapes with
 // too few output tiles to fill the GPU split k when it is large enough
 // (gemm_splitk_ws_floats), otherwise they run unsplit.
@@ -91,15 +95,15 @@ void launch_kv_append(hipStream_t s, const float* qkv, int S, int T, int past, K
 // Prefill c_attn: C = A W^T + bias with the k/v columns ([d, 3d)) of row
 // s*T + t written into the cache at position past + t instead of C (the
 // append of LayerKVCache::append, gpt2.rs:500-514, in the GEMM's epilogue).
-// Falls back to launch_gemm + launch_kv_append where the fused kernels do not
-// apply (they need K % 64 == 0, 16-byte aligned operands and more than 64
-// rows; f32 or bf16 weights).
+// Falls back to launch_gemm + launch_kv_append where no k split does that.
 void launch_gemm_qkv(hipStream_t s, const float* A, int lda, const void* W, int wtype, const float* bias, float* C,
                      long ldc, int M, int K, int S, int T, int past, KvDst kv, float* ws = nullptr,
                      size_t ws_floats = 0);
-// Prefill causal attention for S sequences of T new tokens at offset past.
+// Prefill causal attention for S sequences of T new tokens at offset past: f32
+// rows to out, or with pair set the pair GEMM's input (f16 pairs, scaled).
 void launch_attn_prefill(hipStream_t s, const float* qkv, int S, int T, int past, const float* kc, const float* vc,
-                         int n_head, int n_pos, int d, float* out);
+                         int n_head, int n_pos, int d, float* out, uint16_t* pair = nullptr,
+                         const float* scale = nullptr);
 
 // LayerNorm folded into the GEMV that follows it (computed once per model,
 // accumulated in double): for output row r of W^T[N][K],

@@ -12,7 +12,7 @@
 
 #include "argmax_key.h"
 #include "attn_core.h"
-#include "bf16_split.h"
+#include "f16_pair.h"
 #include "gelu.h"
 #include "kernels.h"
 
@@ -101,11 +101,15 @@ void launch_embed(hipStream_t s, const void* wte, int wtype, const float* wpe, c
 // LayerNorm (gpt2.rs:636-666): two-pass mean / variance, one block per row.
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                        const float* __restrict__ b, float eps, int d,
-                                                        float* __restrict__ out) {
+// PAIR: the row times scale goes out as f16 pairs (the pair GEMM's input)
+// instead of f32, the same bytes.
+template <bool PAIR>
+__global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict__ x, long ldx,
+                                                        const float* __restrict__ w, const float* __restrict__ b,
+                                                        float eps, int d, void* __restrict__ out,
+                                                        const float* __restrict__ scale) {
   __shared__ float red[16];
-  const float* row = x + (size_t)blockIdx.x * d;
+  const float* row = x + (size_t)blockIdx.x * ldx;
   float s = 0.f;
   for (int j = threadIdx.x; j < d; j += blockDim.x) s += row[j];
   const float mean = block_reduce<false>(s, red) / (float)d;
@@ -116,8 +120,18 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict_
   }
   const float var = block_reduce<false>(v, red) / (float)d;
   const float inv_std = 1.0f / sqrtf(var + eps);
-  for (int j = threadIdx.x; j < d; j += blockDim.x)
-    out[(size_t)blockIdx.x * d + j] = (row[j] - mean) * inv_std * w[j] + b[j];
+  for (int j = threadIdx.x; j < d; j += blockDim.x) {
+    const float y = (row[j] - mean) * inv_std * w[j] + b[j];
+    if (PAIR) {
+      unsigned hi, lo;
+      f16_split(y * scale[j], &hi, &lo);
+      uint16_t* p = static_cast<uint16_t*>(out) + pair_index(blockIdx.x, j, d);
+      p[0] = (uint16_t)hi;
+      p[32] = (uint16_t)lo;
+    } else {
+      static_cast<float*>(out)[(size_t)blockIdx.x * d + j] = y;
+    }
+  }
 }
 
 // The same two-pass LayerNorm with one wave per row (4 rows per workgroup)
@@ -130,25 +144,27 @@ constexpr int LNW_MAXC = 8;  // 16-byte chunks per lane: d <= 64 * 4 * 8
 // full-wave sum in every lane on DPP and permlane swaps (no LDS traffic)
 __device__ __forceinline__ float wave_sum_dpp(float v) { return xor32_sum_k(xor16_sum_k(row16_sum_k(v))); }
 
-template <int NU>
-__global__ __launch_bounds__(256) void layernorm_wave_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                             const float* __restrict__ b, float eps, int rows, int d,
-                                                             float* __restrict__ out) {
+template <int NU, bool PAIR>
+__global__ __launch_bounds__(256) void layernorm_wave_kernel(const float* __restrict__ x, long ldx,
+                                                             const float* __restrict__ w, const float* __restrict__ b,
+                                                             float eps, int rows, int d, void* __restrict__ out,
+                                                             const float* __restrict__ scale) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= rows) return;  // wave-uniform
-  const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * d);
+  const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * ldx);
   const int nc = d >> 2;  // 16-byte chunks of the row, NU per lane at most
   const float4* w4 = reinterpret_cast<const float4*>(w);
   const float4* b4 = reinterpret_cast<const float4*>(b);
   // the row, the gain and the bias in flight together (branch-free: chunks
   // past the row's end re-read its last chunk and are dropped)
-  float4 v[NU], gv[NU], bv[NU];
+  float4 v[NU], gv[NU], bv[NU], sv[PAIR ? NU : 1];
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     const int ch = min(lane + 64 * u, nc - 1);
     v[u] = xr[ch];
     gv[u] = w4[ch];
     bv[u] = b4[ch];
+    if (PAIR) sv[u] = reinterpret_cast<const float4*>(scale)[ch];
   }
   float sum = 0.f;
 #pragma unroll
@@ -167,34 +183,52 @@ __global__ __launch_bounds__(256) void layernorm_wave_kernel(const float* __rest
   }
   const float var = wave_sum_dpp(sq) / (float)d;
   const float inv_std = 1.0f / sqrtf(var + eps);
-  float4* orow = reinterpret_cast<float4*>(out + (size_t)row * d);
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     const int ch = lane + 64 * u;
     if (ch < nc) {
       const float4 g = gv[u], bi = bv[u];
-      orow[ch] = make_float4((v[u].x - mean) * inv_std * g.x + bi.x, (v[u].y - mean) * inv_std * g.y + bi.y,
+      float4 y = make_float4((v[u].x - mean) * inv_std * g.x + bi.x, (v[u].y - mean) * inv_std * g.y + bi.y,
                              (v[u].z - mean) * inv_std * g.z + bi.z, (v[u].w - mean) * inv_std * g.w + bi.w);
+      if (PAIR) {
+        const float4 sc = sv[PAIR ? u : 0];
+        y = make_float4(y.x * sc.x, y.y * sc.y, y.z * sc.z, y.w * sc.w);
+        pair_store4(static_cast<uint16_t*>(out), row, 4 * ch, d, y);
+      } else {
+        static_cast<float4*>(out)[(size_t)row * nc + ch] = y;
+      }
     }
   }
 }
 
+template <bool PAIR>
+static bool launch_layernorm_wave(hipStream_t s, const float* x, long ldx, const float* w, const float* b, float eps,
+                                  int rows, int d, void* out, const float* scale) {
+  if (d % 4 != 0 || d > 256 * LNW_MAXC) return false;
+  const dim3 grid((rows + 3) / 4);
+  switch ((d + 255) / 256) {
+    case 1: layernorm_wave_kernel<1, PAIR><<<grid, 256, 0, s>>>(x, ldx, w, b, eps, rows, d, out, scale); break;
+    case 2: layernorm_wave_kernel<2, PAIR><<<grid, 256, 0, s>>>(x, ldx, w, b, eps, rows, d, out, scale); break;
+    case 3: layernorm_wave_kernel<3, PAIR><<<grid, 256, 0, s>>>(x, ldx, w, b, eps, rows, d, out, scale); break;
+    case 4: layernorm_wave_kernel<4, PAIR><<<grid, 256, 0, s>>>(x, ldx, w, b, eps, rows, d, out, scale); break;
+    case 5: layernorm_wave_kernel<5, PAIR><<<grid, 256, 0, s>>>(x, ldx, w, b, eps, rows, d, out, scale); break;
+    case 6: layernorm_wave_kernel<6, PAIR><<<grid, 256, 0, s>>>(x, ldx, w, b, eps, rows, d, out, scale); break;
+    case 7: layernorm_wave_kernel<7, PAIR><<<grid, 256, 0, s>>>(x, ldx, w, b, eps, rows, d, out, scale); break;
+    default: layernorm_wave_kernel<8, PAIR><<<grid, 256, 0, s>>>(x, ldx, w, b, eps, rows, d, out, scale); break;
+  }
+  return true;
+}
+
 void launch_layernorm(hipStream_t s, const float* x, const float* w, const float* b, float eps, int rows, int d,
                       float* out) {
-  if (d % 4 == 0 && d <= 256 * LNW_MAXC) {
-    const dim3 grid((rows + 3) / 4);
-    switch ((d + 255) / 256) {
-      case 1: layernorm_wave_kernel<1><<<grid, 256, 0, s>>>(x, w, b, eps, rows, d, out); break;
-      case 2: layernorm_wave_kernel<2><<<grid, 256, 0, s>>>(x, w, b, eps, rows, d, out); break;
-      case 3: layernorm_wave_kernel<3><<<grid, 256, 0, s>>>(x, w, b, eps, rows, d, out); break;
-      case 4: layernorm_wave_kernel<4><<<grid, 256, 0, s>>>(x, w, b, eps, rows, d, out); break;
-      case 5: layernorm_wave_kernel<5><<<grid, 256, 0, s>>>(x, w, b, eps, rows, d, out); break;
-      case 6: layernorm_wave_kernel<6><<<grid, 256, 0, s>>>(x, w, b, eps, rows, d, out); break;
-      case 7: layernorm_wave_kernel<7><<<grid, 256, 0, s>>>(x, w, b, eps, rows, d, out); break;
-      default: layernorm_wave_kernel<8><<<grid, 256, 0, s>>>(x, w, b, eps, rows, d, out); break;
-    }
-  } else
-    layernorm_kernel<<<rows, 256, 0, s>>>(x, w, b, eps, d, out);
+  if (!launch_layernorm_wave<false>(s, x, d, w, b, eps, rows, d, out, nullptr))
+    layernorm_kernel<false><<<rows, 256, 0, s>>>(x, d, w, b, eps, d, out, nullptr);
+}
+
+void launch_layernorm_pair(hipStream_t s, const float* x, long ldx, const float* w, const float* b, float eps,
+                           int rows, int d, const float* scale, uint16_t* out) {
+  if (!launch_layernorm_wave<true>(s, x, ldx, w, b, eps, rows, d, out, scale))
+    layernorm_kernel<true><<<rows, 256, 0, s>>>(x, ldx, w, b, eps, d, out, scale);
 }
 
 // ---------------------------------------------------------------------------
@@ -708,19 +742,9 @@ __global__ __launch_bounds__(256) void gemm_kernel(const float* __restrict__ A, 
   }
 }
 
-// Prefill GEMM for f32 weights, K % 64 == 0: the same 128x128 tile and MFMA
-// arrangement, fed by LDS-direct loads (global_load_lds_dwordx4) through a
-// GL_NS-stage LDS ring, so no registers hold tiles in flight and three k-tiles
-// are in flight while one is computed.
-// - A stage holds the A and W tiles as 8 + 8 groups of 16 rows x 16 k (1 KiB,
-//   one load instruction each: lane i fills bytes [16i, 16i + 16) of its
-//   group). Lane i loads row r = i / 4 of the group, 4-float chunk
-//   c = (i % 4) ^ gl_swz(row): an XOR swizzle that makes the operand reads
-//   below conflict-free.
-// - k is permuted inside a tile: MFMA step s of lane half h (lane / 32) uses
-//   k = 8h + s, so a lane reads its 8 values of a row with two ds_read_b128.
-//   A and W use the same permutation, so the products are those of the plain
-//   order (the sum is taken over all 16 k of the tile either way).
+// LDS-direct loads in a ring of GL_NS stages (gemm_skinny_lds_kernel): rows of
+// 16 k (64 bytes), 16-byte chunks XOR-swizzled so that the operand reads hit
+// distinct banks.
 constexpr int GL_NS = 4;
 __device__ __forceinline__ int gl_swz(int row) { return (row >> 2) & 3; }
 
@@ -738,411 +762,6 @@ __device__ __forceinline__ void gl_dma16(const float* src, const float* lds_dst)
 template <int N>
 __device__ __forceinline__ void gl_wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-// One k-tile step of gemm_lds_kernel on stage ST. Each stage is its own LDS
-// array and the loop is unrolled over the four stages, so every LDS address
-// is a base plus an immediate offset (about 1% faster than one array indexed
-// by kt % 4).
-template <int ST>
-__device__ __forceinline__ void gl_step(int kt, int nk, float (&lds)[2][GBM * 16], float (&nxt)[2][GBM * 16],
-                                        const float* const (&asrc)[2], const float* const (&wsrc)[2], int wave,
-                                        const int (&aoff)[2][2], const int (&woff)[2][2], floatx16 (&acc)[2][2]) {
-  // tile kt has landed once at most the loads of the GL_NS - 2 later tiles
-  // (4 instructions each) are still outstanding; after the barrier every
-  // wave's loads of tile kt are in and no wave reads tile kt - 1 any more
-  if (kt + GL_NS - 2 < nk) gl_wait_barrier<(GL_NS - 2) * 4>();
-  else gl_wait_barrier<0>();
-  if (kt + GL_NS - 1 < nk) {
-    const int k = (kt + GL_NS - 1) * 16;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int g = 2 * wave + q;
-      gl_dma16(asrc[q] + k, &nxt[0][g * 256]);
-      gl_dma16(wsrc[q] + k, &nxt[1][g * 256]);
-    }
-  }
-  float4 a[2][2], b[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      a[i][c] = *reinterpret_cast<const float4*>(&lds[0][aoff[i][c]]);
-      b[i][c] = *reinterpret_cast<const float4*>(&lds[1][woff[i][c]]);
-    }
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const float4& av = a[i][s >> 2];
-        const float4& bv = b[j][s >> 2];
-        const int e = s & 3;
-        const float x = e == 0 ? av.x : e == 1 ? av.y : e == 2 ? av.z : av.w;
-        const float y = e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[i][j], 0, 0, 0);
-      }
-  }
-}
-
-// Epilogue of the 128x128 tile kernels: wave tile (wm, wn) of block (m0, n0)
-// in acc[i][j] (32x32 blocks, MFMA output layout), to ws[z] as a raw partial
-// tile when ws is set, else with the epilogue (bias, gelu, residual; with kv
-// set, c_attn's k / v columns go into the cache at (sequence, head, past + t)).
-template <int I = 2, int J = 2>
-__device__ __forceinline__ void gl_epilogue(const floatx16 (&acc)[I][J], int lane, int m0, int n0, int wm, int wn,
-                                            int z, const float* __restrict__ bias, float* __restrict__ C, long ldc,
-                                            int M, int N, int epi, const KvDst& kv, int kv_T, int kv_past,
-                                            float* __restrict__ ws) {
-  if (ws != nullptr) {
-    float* wz = ws + (size_t)z * M * N;
-#pragma unroll
-    for (int i = 0; i < I; ++i)
-#pragma unroll
-      for (int j = 0; j < J; ++j) {
-        const int n = n0 + wn + j * 32 + (lane & 31);
-        if (n >= N) continue;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          if (m < M) wz[(size_t)m * N + n] = acc[i][j][e];
-        }
-      }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < I; ++i) {
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const int n = n0 + wn + j * 32 + (lane & 31);
-      if (n >= N) continue;
-      const float bv = bias ? bias[n] : 0.f;
-      if (kv.k != nullptr && n >= kv.d) {
-        // k / v column of c_attn: into the cache at (sequence, head, past + t)
-        const int which = n >= 2 * kv.d, cc = n - kv.d - which * kv.d;
-        float* base = (which ? kv.v : kv.k) + (size_t)(cc >> 6) * kv.n_pos * 64 + (cc & 63);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          if (m < M) {
-            const int sq = m / kv_T, t = m - sq * kv_T;
-            base[((size_t)sq * kv.n_head * kv.n_pos + kv_past + t) * 64] = acc[i][j][e] + bv;
-          }
-        }
-        continue;
-      }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int m = m0 + wm + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-        if (m < M) {
-          float* cp = C + (size_t)m * ldc + n;
-          const float v = acc[i][j][e];
-          if (epi == EPI_BIAS) *cp = v + bv;
-          else if (epi == EPI_BIAS_GELU) *cp = gelu_new(v + bv);
-          else if (epi == EPI_BIAS_RESID) *cp = *cp + (v + bv);
-          else *cp = v;
-        }
-      }
-    }
-  }
-}
-
-__global__ __launch_bounds__(256) void gemm_lds_kernel(const float* __restrict__ A, int lda,
-                                                       const float* __restrict__ W, const float* __restrict__ bias,
-                                                       float* __restrict__ C, long ldc, int M, int N, int K, int epi,
-                                                       int m_fast, KvDst kv, int kv_T, int kv_past, int ks,
-                                                       float* __restrict__ ws) {
-  __shared__ __attribute__((aligned(16))) float st0[2][GBM * 16];
-  __shared__ __attribute__((aligned(16))) float st1[2][GBM * 16];
-  __shared__ __attribute__((aligned(16))) float st2[2][GBM * 16];
-  __shared__ __attribute__((aligned(16))) float st3[2][GBM * 16];
-  static_assert(GL_NS == 4, "four stage arrays");
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  // block order: with m_fast the row blocks of one W column block are
-  // consecutive (W read once while A cycles through the cache), else the
-  // column blocks of one A row block (A read once while W cycles)
-  // with ks > 1 the k range is split: block b handles tile b % (nmb * nnb)
-  // over k-split z = b / (nmb * nnb) and stores its raw partial tile to
-  // ws[z] (summed and finished by splitk_reduce_kernel)
-  const int nmb = (M + GBM - 1) / GBM, nnb = (N + GBN - 1) / GBN;
-  const int bid = blockIdx.x % (nmb * nnb), z = blockIdx.x / (nmb * nnb);
-  const int m0 = (m_fast ? bid % nmb : bid / nnb) * GBM, n0 = (m_fast ? bid / nmb : bid % nnb) * GBN;
-  const int nk = K / 16 / ks;  // k-tiles of this split, a multiple of GL_NS
-
-  // this lane's load sources: groups 2*wave and 2*wave + 1 of A and of W
-  const int lr = lane >> 2;
-  const float* asrc[2];
-  const float* wsrc[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int row = (2 * wave + q) * 16 + lr;
-    const int c = (lane & 3) ^ gl_swz(row);
-    asrc[q] = A + (size_t)min(m0 + row, M - 1) * lda + c * 4 + (size_t)z * nk * 16;
-    wsrc[q] = W + (size_t)min(n0 + row, N - 1) * K + c * 4 + (size_t)z * nk * 16;
-  }
-  auto issue = [&](int kt, float (&st)[2][GBM * 16]) {
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int g = 2 * wave + q;
-      gl_dma16(asrc[q] + kt * 16, &st[0][g * 256]);
-      gl_dma16(wsrc[q] + kt * 16, &st[1][g * 256]);
-    }
-  };
-
-  // operand read offsets (floats within a stage's A or W tile): rows
-  // wm + 32i + lane % 32 (A) and wn + 32j + lane % 32 (W), chunks 2h, 2h + 1
-  const int h = lane >> 5;
-  int aoff[2][2], woff[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int ra = wm + 32 * i + (lane & 31), rw = wn + 32 * i + (lane & 31);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      aoff[i][c] = ra * 16 + (((2 * h + c) ^ gl_swz(ra)) * 4);
-      woff[i][c] = rw * 16 + (((2 * h + c) ^ gl_swz(rw)) * 4);
-    }
-  }
-
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  issue(0, st0);
-  issue(1, st1);
-  issue(2, st2);
-  for (int kt = 0; kt < nk; kt += GL_NS) {
-    gl_step<0>(kt, nk, st0, st3, asrc, wsrc, wave, aoff, woff, acc);
-    gl_step<1>(kt + 1, nk, st1, st0, asrc, wsrc, wave, aoff, woff, acc);
-    gl_step<2>(kt + 2, nk, st2, st1, asrc, wsrc, wave, aoff, woff, acc);
-    gl_step<3>(kt + 3, nk, st3, st2, asrc, wsrc, wave, aoff, woff, acc);
-  }
-
-  gl_epilogue(acc, lane, m0, n0, wm, wn, z, bias, C, ldc, M, N, epi, kv, kv_T, kv_past, ws);
-}
-
-// gemm_lds_kernel with 64 x 128 workgroup tiles (each wave 32 x 64, one A
-// group of 16 rows and two W groups per stage), for f32 GEMMs of at most 1024
-// rows: twice the workgroups of the 128 x 128 tiles, so fewer k splits and
-// reductions (c3's 512-row and c2's 1024-row prefill GEMMs: 5-25% faster
-// each, the split-k reduction included).
-constexpr int G64M = 64;
-template <int ST>
-__device__ __forceinline__ void g64_step(int kt, int nk, float (&la)[G64M * 16], float (&lw)[GBN * 16],
-                                         float (&na)[G64M * 16], float (&nw)[GBN * 16], const float* asrc,
-                                         const float* const (&wsrc)[2], int wave, const int (&aoff)[2],
-                                         const int (&woff)[2][2], floatx16 (&acc)[1][2]) {
-  if (kt + GL_NS - 2 < nk) gl_wait_barrier<(GL_NS - 2) * 3>();
-  else gl_wait_barrier<0>();
-  if (kt + GL_NS - 1 < nk) {
-    const int k = (kt + GL_NS - 1) * 16;
-    gl_dma16(asrc + k, &na[wave * 256]);
-#pragma unroll
-    for (int q = 0; q < 2; ++q) gl_dma16(wsrc[q] + k, &nw[(2 * wave + q) * 256]);
-  }
-  float4 a[2], b[2][2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    a[c] = *reinterpret_cast<const float4*>(&la[aoff[c]]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) b[j][c] = *reinterpret_cast<const float4*>(&lw[woff[j][c]]);
-  }
-#pragma unroll
-  for (int st = 0; st < 8; ++st) {
-    const float4& av = a[st >> 2];
-    const int e = st & 3;
-    const float x = e == 0 ? av.x : e == 1 ? av.y : e == 2 ? av.z : av.w;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const float4& bv = b[j][st >> 2];
-      const float y = e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w;
-      acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[0][j], 0, 0, 0);
-    }
-  }
-}
-
-__global__ __launch_bounds__(256) void gemm_lds64_kernel(const float* __restrict__ A, int lda,
-                                                         const float* __restrict__ W, const float* __restrict__ bias,
-                                                         float* __restrict__ C, long ldc, int M, int N, int K, int epi,
-                                                         int m_fast, KvDst kv, int kv_T, int kv_past, int ks,
-                                                         float* __restrict__ ws) {
-  __shared__ __attribute__((aligned(16))) float a0[G64M * 16], a1[G64M * 16], a2[G64M * 16], a3[G64M * 16];
-  __shared__ __attribute__((aligned(16))) float w0[GBN * 16], w1[GBN * 16], w2[GBN * 16], w3[GBN * 16];
-  static_assert(GL_NS == 4, "four stage arrays");
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
-  const int nmb = (M + G64M - 1) / G64M, nnb = (N + GBN - 1) / GBN;
-  const int bid = blockIdx.x % (nmb * nnb), z = blockIdx.x / (nmb * nnb);
-  const int m0 = (m_fast ? bid % nmb : bid / nnb) * G64M, n0 = (m_fast ? bid / nmb : bid % nnb) * GBN;
-  const int nk = K / 16 / ks;
-  const int lr = lane >> 2;
-  const float* asrc;
-  {
-    const int row = wave * 16 + lr;
-    const int c = (lane & 3) ^ gl_swz(row);
-    asrc = A + (size_t)min(m0 + row, M - 1) * lda + c * 4 + (size_t)z * nk * 16;
-  }
-  const float* wsrc[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int row = (2 * wave + q) * 16 + lr;
-    const int c = (lane & 3) ^ gl_swz(row);
-    wsrc[q] = W + (size_t)min(n0 + row, N - 1) * K + c * 4 + (size_t)z * nk * 16;
-  }
-  auto issue = [&](int kt, float (&la)[G64M * 16], float (&lw)[GBN * 16]) {
-    gl_dma16(asrc + kt * 16, &la[wave * 256]);
-#pragma unroll
-    for (int q = 0; q < 2; ++q) gl_dma16(wsrc[q] + kt * 16, &lw[(2 * wave + q) * 256]);
-  };
-  const int h = lane >> 5;
-  int aoff[2], woff[2][2];
-  {
-    const int ra = wm + (lane & 31);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) aoff[c] = ra * 16 + (((2 * h + c) ^ gl_swz(ra)) * 4);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int rw = wn + 32 * j + (lane & 31);
-#pragma unroll
-      for (int c = 0; c < 2; ++c) woff[j][c] = rw * 16 + (((2 * h + c) ^ gl_swz(rw)) * 4);
-    }
-  }
-  floatx16 acc[1][2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[0][j][e] = 0.f;
-  issue(0, a0, w0);
-  issue(1, a1, w1);
-  issue(2, a2, w2);
-  for (int kt = 0; kt < nk; kt += GL_NS) {
-    g64_step<0>(kt, nk, a0, w0, a3, w3, asrc, wsrc, wave, aoff, woff, acc);
-    g64_step<1>(kt + 1, nk, a1, w1, a0, w0, asrc, wsrc, wave, aoff, woff, acc);
-    g64_step<2>(kt + 2, nk, a2, w2, a1, w1, asrc, wsrc, wave, aoff, woff, acc);
-    g64_step<3>(kt + 3, nk, a3, w3, a2, w2, asrc, wsrc, wave, aoff, woff, acc);
-  }
-  gl_epilogue<1, 2>(acc, lane, m0, n0, wm, wn, z, bias, C, ldc, M, N, epi, kv, kv_T, kv_past, ws);
-}
-
-// gemm_lds_kernel for bf16 weights (the f32 activations times W stored as
-// bf16, gpt2.rs Conv1D with bf16-rounded weights upcast in the product): the
-// same 128x128 tiles, k-tiles of 16 and LDS-direct stage ring, with W's tile
-// as 128 rows of 32 bytes (one load instruction per wave: lane i fills row
-// 32 * wave + i / 2, 16-byte chunk (i % 2) ^ ((row >> 3) & 1)). Each lane's 8
-// A values of a 32-row block enter v_mfma_f32_32x32x16_bf16 as three exact
-// bf16 parts (split3), so every product is exact in f32 and the MFMA
-// accumulates in f32: the f32 GEMM up to summation order, at the bf16 rate.
-// Lane l holds A[row l % 32][k 8 (l / 32) .. + 8) and W[col l % 32][the same
-// k] of a tile, the A reads of gemm_lds_kernel.
-template <int ST>
-__device__ __forceinline__ void glb_step(int kt, int nk, float (&la)[GBM * 16], float (&lw)[GBM * 8],
-                                         float (&na)[GBM * 16], float (&nw)[GBM * 8], const float* const (&asrc)[2],
-                                         const uint16_t* wsrc, int wave, const int (&aoff)[2][2], const int (&woff)[2],
-                                         floatx16 (&acc)[2][2]) {
-  // tile kt has landed once at most the loads of the GL_NS - 2 later tiles
-  // (3 instructions each) are outstanding
-  if (kt + GL_NS - 2 < nk) gl_wait_barrier<(GL_NS - 2) * 3>();
-  else gl_wait_barrier<0>();
-  if (kt + GL_NS - 1 < nk) {
-    const int k = (kt + GL_NS - 1) * 16;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) gl_dma16(asrc[q] + k, &na[(2 * wave + q) * 256]);
-    gl_dma16(reinterpret_cast<const float*>(wsrc + k), &nw[wave * 256]);
-  }
-  u4v b[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const u4v*>(&lw[woff[j]]);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const float4 a0 = *reinterpret_cast<const float4*>(&la[aoff[i][0]]);
-    const float4 a1 = *reinterpret_cast<const float4*>(&la[aoff[i][1]]);
-    const float xs[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-    u4v xh, xm, xl;
-    split3(xs, xh, xm, xl);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const bf16x8 wb = as_bf16x8(b[j]);
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xh), wb, acc[i][j], 0, 0, 0);
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xm), wb, acc[i][j], 0, 0, 0);
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xl), wb, acc[i][j], 0, 0, 0);
-    }
-  }
-}
-
-__device__ __forceinline__ int glb_swz(int row) { return (row >> 3) & 1; }
-
-__global__ __launch_bounds__(256) void gemm_lds_bf16_kernel(const float* __restrict__ A, int lda,
-                                                            const uint16_t* __restrict__ W,
-                                                            const float* __restrict__ bias, float* __restrict__ C,
-                                                            long ldc, int M, int N, int K, int epi, int m_fast,
-                                                            KvDst kv, int kv_T, int kv_past, int ks,
-                                                            float* __restrict__ ws) {
-  __shared__ __attribute__((aligned(16))) float a0[GBM * 16], a1[GBM * 16], a2[GBM * 16], a3[GBM * 16];
-  __shared__ __attribute__((aligned(16))) float w0[GBM * 8], w1[GBM * 8], w2[GBM * 8], w3[GBM * 8];
-  static_assert(GL_NS == 4, "four stage arrays");
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  const int nmb = (M + GBM - 1) / GBM, nnb = (N + GBN - 1) / GBN;
-  const int bid = blockIdx.x % (nmb * nnb), z = blockIdx.x / (nmb * nnb);
-  const int m0 = (m_fast ? bid % nmb : bid / nnb) * GBM, n0 = (m_fast ? bid / nmb : bid % nnb) * GBN;
-  const int nk = K / 16 / ks;  // k-tiles of this split, a multiple of GL_NS
-
-  // load sources: A groups 2*wave and 2*wave + 1 (as gemm_lds_kernel), W rows
-  // 32*wave + lane / 2
-  const int lr = lane >> 2;
-  const float* asrc[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int row = (2 * wave + q) * 16 + lr;
-    const int c = (lane & 3) ^ gl_swz(row);
-    asrc[q] = A + (size_t)min(m0 + row, M - 1) * lda + c * 4 + (size_t)z * nk * 16;
-  }
-  const uint16_t* wsrc;
-  {
-    const int row = 32 * wave + (lane >> 1);
-    const int c = (lane & 1) ^ glb_swz(row);
-    wsrc = W + (size_t)min(n0 + row, N - 1) * K + c * 8 + (size_t)z * nk * 16;
-  }
-  auto issue = [&](int kt, float (&la)[GBM * 16], float (&lw)[GBM * 8]) {
-#pragma unroll
-    for (int q = 0; q < 2; ++q) gl_dma16(asrc[q] + kt * 16, &la[(2 * wave + q) * 256]);
-    gl_dma16(reinterpret_cast<const float*>(wsrc + kt * 16), &lw[wave * 256]);
-  };
-  // operand reads: A rows wm + 32i + lane % 32, chunks 2h and 2h + 1 (floats);
-  // W rows wn + 32j + lane % 32, chunk h (8 bf16 = 4 floats' bytes)
-  const int h = lane >> 5;
-  int aoff[2][2], woff[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int ra = wm + 32 * i + (lane & 31), rw = wn + 32 * i + (lane & 31);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) aoff[i][c] = ra * 16 + (((2 * h + c) ^ gl_swz(ra)) * 4);
-    woff[i] = rw * 8 + ((h ^ glb_swz(rw)) * 4);
-  }
-
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  issue(0, a0, w0);
-  issue(1, a1, w1);
-  issue(2, a2, w2);
-  for (int kt = 0; kt < nk; kt += GL_NS) {
-    glb_step<0>(kt, nk, a0, w0, a3, w3, asrc, wsrc, wave, aoff, woff, acc);
-    glb_step<1>(kt + 1, nk, a1, w1, a0, w0, asrc, wsrc, wave, aoff, woff, acc);
-    glb_step<2>(kt + 2, nk, a2, w2, a1, w1, asrc, wsrc, wave, aoff, woff, acc);
-    glb_step<3>(kt + 3, nk, a3, w3, a2, w2, asrc, wsrc, wave, aoff, woff, acc);
-  }
-  gl_epilogue(acc, lane, m0, n0, wm, wn, z, bias, C, ldc, M, N, epi, kv, kv_T, kv_past, ws);
 }
 
 // Skinny GEMM for few rows (a short prompt): the 128x128 tile kernel would
@@ -1335,7 +954,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny16_kernel(const float* __r
   }
 }
 
-// Prompt GEMM for 17..32 rows with f32 weights, K % 64 == 0: gemm_lds_kernel's
+// GEMM for 17..32 rows with f32 weights, K % 64 == 0, on an
 // LDS-direct ring (4 stages, XOR-swizzled 16-byte chunks, k permuted inside a
 // tile) with a 32 x 128 tile: the 32 rows of A and 128 rows of W (output
 // columns) per 16-k stage, wave w computing columns [32w, 32w + 32) with one
@@ -1548,8 +1167,8 @@ static bool launch_skinny(hipStream_t s, const float* A, int lda, const void* W,
   return true;
 }
 
-// Sum of the ks split-k partial tiles of gemm_lds_kernel (ws[z][m][n], in z
-// order) and the epilogue that kernel applies without a split (bias, gelu,
+// Sum of the ks split-k partial tiles of a GEMM (ws[z][m][n], in z order) and
+// the epilogue the kernel applies without a split (bias, gelu,
 // residual; with kv set, the k / v columns of c_attn go into the cache).
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int ks, int M, int N,
                                                             const float* __restrict__ bias, float* __restrict__ C,
@@ -1592,37 +1211,18 @@ static void splitk_reduce(hipStream_t s, const float* ws, int ks, int M, int N, 
                                                                       kv_past);
 }
 
-// k-splits of gemm_lds_kernel for an M x N x K GEMM: 1 when the output tiles
+// k-splits of gemm_kernel for an M x N x K GEMM: 1 when the output tiles
 // alone give enough workgroups (>= 192) or M < 128, else the smallest split
-// that gives >= 240 workgroups (each split a multiple of 4 k-tiles), or the
-// largest valid one up to 16. (Prefills of a few hundred rows otherwise run
-// their d-wide GEMMs on 32-48 of the 256 CUs.)
-// granule: k-tiles of 16 a split must hold a multiple of (GL_NS for
-// gemm_lds_kernel's stage ring, 1 for gemm_kernel).
-int gemm_splitk_factor(int M, int N, int K, int granule) {
+// that gives >= 240 workgroups, or the largest valid one up to 16.
+static int gemm_splitk_factor(int M, int N, int K) {
   const int tiles = ((M + GBM - 1) / GBM) * ((N + GBN - 1) / GBN);
-  if (M < 128 || tiles >= 192 || K % (16 * granule) != 0) return 1;
+  if (M < 128 || tiles >= 192 || K % 16 != 0) return 1;
   const int nk = K / 16;
   int best = 1;
   for (int s = 2; s <= 16; ++s) {
-    if (nk % (granule * s) != 0) continue;
+    if (nk % s != 0) continue;
     best = s;
     if (tiles * s >= 240) break;
-  }
-  return best;
-}
-
-// k-splits of gemm_lds64_kernel (M <= 1024): as gemm_splitk_factor, over its
-// 64 x 128 output tiles (and, as there, none below 128 rows).
-static int gemm64_splitk_factor(int M, int N, int K) {
-  const int tiles = ((N + GBN - 1) / GBN) * ((M + G64M - 1) / G64M);
-  if (M < 128 || M > 1024 || tiles >= 192 || K % (16 * GL_NS) != 0) return 1;
-  const int nkt = K / 16;
-  int best = 1;
-  for (int sp = 2; sp <= 16; ++sp) {
-    if (nkt % (GL_NS * sp) != 0) continue;
-    best = sp;
-    if (tiles * sp >= 240) break;
   }
   return best;
 }
@@ -1630,77 +1230,31 @@ static int gemm64_splitk_factor(int M, int N, int K) {
 size_t gemm_splitk_ws_floats(int M, int N, int K) {
   // the largest of the kernels' needs (which one runs depends on the weight
   // type, the row count and alignment)
-  const int ks = std::max(std::max(std::max(gemm_splitk_factor(M, N, K, GL_NS), gemm_splitk_factor(M, N, K, 1)),
-                                   std::max(skinny_splitk_factor(M, N, K), skinny_lds_splitk_factor(M, N, K))),
-                          gemm64_splitk_factor(M, N, K));
+  const int ks = std::max(gemm_splitk_factor(M, N, K),
+                          std::max(skinny_splitk_factor(M, N, K), skinny_lds_splitk_factor(M, N, K)));
   return ks > 1 ? (size_t)ks * M * N : 0;
-}
-
-static bool gemm_lds_ok(const float* A, int lda, const void* W, int wtype, int K) {
-  return K % 64 == 0 && lda % 4 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
-         (reinterpret_cast<uintptr_t>(W) & 15) == 0;
-}
-
-// gemm_lds_kernel (f32 W) or gemm_lds_bf16_kernel (bf16 W), split over k
-// when that fills the GPU and ws holds the partial tiles (ws_floats of them),
-// then the split-k reduction.
-static void launch_gemm_lds(hipStream_t s, const float* A, int lda, const void* W, int wtype, const float* bias,
-                            float* C, long ldc, int M, int N, int K, int epi, KvDst kv, int kv_T, int kv_past,
-                            float* ws, size_t ws_floats) {
-  const int nb = ((N + GBN - 1) / GBN) * ((M + GBM - 1) / GBM);
-  int ks = gemm_splitk_factor(M, N, K, GL_NS);
-  if (ks > 1 && (ws == nullptr || (size_t)ks * M * N > ws_floats)) ks = 1;
-  if (wtype == W_F32 && M <= 1024) {
-    // 64 x 128 tiles (gemm_lds64_kernel)
-    const int nb64 = ((N + GBN - 1) / GBN) * ((M + G64M - 1) / G64M);
-    int ks64 = gemm64_splitk_factor(M, N, K);
-    if (ks64 > 1 && (ws == nullptr || (size_t)ks64 * M * N > ws_floats)) ks64 = 1;
-    gemm_lds64_kernel<<<nb64 * ks64, 256, 0, s>>>(A, lda, static_cast<const float*>(W), bias, C, ldc, M, N, K, epi,
-                                                  N > M ? 1 : 0, kv, kv_T, kv_past, ks64, ks64 > 1 ? ws : nullptr);
-    if (ks64 > 1) splitk_reduce(s, ws, ks64, M, N, bias, C, ldc, epi, kv, kv_T, kv_past);
-    return;
-  }
-  float* wsk = ks > 1 ? ws : nullptr;
-  if (wtype == W_F32)
-    gemm_lds_kernel<<<nb * ks, 256, 0, s>>>(A, lda, static_cast<const float*>(W), bias, C, ldc, M, N, K, epi,
-                                            N > M ? 1 : 0, kv, kv_T, kv_past, ks, wsk);
-  else
-    gemm_lds_bf16_kernel<<<nb * ks, 256, 0, s>>>(A, lda, static_cast<const uint16_t*>(W), bias, C, ldc, M, N, K,
-                                                 epi, N > M ? 1 : 0, kv, kv_T, kv_past, ks, wsk);
-  if (ks > 1) splitk_reduce(s, ws, ks, M, N, bias, C, ldc, epi, kv, kv_T, kv_past);
 }
 
 void launch_gemm(hipStream_t s, const float* A, int lda, const void* W, int wtype, const float* bias, float* C,
                  long ldc, int M, int N, int K, int epi, float* ws, size_t ws_floats) {
   if (launch_skinny(s, A, lda, W, wtype, bias, C, ldc, M, N, K, epi, SkinnyQkv{}, ws, ws_floats)) return;
-  dim3 grid((N + GBN - 1) / GBN, (M + GBM - 1) / GBM);
-  if (gemm_lds_ok(A, lda, W, wtype, K))
-    // (256 x 128 tiles with 3 stages, bounded to two waves per SIMD, were 2-4%
-    // faster on the c4 shapes without an epilogue but made the c4 prefill
-    // slower, 70.7k against 72.5k tokens/s; 3 stages at three waves per SIMD
-    // and 2 stages at four were no faster than this kernel)
-    launch_gemm_lds(s, A, lda, W, wtype, bias, C, ldc, M, N, K, epi, KvDst{}, 1, 0, ws, ws_floats);
-  else {
-    int ks = gemm_splitk_factor(M, N, K, 1);
-    if (ks > 1 && (ws == nullptr || (size_t)ks * M * N > ws_floats)) ks = 1;
-    grid.z = ks;
-    float* wsk = ks > 1 ? ws : nullptr;
-    if (wtype == W_F32) gemm_kernel<W_F32><<<grid, 256, 0, s>>>(A, lda, W, bias, C, ldc, M, N, K, epi, ks, wsk);
-    else gemm_kernel<W_BF16><<<grid, 256, 0, s>>>(A, lda, W, bias, C, ldc, M, N, K, epi, ks, wsk);
-    if (ks > 1) splitk_reduce(s, ws, ks, M, N, bias, C, ldc, epi, KvDst{}, 1, 0);
-  }
+  int ks = gemm_splitk_factor(M, N, K);
+  if (ks > 1 && (ws == nullptr || (size_t)ks * M * N > ws_floats)) ks = 1;
+  const dim3 grid((N + GBN - 1) / GBN, (M + GBM - 1) / GBM, ks);
+  float* wsk = ks > 1 ? ws : nullptr;
+  if (wtype == W_F32) gemm_kernel<W_F32><<<grid, 256, 0, s>>>(A, lda, W, bias, C, ldc, M, N, K, epi, ks, wsk);
+  else gemm_kernel<W_BF16><<<grid, 256, 0, s>>>(A, lda, W, bias, C, ldc, M, N, K, epi, ks, wsk);
+  if (ks > 1) splitk_reduce(s, ws, ks, M, N, bias, C, ldc, epi, KvDst{}, 1, 0);
 }
 
 void launch_gemm_qkv(hipStream_t s, const float* A, int lda, const void* W, int wtype, const float* bias, float* C,
                      long ldc, int M, int K, int S, int T, int past, KvDst kv, float* ws, size_t ws_floats) {
   const int N = 3 * kv.d;
-  if (M > 64 && gemm_lds_ok(A, lda, W, wtype, K) && kv.d == 64 * kv.n_head) {
-    launch_gemm_lds(s, A, lda, W, wtype, bias, C, ldc, M, N, K, EPI_BIAS, kv, T, past, ws, ws_floats);
-    return;
-  }
   // a prompt of at most 64 rows: the split skinny GEMM's reduction writes the
-  // k / v columns into the cache itself
-  if (launch_skinny(s, A, lda, W, wtype, bias, C, ldc, M, N, K, EPI_BIAS, SkinnyQkv{}, ws, ws_floats, kv, T, past))
+  // k / v columns into the cache itself (head_dim 64)
+  if (kv.d == 64 * kv.n_head &&
+      launch_skinny(s, A, lda, W, wtype, bias, C, ldc, M, N, K, EPI_BIAS, SkinnyQkv{}, ws, ws_floats, kv, T,
+                    past))
     return;
   launch_gemm(s, A, lda, W, wtype, bias, C, ldc, M, N, K, EPI_BIAS, ws, ws_floats);
   launch_kv_append(s, C, S, T, past, kv);
@@ -1738,9 +1292,25 @@ constexpr int PQ = 64;   // queries per block (one wave)
 constexpr int PK = 64;   // keys per tile
 constexpr int HDM = 64;  // max head_dim
 
+// Where prefill attention writes: f32 rows out [rows][d], or with pair set the
+// pair GEMM's input, scaled by scale[column].
+struct AttnOut {
+  float* out;
+  uint16_t* pair;
+  const float* scale;
+};
+__device__ __forceinline__ void attn_put4(const AttnOut& o, size_t row, int col, int d, float4 v) {
+  if (o.pair != nullptr) {
+    const float4 sc = *reinterpret_cast<const float4*>(o.scale + col);
+    pair_store4(o.pair, row, col, d, make_float4(v.x * sc.x, v.y * sc.y, v.z * sc.z, v.w * sc.w));
+  } else {
+    *reinterpret_cast<float4*>(o.out + row * d + col) = v;
+  }
+}
+
 __global__ __launch_bounds__(64) void attn_prefill_kernel(const float* __restrict__ qkv, int T, int past,
                                                           const float* __restrict__ kc, const float* __restrict__ vc,
-                                                          int H, int P, int d, int hd, float* __restrict__ out) {
+                                                          int H, int P, int d, int hd, AttnOut out) {
   __shared__ float Ks[PK][HDM + 1];
   __shared__ float Vs[PK][HDM + 1];
   __shared__ float Ss[PQ][PK + 1];
@@ -1803,7 +1373,19 @@ __global__ __launch_bounds__(64) void attn_prefill_kernel(const float* __restric
   }
   if (active) {
     const float inv = 1.0f / l;
-    for (int dd = 0; dd < hd; ++dd) out[((size_t)sidx * T + i) * d + h * hd + dd] = o[dd] * inv;
+    const size_t row = (size_t)sidx * T + i;
+    for (int dd = 0; dd < hd; ++dd) {
+      const int col = h * hd + dd;
+      if (out.pair != nullptr) {
+        unsigned hi, lo;
+        f16_split(o[dd] * inv * out.scale[col], &hi, &lo);
+        uint16_t* p = out.pair + pair_index(row, col, d);
+        p[0] = (uint16_t)hi;
+        p[32] = (uint16_t)lo;
+      } else {
+        out.out[row * d + col] = o[dd] * inv;
+      }
+    }
   }
 }
 
@@ -1834,7 +1416,7 @@ constexpr int FA_VP = FA_K + 4;   // padded V^T row (floats)
 template <int FW>
 __global__ __launch_bounds__(64 * FW) void attn_prefill_mfma_kernel(
     const float* __restrict__ qkv, int T, int past, const float* __restrict__ kc, const float* __restrict__ vc,
-    int H, int P, int d, int nqb, float* __restrict__ out) {
+    int H, int P, int d, int nqb, AttnOut out) {
   constexpr int NT = 64 * FW, U = 512 / NT;  // threads; float4 of K (and of V) a thread stages per block
   __shared__ __attribute__((aligned(16))) float Ks[FA_K][FA_KP];
   __shared__ __attribute__((aligned(16))) float Vt[64][FA_VP];
@@ -1955,12 +1537,13 @@ __global__ __launch_bounds__(64 * FW) void attn_prefill_mfma_kernel(
   l = xor32_sum_k(l);
   if (qvalid) {
     const float inv = 1.0f / l;
-    float* orow = out + ((size_t)sidx * T + qi) * d + h * 64;
+    const size_t row = (size_t)sidx * T + qi;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = (i / 4) * 8 + hh * 4 + (i % 4);
-      orow[r] = o0[i] * inv;
-      orow[32 + r] = o1[i] * inv;
+    for (int g = 0; g < 4; ++g) {
+      const int col = h * 64 + 8 * g + 4 * hh;
+      attn_put4(out, row, col, d, make_float4(o0[4 * g] * inv, o0[4 * g + 1] * inv, o0[4 * g + 2] * inv, o0[4 * g + 3] * inv));
+      attn_put4(out, row, col + 32, d,
+                make_float4(o1[4 * g] * inv, o1[4 * g + 1] * inv, o1[4 * g + 2] * inv, o1[4 * g + 3] * inv));
     }
   }
 }
@@ -1976,7 +1559,7 @@ template <int KS>
 __global__ __launch_bounds__(64 * KS) void attn_prefill_ks_kernel(const float* __restrict__ qkv, int T, int past,
                                                                   const float* __restrict__ kc,
                                                                   const float* __restrict__ vc, int H, int P, int d,
-                                                                  int nqb, float* __restrict__ out) {
+                                                                  int nqb, AttnOut out) {
   constexpr int REG = FA_K * FA_KP + 64 * FA_VP;  // floats of one wave's K block and V^T block
   constexpr int MW = 64 + 2;                      // merge record of one query: m, l, O[64]
   static_assert(FA_QW * MW <= REG, "merge records fit the staging region");
@@ -2117,24 +1700,27 @@ __global__ __launch_bounds__(64 * KS) void attn_prefill_ks_kernel(const float* _
       L += sm[w][c * MW + 1] * f[w];
     }
     const float inv = 1.0f / L;
-    float* orow = out + ((size_t)sidx * T + qi) * d + h * 64;
+    const size_t row = (size_t)sidx * T + qi;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = (i / 4) * 8 + hh * 4 + (i % 4);
-      float a = 0.f, b = 0.f;
+    for (int g = 0; g < 8; ++g) {
+      const int r = (g & 3) * 8 + hh * 4 + (g >> 2) * 32;  // four consecutive dims
+      float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int w = 0; w < KS; ++w) {
-        a += sm[w][c * MW + 2 + r] * f[w];
-        b += sm[w][c * MW + 2 + 32 + r] * f[w];
+        const float* p = &sm[w][c * MW + 2 + r];
+        a.x += p[0] * f[w];
+        a.y += p[1] * f[w];
+        a.z += p[2] * f[w];
+        a.w += p[3] * f[w];
       }
-      orow[r] = a * inv;
-      orow[32 + r] = b * inv;
+      attn_put4(out, row, h * 64 + r, d, make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv));
     }
   }
 }
 
 void launch_attn_prefill(hipStream_t s, const float* qkv, int S, int T, int past, const float* kc, const float* vc,
-                         int n_head, int n_pos, int d, float* out) {
+                         int n_head, int n_pos, int d, float* out_rows, uint16_t* pair, const float* scale) {
+  const AttnOut out{out_rows, pair, scale};
   if (d / n_head == 64 && (long)n_head * S < 256 && T + past >= 4 * FA_K) {
     // few (sequence, head) pairs with long key ranges: split the keys over 4
     // waves, 8 from 16 key blocks on (c3, 512 tokens of GPT-2 medium: 85.4k

@@ -20,6 +20,7 @@
 #include "../../include/rtgpu.h"
 #include "decode_persistent.h"
 #include "bgemv.h"
+#include "gemm_pair.h"
 #include "kernels.h"
 #include "rows.h"
 #include "safetensors_reader.h"
@@ -103,6 +104,22 @@ struct BatchedWeights {
   }
 };
 
+// The weights as the prefill's pair GEMM reads them (gemm_pair.h), with the
+// scales of the inputs they multiply; built with the model.
+struct PrefillWeights {
+  void* arena = nullptr;
+  struct Layer {
+    PairWeights qkv, proj, fc, mproj;
+    const float *s1, *satt, *s2, *sh;  // input scales: LN1, attention output, LN2, gelu output
+  };
+  std::vector<Layer> layers;
+  PairWeights lm;              // wte
+  const float* sf = nullptr;   // scale of LN_f
+  ~PrefillWeights() {
+    if (arena) hipFree(arena);
+  }
+};
+
 struct rtg_model {
   rtg_config cfg;
   int hd = 0;
@@ -117,6 +134,7 @@ struct rtg_model {
   size_t nparams = 0;
   PersistentPlan* pplan = nullptr;
   RowsPlan* rplan = nullptr;  // multi-row forward (short prompts), null where unsupported
+  std::unique_ptr<PrefillWeights> pw;  // null where the f32-MFMA GEMMs run the prefill
   std::mutex bw_mu;
   std::unique_ptr<BatchedWeights> bw;
   // Pool of caches reused by the generate entry points (keyed by batch).
@@ -181,6 +199,17 @@ static void destroy_graph(rtg_cache* c) {
   c->graph = nullptr;
 }
 
+// Floats the layer GEMMs of a prefill over M rows use to split over k.
+static size_t prefill_ws_floats(const rtg_model* m, size_t M) {
+  const int d = (int)m->cfg.n_embd, planes = m->wtype == W_F32 ? 2 : 1;
+  size_t ws = 0;
+  for (const auto& nk : {std::make_pair(3 * d, d), std::make_pair(d, d), std::make_pair(4 * d, d),
+                         std::make_pair(d, 4 * d)})
+    ws = std::max(ws, m->pw ? pair_gemm_ws_floats((int)M, nk.first, nk.second, planes)
+                            : gemm_splitk_ws_floats((int)M, nk.first, nk.second));
+  return ws;
+}
+
 static void ensure_rows(rtg_cache* c, size_t rows) {
   if (rows <= c->rows_cap) return;
   destroy_graph(c);
@@ -195,12 +224,8 @@ static void ensure_rows(rtg_cache* c, size_t rows) {
   // the split-k workspace for the largest need of the four layer GEMMs at
   // any row count up to cap (the split depends on the row blocks)
   size_t ws = 0;
-  for (size_t r = 32; r < cap + 128; r += (r < 128 ? 32 : 128)) {
-    const int M = (int)std::min(r, cap);
-    for (const auto& nk : {std::make_pair(3 * d, d), std::make_pair(d, d), std::make_pair(4 * d, d),
-                           std::make_pair(d, 4 * d)})
-      ws = std::max(ws, gemm_splitk_ws_floats(M, (int)nk.first, (int)nk.second));
-  }
+  for (size_t r = 32; r < cap + 128; r += (c->m->pw || r < 128 ? 32 : 128))
+    ws = std::max(ws, prefill_ws_floats(c->m, std::min(r, cap)));
   if (ws) HIPX(hipMalloc(&c->ws, ws * 4));
   c->ws_floats = ws;
   c->rows_cap = cap;
@@ -282,12 +307,70 @@ static Work cache_work(const rtg_cache* c) {
 }
 
 // forward_cached body for S sequences x T new tokens (gpt2.rs:376-396) on the
+// pair GEMMs (gemm_pair.h): w.ln, w.att and w.h hold f16 pairs, 4 bytes per
+// element like the f32 rows they replace.
+static void enqueue_prefill_pair(rtg_cache* c, const Work& w, const uint32_t* ids_dev, size_t S, size_t T, size_t past,
+                                 int logit_mode) {
+  const rtg_model* m = c->m;
+  const PrefillWeights& pw = *m->pw;
+  const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, M = (int)(S * T);
+  const float eps = m->cfg.layer_norm_epsilon;
+  hipStream_t s = c->stream;
+  uint16_t *ln = reinterpret_cast<uint16_t*>(w.ln), *att = reinterpret_cast<uint16_t*>(w.att),
+           *h = reinterpret_cast<uint16_t*>(w.h);
+  auto args = [&](const uint16_t* A, int K, const float* bias, float* C, long ldc, int epi) {
+    PairGemmArgs a;
+    a.A = A;
+    a.lda = 2 * K;
+    a.M = M;
+    a.bias = bias;
+    a.C = C;
+    a.ldc = ldc;
+    a.epi = epi;
+    a.ws = w.ws;
+    a.ws_floats = w.ws_floats;
+    return a;
+  };
+  launch_embed(s, m->wte, m->wtype, m->wpe, ids_dev, M, (int)T, (int)past, nullptr, d, w.x);
+  for (size_t l = 0; l < m->layers.size(); ++l) {
+    const LayerW& L = m->layers[l];
+    const PrefillWeights::Layer& P = pw.layers[l];
+    KvDst kv = kv_layer(c, l);
+    launch_layernorm_pair(s, w.x, d, L.ln1w, L.ln1b, eps, M, d, P.s1, ln);
+    PairGemmArgs a = args(ln, d, L.bqkv, w.qkv, 3 * d, EPI_BIAS);
+    a.kv = kv;
+    a.kv_T = (int)T;
+    a.kv_past = (int)past;
+    launch_pair_gemm(s, P.qkv, a);
+    launch_attn_prefill(s, w.qkv, (int)S, (int)T, (int)past, kv.k, kv.v, kv.n_head, kv.n_pos, d, nullptr, att,
+                        P.satt);
+    launch_pair_gemm(s, P.proj, args(att, d, L.baproj, w.x, d, EPI_BIAS_RESID));
+    launch_layernorm_pair(s, w.x, d, L.ln2w, L.ln2b, eps, M, d, P.s2, ln);
+    a = args(ln, d, L.bfc, nullptr, 0, EPI_BIAS_GELU);
+    a.P = h;
+    a.p_scale = P.sh;
+    launch_pair_gemm(s, P.fc, a);
+    launch_pair_gemm(s, P.mproj, args(h, 4 * d, L.bmproj, w.x, d, EPI_BIAS_RESID));
+  }
+  // ln_f and the logits of every row, or of the last row of each sequence
+  const int rows = logit_mode == 0 ? M : (int)S;
+  const long ldx = logit_mode == 0 ? d : (long)T * d;
+  launch_layernorm_pair(s, w.x + (logit_mode == 0 ? 0 : (T - 1) * d), ldx, m->lnfw, m->lnfb, eps, rows, d, pw.sf, ln);
+  PairGemmArgs a = args(ln, d, nullptr, w.logits, V, EPI_NONE);
+  a.M = rows;
+  a.ws = nullptr;
+  launch_pair_gemm(s, pw.lm, a);
+  HIPX(hipGetLastError());
+}
+
+// forward_cached body for S sequences x T new tokens (gpt2.rs:376-396) on the
 // MFMA prefill path, on the activation buffers w. ids_dev holds S*T ids;
 // logits rows: all S*T (mode 0) or the last row of each sequence (mode 1,
 // written as S rows).
 static void enqueue_prefill(rtg_cache* c, const Work& w, const uint32_t* ids_dev, size_t S, size_t T, size_t past,
                             int logit_mode) {
   const rtg_model* m = c->m;
+  if (m->pw) return enqueue_prefill_pair(c, w, ids_dev, S, T, past, logit_mode);
   const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, M = (int)(S * T);
   const float eps = m->cfg.layer_norm_epsilon;
   hipStream_t s = c->stream;
@@ -831,6 +914,76 @@ static void generate_greedy(const rtg_model* m, const uint32_t* prompts, size_t 
 // Model construction (gpt2.rs:214-263)
 // ---------------------------------------------------------------------------
 
+// Builds the model's PrefillWeights. Left null where the pair GEMM does not
+// apply (n_embd not a multiple of 64, a negative epsilon), where a weight or a
+// bound of an activation is not finite, or where the copy does not fit the
+// device: the f32-MFMA GEMMs then run the prefill.
+static void build_prefill_weights(rtg_model* m) {
+  const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, L = (int)m->layers.size(), wt = m->wtype;
+  if (d % 64 != 0 || !(m->cfg.layer_norm_epsilon >= 0.f)) return;
+  std::unique_ptr<PrefillWeights> pw(new PrefillWeights());
+  struct Shape {
+    int N, K;
+  };
+  const Shape sh[4] = {{3 * d, d}, {d, d}, {4 * d, d}, {d, 4 * d}};
+  size_t total = 256;  // the flag
+  for (const Shape& x : sh) total += L * (align_up(pair_weight_bytes(x.N, x.K, wt), 256) + align_up(x.N * 4, 256));
+  total += L * (3 * align_up(d * 4, 256) + align_up(4 * d * 4, 256));
+  total += align_up(pair_weight_bytes(V, d, wt), 256) + align_up((size_t)V * 4, 256) + align_up(d * 4, 256);
+  if (hipMalloc(&pw->arena, total) != hipSuccess) {
+    hipGetLastError();
+    return;
+  }
+  char* p = static_cast<char*>(pw->arena);
+  auto take = [&](size_t n) {
+    char* r = p;
+    p += align_up(n, 256);
+    return r;
+  };
+  auto floats = [&](int n) { return reinterpret_cast<float*>(take((size_t)n * 4)); };
+  hipStream_t s = nullptr;
+  int* bad = reinterpret_cast<int*>(take(256));
+  HIPX(hipMemset(bad, 0, 4));
+  auto weights = [&](const void* W, int N, int K, const float* in_scale) {
+    PairWeights w;
+    w.planes = wt == W_F32 ? 2 : 1;
+    w.N = N;
+    w.K = K;
+    w.w = reinterpret_cast<uint16_t*>(take(pair_weight_bytes(N, K, wt)));
+    w.out_scale = floats(N);
+    launch_pair_weights(s, W, wt, in_scale, w, bad);
+    return w;
+  };
+  const size_t wb = wt == W_BF16 ? 2 : 4;
+  for (const LayerW& W : m->layers) {
+    PrefillWeights::Layer l;
+    float *s1 = floats(d), *satt = floats(d), *s2 = floats(d), *sh4 = floats(4 * d);
+    launch_pair_ln_scale(s, W.ln1w, W.ln1b, d, s1, bad);
+    launch_pair_ln_scale(s, W.ln2w, W.ln2b, d, s2, bad);
+    // attention averages value rows: the bound of c_attn's v outputs
+    launch_pair_row_scale(s, static_cast<const char*>(W.wqkv) + 2 * (size_t)d * d * wb, wt, d, d, W.ln1w, W.ln1b,
+                          W.bqkv + 2 * d, satt, bad);
+    launch_pair_row_scale(s, W.wfc, wt, 4 * d, d, W.ln2w, W.ln2b, W.bfc, sh4, bad);
+    l.s1 = s1;
+    l.satt = satt;
+    l.s2 = s2;
+    l.sh = sh4;
+    l.qkv = weights(W.wqkv, 3 * d, d, s1);
+    l.proj = weights(W.waproj, d, d, satt);
+    l.fc = weights(W.wfc, 4 * d, d, s2);
+    l.mproj = weights(W.wmproj, d, 4 * d, sh4);
+    pw->layers.push_back(l);
+  }
+  float* sf = floats(d);
+  launch_pair_ln_scale(s, m->lnfw, m->lnfb, d, sf, bad);
+  pw->sf = sf;
+  pw->lm = weights(m->wte, V, d, sf);
+  int flag = 0;
+  HIPX(hipGetLastError());
+  HIPX(hipMemcpy(&flag, bad, 4, hipMemcpyDeviceToHost));
+  if (flag == 0) m->pw = std::move(pw);
+}
+
 namespace {
 // A weight as the caller or the file holds it: f32, bf16 or f16 elements
 // (uploaded as they are and converted on the device), or an f32 decode on the
@@ -1001,6 +1154,7 @@ rtg_result build_model(const rtg_config* cfg, Lookup& lk, rtg_storage storage, r
     m->lnfb = reinterpret_cast<float*>(A + o_lnfb);
     HIPX(hipFree(staging));
     staging = nullptr;
+    build_prefill_weights(m.get());
   } catch (const HipError& he) {
     if (staging) hipFree(staging);
     return err(he.msg);  } catch (const std::exception& ex) {
@@ -1240,10 +1394,7 @@ rtg_result rtg_forward_cached_noalloc(const rtg_model* model, rtg_cache* cache, 
   const size_t pv = align_up(n * V, 64);
   // the split-k partial tiles the pass's GEMMs use at n rows (as much as the
   // cache's own workspace would hold for them, so the same kernels run)
-  size_t pw = 0;
-  for (const auto& nk : {std::make_pair(3 * d, d), std::make_pair(d, d), std::make_pair(4 * d, d),
-                         std::make_pair(d, 4 * d)})
-    pw = std::max(pw, gemm_splitk_ws_floats((int)n, (int)nk.first, (int)nk.second));
+  size_t pw = prefill_ws_floats(model, n);
   pw = align_up(pw, 64);
   const size_t need = 3 * pd + p3 + p4 + pv;
   if (need > kScratchFloats)

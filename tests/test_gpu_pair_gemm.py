@@ -1,0 +1,126 @@
+"""The prefill on f16-pair GEMMs (gemm_pair.hip) through forward_cached, against
+float64 (tests/ref64.py).
+
+The bar is the CPU oracle's own distance from float64 on the same model and
+ids (f32 throughout, sums in k order): the library may be at most twice as far
+in the 2-norm, plus 2e-7 (3 ulp of f32) where the oracle happens to be closer.
+bf16 storage is compared on weights that are bf16 values already.
+
+Shapes: one layer, chosen so that every tile of the dispatch and the k split
+occur (short and long M against wide and narrow N), with ragged M and V and
+head dims 64 and 32; a second chunk behind cached rows; widths above 2048
+(the block-per-row LayerNorm); weights and gains whose magnitudes spread over
+many powers of two; and weights for which the path is not taken at all.
+"""
+import numpy as np
+import pytest
+
+from rusttorch_amd import synth
+from rusttorch_amd.gpt2 import Gpt2Config, Gpt2Model
+from tests import ref64
+
+pytestmark = pytest.mark.gpu
+
+
+def build(sh, storage="f32", change=None):
+    sd = synth.make_weights(sh, bf16=storage == "bf16")
+    if change:
+        change(sd)
+    cfg = Gpt2Config(sh.vocab_size, sh.n_positions, sh.n_embd, sh.n_layer, sh.n_head, sh.layer_norm_epsilon)
+    return sd, Gpt2Model.from_state_dict(sd, cfg, storage=storage)
+
+
+def off(a, ref):
+    return float(np.linalg.norm(np.asarray(a, np.float64) - ref) / np.linalg.norm(ref))
+
+
+def check(oracle_lib, sh, sd, m, chunks, batch=1):
+    print(f"[gpu] pair gemm {sh} {m.storage} chunks {chunks} batch {batch}", flush=True)
+    total = sum(chunks)
+    ids = np.stack([synth.make_tokens(total, sh.vocab_size, stream=40 + b) for b in range(batch)])
+    c = m.new_cache(batch)
+    got, at = [], 0
+    for n in chunks:
+        got.append(m.forward_cached_batched(ids[:, at:at + n], c))
+        at += n
+    got = np.concatenate(got, axis=1)
+    om = oracle_lib.OracleModel.from_shape(sd, sh, threads=8)
+    for b in sorted({0, batch - 1}):
+        ref = ref64.forward(sd, ids[b], sh.n_layer, sh.n_head, sh.layer_norm_epsilon)
+        mine, plain = off(got[b], ref), off(om.forward(ids[b]), ref)
+        print(f"  sequence {b}: {mine:.2e} from float64, oracle {plain:.2e}", flush=True)
+        assert mine <= 2 * plain + 2e-7, (mine, plain)
+    c.close()
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+@pytest.mark.parametrize("d,heads,V,batch,chunks", [
+    (192, 3, 301, 1, (33,)),          # 32 x 64 tiles, split
+    (192, 6, 301, 3, (17,)),          # head_dim 32, 51 rows
+    (192, 3, 301, 5, (131, 7)),       # 655 rows, then 35 behind 131 cached
+    (768, 12, 515, 1, (65,)),
+    (768, 12, 515, 2, (161,)),
+    (768, 12, 515, 9, (129,)),        # 64 x 64 and 64 x 128 tiles
+    (1600, 25, 258, 16, (65,)),       # 128 x 128 tiles, K = 6400 split
+    (128, 2, 50257, 1, (999,)),       # a wide LM head over many rows: 256 x 256 tiles
+])
+def test_shapes(oracle_lib, storage, d, heads, V, batch, chunks):
+    sh = synth.ModelShape(V, 1024, d, 1, heads)
+    sd, m = build(sh, storage)
+    check(oracle_lib, sh, sd, m, chunks, batch)
+    m.close()
+
+
+def test_many_rows(oracle_lib):
+    """Enough rows that the layer GEMMs take the 256 x 256 and 128 x 128 tiles."""
+    sh = synth.ModelShape(130, 512, 640, 1, 10)
+    sd, m = build(sh)
+    check(oracle_lib, sh, sd, m, (403,), batch=32)
+    m.close()
+
+
+def test_wide_rows(oracle_lib):
+    sh = synth.ModelShape(70, 64, 2112, 1, 33)
+    sd, m = build(sh)
+    check(oracle_lib, sh, sd, m, (35,))
+    m.close()
+
+
+def test_spread_magnitudes(oracle_lib):
+    """Gains, weight rows and columns of very different sizes: the input and
+    row scales keep every pair as good as f32."""
+    def change(sd):
+        for k in ("h.0.ln_1.weight", "h.0.ln_2.weight", "ln_f.weight"):
+            sd[k][5] *= 3000.0
+            sd[k][7:40] *= 2.0 ** -14
+        for k, n in (("h.0.attn.c_attn.weight", 192), ("h.0.mlp.c_fc.weight", 192), ("h.0.mlp.c_proj.weight", 768)):
+            sd[k][:, 3::7] *= 2.0 ** -20
+            sd[k][n // 2:n // 2 + 9] *= 2.0 ** 9
+        sd["h.0.mlp.c_fc.bias"][::5] = 40.0
+        sd["wte.weight"][17] *= 2.0 ** 12
+    sh = synth.ModelShape(301, 256, 192, 1, 3)
+    sd, m = build(sh, change=change)
+    check(oracle_lib, sh, sd, m, (77, 120))
+    m.close()
+
+
+@pytest.mark.parametrize("what", ["nan bias", "inf weight", "negative epsilon"])
+def test_models_outside_the_bounds(oracle_lib, what):
+    """No finite bound, or an epsilon for which it does not hold: the f32 GEMMs
+    run, with the oracle's pattern of finite values."""
+    def change(sd):
+        if what == "nan bias":
+            sd["h.0.mlp.c_fc.bias"][3] = np.nan
+        if what == "inf weight":
+            sd["wte.weight"][9, 4] = np.inf  # one logit column
+    eps = -1e-9 if what == "negative epsilon" else 1e-5
+    sh = synth.ModelShape(301, 64, 192, 1, 3, eps)
+    sd, m = build(sh, change=change)
+    ids = synth.make_tokens(40, 300, stream=3)
+    ids[ids == 9] = 8
+    got = m.forward(ids)
+    ref = oracle_lib.OracleModel.from_shape(sd, sh, threads=8).forward(ids)
+    assert np.array_equal(np.isfinite(got), np.isfinite(ref))
+    fine = np.isfinite(ref)
+    assert np.all(np.abs(got[fine] - ref[fine]) <= 1e-3 + 1e-4 * np.abs(ref[fine]))
+    m.close()
