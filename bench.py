@@ -116,17 +116,20 @@ MFMA_FP32_PEAK_TFLOPS = 157.3
 MFMA_BF16_PEAK_TFLOPS = 2500.0
 BF16X3_PEAK_TFLOPS = MFMA_BF16_PEAK_TFLOPS / 3
 PREFILL_WORKLOADS = {
-    # name: (shape, batch, tokens): forward_cached on an empty cache, full [T, V] logits per sequence
+    # name: (shape, batch, tokens): forward_cached on an empty cache, prompts read without their logits
     "c4": ("large", 32, 1024),
 }
 
 
-def prefill_flops(sh, B, T):
+def prefill_flops(sh, B, T, head_rows=None):
     """Algorithmic flops of forward_cached over T new tokens on an empty
     cache: the four Conv1D GEMMs, causal QK^T and PV, and the LM head over
-    every row (the reference computes [T, V] logits)."""
+    head_rows rows per sequence (default every row: the [T, V] logits the
+    reference returns; 1 in generate, which reads the last row's; 0 for a
+    prompt read without logits)."""
     L, d, V = sh.n_layer, sh.n_embd, sh.vocab_size
-    return B * (2 * T * 12 * d * d * L + 4 * d * L * T * (T + 1) // 2 + 2 * T * d * V)
+    head = T if head_rows is None else head_rows
+    return B * (2 * T * 12 * d * d * L + 4 * d * L * T * (T + 1) // 2 + 2 * head * d * V)
 
 
 def run_prefill(a):
@@ -148,12 +151,12 @@ def run_prefill(a):
     for _ in range(a.steps):
         cache.clear()
         t0 = time.perf_counter()
-        m.forward_cached_batched(ids, cache, want_logits=False)  # logits stay in HBM
+        m.forward_cached_batched(ids, cache, want_logits=False)
         times.append(time.perf_counter() - t0)
     print("[bench] timed steps done", file=sys.stderr, flush=True)
     del m
     step_s = float(np.mean(times))
-    flops = prefill_flops(sh, B, T)
+    flops = prefill_flops(sh, B, T, 0)
     achieved = flops / step_s / 1e12
     out = {
         "metric": f"prefill tokens/s (GPT-2 {shape_name} b={B}, {T} tokens)",
@@ -164,7 +167,7 @@ def run_prefill(a):
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f32",
         "data": "synthetic: seeded N(0,0.02) random-init weights, uniform random token ids",
-        "config": {"workload": f"{a.workload}: GPT-2 {shape_name}, batch {B}, prefill {T} tokens, full logits",
+        "config": {"workload": f"{a.workload}: GPT-2 {shape_name}, batch {B}, prefill {T} tokens, no logits",
                    "batch": B, "tokens": T, "weights": "f32"},
         "roofline": {"bound": "mfma", "kernel": "whole prefill (pair_gemm_kernel dominant: f32 products as three f16 MFMA products; "
                                "frac is of the f32 MFMA peak)",
@@ -196,25 +199,27 @@ def measured_traffic(workload, persistent):
     return None
 
 
-def prefill_bytes(sh, B, T, wbytes):
+def prefill_bytes(sh, B, T, wbytes, head_rows=None):
     """Algorithmic HBM bytes of forward_cached over T tokens on an empty
-    cache: weights once, the T embedding rows, the K/V rows written and every
-    row's logits written (the reference computes [T, V])."""
+    cache: weights once, the T embedding rows, the K/V rows written and the
+    logits of head_rows rows per sequence written (default every row)."""
     L, d, V = sh.n_layer, sh.n_embd, sh.vocab_size
     weights = (L * (12 * d * d + 13 * d) + V * d + 2 * d)
     mats = L * 12 * d * d + V * d
     wb = mats * wbytes + (weights - mats) * 4
-    return wb + B * T * (2 * d * wbytes + L * 2 * d * 4 + V * 4)
+    head = T if head_rows is None else head_rows
+    return wb + B * (T * (2 * d * wbytes + L * 2 * d * 4) + head * V * 4)
 
 
-def prefill_roofline(sh, B, T, wbytes, ms):
+def prefill_roofline(sh, B, T, wbytes, ms, head_rows=None):
     """Roofline of the prefill leg: HBM when its arithmetic intensity is
     below the MFMA ridge (peak / 8 TB/s), MFMA otherwise. The peak is fp32
-    MFMA for f32 weights; for bf16 weights the GEMMs run on bf16 MFMA with
-    three exact products per f32 product (mfma "bf16x3"), so the peak in
-    algorithmic f32 flops is the dense bf16 peak / 3."""
-    flops = prefill_flops(sh, B, T)
-    nbytes = prefill_bytes(sh, B, T, wbytes)
+    MFMA for f32 weights and a third of the dense bf16 MFMA rate for bf16
+    weights (three 16-bit products per f32 product, mfma "bf16x3"). The
+    GEMMs run on f16 pairs, three (bf16 weights: two) f16 products per f32
+    product, so long f32 prompts exceed the fp32 MFMA peak."""
+    flops = prefill_flops(sh, B, T, head_rows)
+    nbytes = prefill_bytes(sh, B, T, wbytes, head_rows)
     s = ms / 1e3
     bf16 = wbytes == 2
     peak = BF16X3_PEAK_TFLOPS if bf16 else MFMA_FP32_PEAK_TFLOPS
@@ -335,7 +340,7 @@ def main():
         "config": {"workload": f"{a.workload}: GPT-2 {shape_name}, batch {B}, prompt {n_prompt}, greedy {n_new}",
                    "batch": B, "prompt": n_prompt, "new_tokens": n_new, "weights": storage},
         "prefill_tok_s": round(B * n_prompt * a.steps / (pre_ms / 1e3), 1),
-        "prefill_roofline": prefill_roofline(sh, B, n_prompt, wbytes, pre_ms / a.steps),
+        "prefill_roofline": prefill_roofline(sh, B, n_prompt, wbytes, pre_ms / a.steps, head_rows=1),
         "decode_ms_per_token_step": round(step_ms, 4),
         "roofline": {"bound": "hbm", "kernel": kernel, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),

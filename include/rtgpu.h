@@ -143,7 +143,8 @@ rtg_result rtg_cache_read(const rtg_cache* cache, size_t layer, size_t head, siz
 /* Gpt2Model::forward, gpt2.rs:269-304: logits_out[n * vocab_size]. */
 rtg_result rtg_forward(const rtg_model* model, const uint32_t* ids, size_t n, float* logits_out);
 /* Gpt2Model::forward_cached, gpt2.rs:358-399: logits_out[n * vocab_size]
- * (may be NULL to skip the device-to-host copy). The cache must have batch 1
+ * (may be NULL: nothing is copied, and a prompt of more than one token runs
+ * without its LM head). The cache must have batch 1
  * and belong to model. One new token (n == 1) runs the persistent decode
  * step that generate_cached runs per token, where the model's shape has one;
  * 2..32 tokens run the multi-row forward in one launch (f32 weights, n_embd

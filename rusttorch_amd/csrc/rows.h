@@ -42,7 +42,7 @@ unsigned* rows_err(RowsState* s);
 // Enqueues forward_cached of S sequences x T new tokens: ids_dev [S*T], cache
 // layer 0 at kc / vc ([seq][head][P][64], kv_layer floats per layer), every
 // sequence's first new token at position past, or *pos_dev when pos_dev is
-// set; logits [S*T][V]. The caller must hold persistent_launch_lock(device)
+// set; logits [S*T][V] (null: the LM head is not run; not with fin). The caller must hold persistent_launch_lock(device)
 // from the launch until the stream has drained.
 // With fin set, the launch also finishes a greedy step the way launch_argmax
 // + launch_finalize do: keys [S] (zero on entry, cleared again), the argmax

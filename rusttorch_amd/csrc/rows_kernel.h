@@ -142,7 +142,7 @@ struct RParams {
   float* p0;  long p0_stride;  // c_attn partials [KSQ][MR][3D] of layer l, then its c_fc partials
   long p0_fc;                  //   [KSF][MR][4D] at this offset
   float* p1;                   // attn / mlp c_proj partials [ks][MR][D]
-  float* logits;       // [M][V]
+  float* logits;       // [M][V] (null: no LM head)
   // Optional greedy finish (keys set): the argmax of each sequence's last row
   // (argmax_key, gpt2.rs:858-868) into keys[s]; the last workgroup to finish
   // then writes token[s] = that index and ids_out[s * ld_ids + *step], clears
@@ -1213,7 +1213,7 @@ __global__ __launch_bounds__(NTH, 1) void rows_kernel(RParams p) {
       asm volatile("" : : "v"(prev));
     }
     mark(L, PH_QKV, 3);
-  } else
+  } else if (p.logits != nullptr)
   // ---- tied LM head (gpt2.rs:392-396): logits[r][n] = ln_f(x_r) . wte[n] ----
   // Tiles of 32 vocabulary rows, workgroup wg taking tiles wg, wg + G, ...;
   // each tile in NS = D / 128 k steps, compute wave w taking k [128 s + 32 w,

@@ -306,11 +306,16 @@ static Work cache_work(const rtg_cache* c) {
   return Work{c->x, c->ln, c->qkv, c->att, c->h, c->logits, c->ws, c->ws_floats};
 }
 
+// The rows whose logits a prefill computes: all S*T, the last row of each
+// sequence (written as S rows: all that generation reads, gpt2.rs:420-423), or
+// none (a prompt read into the cache without logits_out).
+enum LogitRows { LOGITS_ALL, LOGITS_LAST, LOGITS_NONE };
+
 // forward_cached body for S sequences x T new tokens (gpt2.rs:376-396) on the
 // pair GEMMs (gemm_pair.h): w.ln, w.att and w.h hold f16 pairs, 4 bytes per
 // element like the f32 rows they replace.
 static void enqueue_prefill_pair(rtg_cache* c, const Work& w, const uint32_t* ids_dev, size_t S, size_t T, size_t past,
-                                 int logit_mode) {
+                                 LogitRows logit_rows) {
   const rtg_model* m = c->m;
   const PrefillWeights& pw = *m->pw;
   const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, M = (int)(S * T);
@@ -352,25 +357,25 @@ static void enqueue_prefill_pair(rtg_cache* c, const Work& w, const uint32_t* id
     launch_pair_gemm(s, P.fc, a);
     launch_pair_gemm(s, P.mproj, args(h, 4 * d, L.bmproj, w.x, d, EPI_BIAS_RESID));
   }
-  // ln_f and the logits of every row, or of the last row of each sequence
-  const int rows = logit_mode == 0 ? M : (int)S;
-  const long ldx = logit_mode == 0 ? d : (long)T * d;
-  launch_layernorm_pair(s, w.x + (logit_mode == 0 ? 0 : (T - 1) * d), ldx, m->lnfw, m->lnfb, eps, rows, d, pw.sf, ln);
-  PairGemmArgs a = args(ln, d, nullptr, w.logits, V, EPI_NONE);
-  a.M = rows;
-  a.ws = nullptr;
-  launch_pair_gemm(s, pw.lm, a);
+  if (logit_rows != LOGITS_NONE) {
+    const bool all = logit_rows == LOGITS_ALL;
+    const int rows = all ? M : (int)S;
+    launch_layernorm_pair(s, w.x + (all ? 0 : (T - 1) * d), all ? d : (long)T * d, m->lnfw, m->lnfb, eps, rows, d,
+                          pw.sf, ln);
+    PairGemmArgs a = args(ln, d, nullptr, w.logits, V, EPI_NONE);
+    a.M = rows;
+    a.ws = nullptr;
+    launch_pair_gemm(s, pw.lm, a);
+  }
   HIPX(hipGetLastError());
 }
 
 // forward_cached body for S sequences x T new tokens (gpt2.rs:376-396) on the
-// MFMA prefill path, on the activation buffers w. ids_dev holds S*T ids;
-// logits rows: all S*T (mode 0) or the last row of each sequence (mode 1,
-// written as S rows).
+// MFMA prefill path, on the activation buffers w. ids_dev holds S*T ids.
 static void enqueue_prefill(rtg_cache* c, const Work& w, const uint32_t* ids_dev, size_t S, size_t T, size_t past,
-                            int logit_mode) {
+                            LogitRows logit_rows) {
   const rtg_model* m = c->m;
-  if (m->pw) return enqueue_prefill_pair(c, w, ids_dev, S, T, past, logit_mode);
+  if (m->pw) return enqueue_prefill_pair(c, w, ids_dev, S, T, past, logit_rows);
   const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, M = (int)(S * T);
   const float eps = m->cfg.layer_norm_epsilon;
   hipStream_t s = c->stream;
@@ -388,8 +393,9 @@ static void enqueue_prefill(rtg_cache* c, const Work& w, const uint32_t* ids_dev
     launch_gemm(s, w.h, 4 * d, L.wmproj, m->wtype, L.bmproj, w.x, d, M, d, 4 * d, EPI_BIAS_RESID, w.ws,
                 w.ws_floats);
   }
+  if (logit_rows == LOGITS_NONE) return;
   launch_layernorm(s, w.x, m->lnfw, m->lnfb, eps, M, d, w.ln);
-  if (logit_mode == 0) {
+  if (logit_rows == LOGITS_ALL) {
     launch_gemm(s, w.ln, d, m->wte, m->wtype, nullptr, w.logits, V, M, V, d, EPI_NONE);
   } else {
     // Last row of each sequence: rows (s*T + T-1), stride T*d.
@@ -641,7 +647,7 @@ static bool rows_path(const rtg_cache* c, size_t S, size_t T) {
 
 // Enqueues the multi-row forward on the cache's stream (the caller holds
 // persistent_launch_lock until the stream drains): ids_dev [S*T] at position
-// past, logits [S*T][V]; state st (default: the cache's own, made on first use).
+// past, logits [S*T][V] (null: no LM head); state st (default: the cache's own, made on first use).
 static void enqueue_rows(rtg_cache* c, const uint32_t* ids_dev, size_t S, size_t T, size_t past, float* logits,
                          RowsState* st = nullptr, const RowsFinish* fin = nullptr) {
   const rtg_model* m = c->m;
@@ -703,7 +709,7 @@ static void forward_cached_impl(rtg_cache* c, const uint32_t* ids, size_t n, flo
   const rtg_model* m = c->m;
   const size_t B = c->batch, V = m->cfg.vocab_size;
   ensure_rows(c, B * n);
-  ensure_logits(c, B * n);
+  ensure_logits(c, logits_out ? B * n : B);
   if (n == 1 && B == 1 && persistent_supported(m->pplan, 1)) {
     // one new token at batch 1: the persistent decode step, the kernel
     // generate_cached runs per token; its token is read from token_dev at
@@ -741,7 +747,7 @@ static void forward_cached_impl(rtg_cache* c, const uint32_t* ids, size_t n, flo
   } else if (rows_path(c, B, n)) {
     std::lock_guard<std::mutex> plock(persistent_launch_lock(m->device));
     HIPX(hipMemcpyAsync(c->ids_in, ids, B * n * 4, hipMemcpyHostToDevice, c->stream));
-    enqueue_rows(c, c->ids_in, B, n, c->len, c->logits);
+    enqueue_rows(c, c->ids_in, B, n, c->len, logits_out ? c->logits : nullptr);
     if (logits_out) HIPX(hipMemcpyAsync(logits_out, c->logits, B * n * V * 4, hipMemcpyDeviceToHost, c->stream));
     HIPX(hipStreamSynchronize(c->stream));
     check_rows(c->rstate);
@@ -749,7 +755,7 @@ static void forward_cached_impl(rtg_cache* c, const uint32_t* ids, size_t n, flo
     return;
   } else {
     HIPX(hipMemcpyAsync(c->ids_in, ids, B * n * 4, hipMemcpyHostToDevice, c->stream));
-    enqueue_prefill(c, cache_work(c), c->ids_in, B, n, c->len, 0);
+    enqueue_prefill(c, cache_work(c), c->ids_in, B, n, c->len, logits_out ? LOGITS_ALL : LOGITS_NONE);
   }
   if (logits_out) HIPX(hipMemcpyAsync(logits_out, c->logits, B * n * V * 4, hipMemcpyDeviceToHost, c->stream));
   HIPX(hipStreamSynchronize(c->stream));
@@ -795,8 +801,9 @@ static void generate_greedy(const rtg_model* m, const uint32_t* prompts, size_t 
   rtg_cache* c = lease.c;
   const size_t V = m->cfg.vocab_size, P = m->cfg.n_positions;
   const size_t steps = max_new > 0 ? max_new : 1;  // first token comes from prefill
+  const bool rows = rows_path(c, B, n);
   ensure_rows(c, B * n);
-  ensure_logits(c, B * n);
+  ensure_logits(c, rows ? B * n : B);
   hipStream_t s = c->stream;
   // overwrite the argmax token of the step just enqueued with the sampler's choice
   auto sample = [&](const float* row) {
@@ -812,7 +819,6 @@ static void generate_greedy(const rtg_model* m, const uint32_t* prompts, size_t 
   // The persistent step's workgroups wait on each other: no second persistent
   // step of this process may be in flight on the device (another thread's
   // cache) until this stream has drained.
-  const bool rows = rows_path(c, B, n);
   if (rows && !c->rstate) {  // (allocated before the timed prefill)
     c->rstate = rows_state_create(m->rplan);
     if (!c->rstate) throw HipError{"multi-row forward: state allocation failed"};
@@ -830,12 +836,12 @@ static void generate_greedy(const rtg_model* m, const uint32_t* prompts, size_t 
     const RowsFinish fin{c->keys, c->token_dev, c->ids_dev, (int)P, c->pos_dev, c->step_dev};
     enqueue_rows(c, c->ids_in, B, n, 0, c->logits, nullptr, &fin);
   } else {
-    enqueue_prefill(c, cache_work(c), c->ids_in, B, n, 0, 0);
     // argmax of the last row of each sequence (extract_row(logits, n-1))
-    launch_argmax(s, c->logits + (n - 1) * V, (long)(n * V), (int)B, (int)V, c->keys);
+    enqueue_prefill(c, cache_work(c), c->ids_in, B, n, 0, LOGITS_LAST);
+    launch_argmax(s, c->logits, (long)V, (int)B, (int)V, c->keys);
     launch_finalize(s, (int)B, c->keys, c->token_dev, c->ids_dev, (int)P, c->pos_dev, c->step_dev);
   }
-  sample(c->logits + (n - 1) * V);
+  sample(rows ? c->logits + (n - 1) * V : c->logits);
   HIPX(hipEventRecord(c->ev[1], s));
   // The persistent step (one kernel) is launched directly: replaying it as a
   // one-node graph was measured to leave ~8 us between launches instead of ~1.
@@ -1365,7 +1371,7 @@ static rtg_result noalloc_rows(const rtg_model* model, rtg_cache* cache, const u
     st.fresh = false;
     float* logits = sp + state;
     HIPX(hipMemcpyAsync(cache->ids_in, ids, n * 4, hipMemcpyHostToDevice, cache->stream));
-    enqueue_rows(cache, cache->ids_in, 1, n, cache->len, logits, &st);
+    enqueue_rows(cache, cache->ids_in, 1, n, cache->len, logits_out ? logits : nullptr, &st);
     if (logits_out) HIPX(hipMemcpyAsync(logits_out, logits, n * V * 4, hipMemcpyDeviceToHost, cache->stream));
     HIPX(hipStreamSynchronize(cache->stream));
     check_rows(&st);
@@ -1426,7 +1432,7 @@ rtg_result rtg_forward_cached_noalloc(const rtg_model* model, rtg_cache* cache, 
     w.ws = pw ? w.logits + pv : nullptr;
     w.ws_floats = pw;
     HIPX(hipMemcpyAsync(cache->ids_in, ids, n * 4, hipMemcpyHostToDevice, cache->stream));
-    enqueue_prefill(cache, w, cache->ids_in, 1, n, cache->len, 0);
+    enqueue_prefill(cache, w, cache->ids_in, 1, n, cache->len, logits_out ? LOGITS_ALL : LOGITS_NONE);
     HIPX(hipGetLastError());
     if (logits_out)
       HIPX(hipMemcpyAsync(logits_out, w.logits, n * V * 4, hipMemcpyDeviceToHost, cache->stream));
@@ -1561,7 +1567,7 @@ rtg_result rtg_generate(const rtg_model* model, const uint32_t* prompt, size_t n
     for (size_t i = 0; i < max_new; ++i) {
       const size_t len = n + i;
       const size_t start = len > P ? len - P : 0;
-      enqueue_prefill(c, cache_work(c), toks + start, 1, len - start, 0, 1);  // logits of the last row only
+      enqueue_prefill(c, cache_work(c), toks + start, 1, len - start, 0, LOGITS_LAST);
       if (!launch_sample(s, c->logits, (int)V, toks, (int)n, toks + n, steps + i, sp, c->token_dev))
         throw HipError{"vocabulary too large for the device sampler"};
     }
