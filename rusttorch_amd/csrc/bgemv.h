@@ -1,4 +1,4 @@
-// Batched decode GEMV (2..16 sequences) over tile-ordered weights; see
+// Batched decode GEMV (2..32 sequences) over tile-ordered weights; see
 // bgemv.hip for the tile layout and the work split.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -7,6 +7,8 @@
 #include "kernels.h"
 
 namespace rtg {
+
+constexpr int kBgemvRows = 32;  // most input rows; row stride of the statistics partials and centres
 
 // QKV epilogue target: q part to q[m][ldq], the new token's k/v parts into
 // the cache at *pos_dev. q == nullptr selects the plain epilogues.
@@ -19,7 +21,7 @@ struct BgemvQkv {
 };
 
 struct BgemvArgs {
-  // f32 inputs of M <= 16 rows in the GEMV input layout: element (m, k) at
+  // f32 inputs of M <= kBgemvRows rows in the GEMV input layout: element (m, k) at
   // xt_index(m, k, M, TK) (kernels.h), TK = 16 for f32 weights, 32 for bf16
   const float* X;
   int M;
@@ -67,7 +69,7 @@ struct BgemvArgs {
   // LM head: per-row packed argmax keys (gpt2.rs:858-868), updated with a
   // device-scope atomic max (zero before; the step's finalize resets them).
   unsigned long long* keys;
-  float* part;    // workspace of bgemv_work_floats(plan) floats when plan.S > 1
+  float* part;    // workspace of bgemv_work_floats(plan, M) floats when plan.S > 1
   unsigned* cnt;  // plan.groups zeroed counters when plan.S > 1 (left zeroed)
   int S, ktc;     // filled in from the plan
 };
@@ -88,7 +90,7 @@ bool launch_tile_weights(hipStream_t s, const void* src, int wtype, int N, int K
 BgemvPlan bgemv_plan(int N, int K, int wtype, int npw_force = 0, int s_force = 0, int nw = 4);
 // The argument checks launch_bgemv makes (shape, workspaces, LayerNorm parts).
 bool bgemv_args_ok(const BgemvPlan& pl, const BgemvArgs& a);
-size_t bgemv_work_floats(const BgemvPlan& pl);
+size_t bgemv_work_floats(const BgemvPlan& pl, int M);
 bool launch_bgemv(hipStream_t s, const BgemvPlan& pl, BgemvArgs a);
 // Decode embedding x[r] = wte[token[r]] + wpe[*pos_dev] of rows r < rows,
 // (x[r] - mean_r) * g in the GEMV input layout to xg (xt_index(r, k, rows,

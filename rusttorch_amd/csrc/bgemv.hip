@@ -1,6 +1,7 @@
-// Batched decode GEMV on fp32 MFMA for 2..16 sequences (the graph path of
+// Batched decode GEMV on fp32 MFMA for 2..32 sequences (the graph path of
 // forward_cached with one new token per sequence, gpt2.rs:358-399 / 628-633):
-// y[m][n] = epi(sum_k x[m][k] * W^T[n][k]) for m < M <= 16.
+// y[m][n] = epi(sum_k x[m][k] * W^T[n][k]) for m < M <= 32: one or two blocks
+// of 16 rows, each weight tile loaded once for both.
 //
 // The weights are read from a tile-ordered copy made once per model, so that
 // every wave load is one contiguous KiB that lands in exactly the registers
@@ -55,21 +56,51 @@ __global__ void tile_weights_kernel(const void* __restrict__ src, int wtype, int
   reinterpret_cast<u4v*>(dst)[i] = v;
 }
 
-template <int WT, int NPW, bool LNG, int DEPTH, bool ONESHOT>
+template <int WT, int NPW, bool LNG, int MB, int DEPTH, bool ONESHOT>
 __global__ __launch_bounds__(64 * BG_NW) void bgemv_kernel(BgemvArgs a) {
-  __shared__ float red[BG_NW][NPW][256];
+  __shared__ float red[BG_NW][MB * NPW][256];
   __shared__ unsigned last;
-  bgc::bgemv_unit<WT, NPW, LNG, BG_NW, DEPTH, ONESHOT>(a, blockIdx.x, blockIdx.y, red, &last);
+  bgc::bgemv_unit<WT, NPW, LNG, BG_NW, MB, DEPTH, ONESHOT>(a, blockIdx.x, blockIdx.y, red, &last);
 }
 
-// k-tiles a wave keeps in flight: its whole chunk at once when that fits
-// the register budget (about 160 registers of tiles: weights and x), else a
-// ring of 4.
-int bgemv_depth(const BgemvPlan& pl, int wtype) {
-  const int per_tile = 4 * pl.npw + (wtype == W_F32 ? 4 : 8);
-  for (int d : {8, 12})
-    if (pl.ktc <= d && per_tile * d <= 160) return d;
-  return 4;
+// k-tiles a wave keeps in flight: its whole chunk (8 or 12) at once when that
+// fits the register budget (about 160 registers of tiles: weights and x), else
+// a ring of 4.
+template <int WT, int NPW, bool LNG, int MB>
+void launch_depth(hipStream_t s, dim3 grid, const BgemvArgs& a) {
+  constexpr int per_tile = 4 * NPW + MB * (WT == W_F32 ? 4 : 8);
+  const dim3 block(64 * BG_NW);
+  if constexpr (per_tile * 8 <= 160) {
+    if (a.ktc <= 8) {
+      bgemv_kernel<WT, NPW, LNG, MB, 8, true><<<grid, block, 0, s>>>(a);
+      return;
+    }
+  }
+  if constexpr (per_tile * 12 <= 160) {
+    if (a.ktc <= 12) {
+      bgemv_kernel<WT, NPW, LNG, MB, 12, true><<<grid, block, 0, s>>>(a);
+      return;
+    }
+  }
+  bgemv_kernel<WT, NPW, LNG, MB, 4, false><<<grid, block, 0, s>>>(a);
+}
+
+template <int WT, int NPW>
+void launch_rows(hipStream_t s, dim3 grid, const BgemvArgs& a) {
+  if (a.M > 16) {
+    if (a.ln_g) launch_depth<WT, NPW, true, 2>(s, grid, a);
+    else launch_depth<WT, NPW, false, 2>(s, grid, a);
+  } else {
+    if (a.ln_g) launch_depth<WT, NPW, true, 1>(s, grid, a);
+    else launch_depth<WT, NPW, false, 1>(s, grid, a);
+  }
+}
+
+template <int WT>
+void launch_panels(hipStream_t s, int npw, dim3 grid, const BgemvArgs& a) {
+  if (npw == 1) launch_rows<WT, 1>(s, grid, a);
+  else if (npw == 2) launch_rows<WT, 2>(s, grid, a);
+  else launch_rows<WT, 4>(s, grid, a);
 }
 
 // Decode embedding of B rows (gpt2.rs:377-384: wte[token] + wpe[position]),
@@ -196,7 +227,7 @@ BgemvPlan bgemv_plan(int N, int K, int wtype, int npw_force, int s_force, int nw
 
 bool bgemv_args_ok(const BgemvPlan& pl, const BgemvArgs& a) {
   const int TK = a.wtype == W_F32 ? 16 : 32;
-  if (a.M < 1 || a.M > 16 || a.K % TK != 0) return false;
+  if (a.M < 1 || a.M > kBgemvRows || a.K % TK != 0) return false;
   if (a.c_tiled && (a.epi == EPI_BIAS_RESID || a.qkv.q || a.N % TK != 0)) return false;
   if (pl.S < 1 || pl.S > bgc::SMAX || (pl.S > 1 && (!a.part || !a.cnt))) return false;
   if (a.ln_g && (!a.ln_s || !a.ln_part || a.ln_groups < 1 || a.ln_groups > 16 * bgc::LNG_PER || a.ln_cols < 1 ||
@@ -208,37 +239,17 @@ bool bgemv_args_ok(const BgemvPlan& pl, const BgemvArgs& a) {
   return true;
 }
 
-size_t bgemv_work_floats(const BgemvPlan& pl) { return pl.S > 1 ? (size_t)pl.groups * pl.S * pl.npw * 256 : 0; }
+size_t bgemv_work_floats(const BgemvPlan& pl, int M) {
+  return pl.S > 1 ? (size_t)pl.groups * pl.S * (M > 16 ? 2 : 1) * pl.npw * 256 : 0;
+}
 
 bool launch_bgemv(hipStream_t s, const BgemvPlan& pl, BgemvArgs a) {
   if (!bgemv_args_ok(pl, a)) return false;
   a.S = pl.S;
   a.ktc = pl.ktc;
   const dim3 grid(pl.groups, pl.S);
-  const dim3 block(64 * BG_NW);
-  const int depth = bgemv_depth(pl, a.wtype);
-#define BG_LAUNCH_D(WT, NPW, LNG)                                                         \
-  do {                                                                                    \
-    if (depth == 12) bgemv_kernel<WT, NPW, LNG, 12, true><<<grid, block, 0, s>>>(a);      \
-    else if (depth == 8) bgemv_kernel<WT, NPW, LNG, 8, true><<<grid, block, 0, s>>>(a);   \
-    else bgemv_kernel<WT, NPW, LNG, 4, false><<<grid, block, 0, s>>>(a);                  \
-  } while (0)
-#define BG_LAUNCH(WT, NPW)                 \
-  do {                                     \
-    if (a.ln_g) BG_LAUNCH_D(WT, NPW, true); \
-    else BG_LAUNCH_D(WT, NPW, false);       \
-  } while (0)
-  if (a.wtype == W_F32) {
-    if (pl.npw == 1) BG_LAUNCH(W_F32, 1);
-    else if (pl.npw == 2) BG_LAUNCH(W_F32, 2);
-    else BG_LAUNCH(W_F32, 4);
-  } else {
-    if (pl.npw == 1) BG_LAUNCH(W_BF16, 1);
-    else if (pl.npw == 2) BG_LAUNCH(W_BF16, 2);
-    else BG_LAUNCH(W_BF16, 4);
-  }
-#undef BG_LAUNCH
-#undef BG_LAUNCH_D
+  if (a.wtype == W_F32) launch_panels<W_F32>(s, pl.npw, grid, a);
+  else launch_panels<W_BF16>(s, pl.npw, grid, a);
   return hipGetLastError() == hipSuccess;
 }
 

@@ -48,21 +48,23 @@ struct Tile<W_BF16> {
   }
 };
 
-// The epilogue's operands for output (m, n) of one thread. The residual
-// epilogue loads them before the k loop, so that the epilogue after it makes
-// no global round trip before its stores (measured: 12.3 -> 11.7 us for
-// 1600 x 6400 bf16 at M = 16); for the others, loading them early measured
-// ~0.1 us slower, and they are loaded in the epilogue.
+// The epilogue's operands for output (m, n) of one thread, loaded before the k
+// loop so that the epilogue makes no global round trip before its stores
+// (GPT-2 small f32, 8 sequences: 361 -> 356 us per step against loading them
+// in the epilogue of all but the residual GEMVs).
 struct EpiIn {
   float bias, ln_s, g_next, resid;
 };
 __device__ __forceinline__ EpiIn load_epi(const BgemvArgs& a, int m, int n, bool lng) {
   EpiIn e{0.f, 0.f, 0.f, 0.f};
   if (n < a.N) {
+    // (branch-free for the row: one past M re-reads the last one. With a
+    // branch the compiler waited for all weight tiles in flight before it,
+    // 0.5 us per launch)
+    if (!a.qkv.q && a.epi == EPI_BIAS_RESID) e.resid = a.C[(size_t)min(m, a.M - 1) * a.ldc + n];
     if (a.bias) e.bias = a.bias[n];
     if (lng) e.ln_s = a.ln_s[n];
     if (a.xg) e.g_next = a.g_next[n];
-    if (!a.qkv.q && a.epi == EPI_BIAS_RESID && m < a.M) e.resid = a.C[(size_t)m * a.ldc + n];
   }
   return e;
 }
@@ -108,11 +110,11 @@ __device__ __forceinline__ float row16_sum(float v) {
 // Residual epilogue statistics: this group's (mean, M2) per row over the
 // columns it wrote, stored to stats_part[g][m] for the GEMV that reads x
 // next. y[j] are the values thread tid (< 256) wrote (valid[j] false for
-// columns past N or rows past M).
+// columns past N or rows past M) of row m.
 template <int NPW>
-__device__ __forceinline__ void row_stats_partial(const BgemvArgs& a, int g, const float (&y)[NPW],
+__device__ __forceinline__ void row_stats_partial(const BgemvArgs& a, int g, int m, const float (&y)[NPW],
                                                   const bool (&valid)[NPW]) {
-  const int tid = threadIdx.x, m = tid >> 4;
+  const int tid = threadIdx.x;
   float sum = 0.f, cnt = 0.f;
 #pragma unroll
   for (int j = 0; j < NPW; ++j) {
@@ -130,8 +132,8 @@ __device__ __forceinline__ void row_stats_partial(const BgemvArgs& a, int g, con
   }
   m2 = row16_sum(m2);
   if ((tid & 15) == 0 && m < a.M) {
-    a.stats_part[((size_t)g * 16 + m) * 2] = mean;
-    a.stats_part[((size_t)g * 16 + m) * 2 + 1] = m2;
+    a.stats_part[((size_t)g * kBgemvRows + m) * 2] = mean;
+    a.stats_part[((size_t)g * kBgemvRows + m) * 2 + 1] = m2;
   }
 }
 
@@ -165,18 +167,20 @@ __device__ __forceinline__ void row_stats_merge(const BgemvArgs& a, const float2
 }
 
 // One work unit = panel group g, k split s, on the NW waves of this
-// workgroup (wave w takes k-chunk s * NW + w). red: LDS [NW][NPW][256];
+// workgroup (wave w takes k-chunk s * NW + w). red: LDS [NW][MB * NPW][256];
 // last: one LDS word. Every thread of the workgroup calls it.
+// MB: blocks of 16 input rows (M <= 16 MB); each weight tile is loaded once
+// and multiplied with all of them.
 // DEPTH_ k-tiles of a wave are in flight at once: a ring refilled as tiles
 // are consumed, or, with ONESHOT (the caller guarantees ktc <= DEPTH_), the
 // whole chunk loaded at once and consumed without refills.
-template <int WT, int NPW, bool LNG, int NW, int DEPTH_ = DEPTH, bool ONESHOT = false>
-__device__ __forceinline__ void bgemv_unit(const BgemvArgs& a, int g, int s, float (*red)[NPW][256],
+template <int WT, int NPW, bool LNG, int NW, int MB, int DEPTH_ = DEPTH, bool ONESHOT = false>
+__device__ __forceinline__ void bgemv_unit(const BgemvArgs& a, int g, int s, float (*red)[MB * NPW][256],
                                            unsigned* last) {
   typedef Tile<WT> TL;
   constexpr int E = TL::E, TK = TL::TK;
   typedef typename TL::Raw Raw;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
   const bool ep = tid < 256;  // the epilogue threads: element tid of each panel
   const int NP = (a.N + 15) >> 4, KT = a.K / TK;
@@ -189,26 +193,33 @@ __device__ __forceinline__ void bgemv_unit(const BgemvArgs& a, int g, int s, flo
     const int p = min(g * NPW + j, NP - 1);
     wp[j] = reinterpret_cast<const Raw*>(a.Wt) + ((size_t)p * KT + t0) * 64 + lane;
   }
-  // input layout xt_index: lane (r, q) loads chunk (h, q) of row r as 16
-  // bytes at ((h * 4 + q) * M + r) * 4 within tile t (rows past M repeat the
-  // last), so a group of 16 lanes reads M rows of one chunk contiguously
-  const int xr = min(r, a.M - 1);
-  const float* xb = a.X + (size_t)t0 * TK * a.M + (size_t)(q * a.M + xr) * 4;
-  floatx4 acc[NPW];
+  // input layout xt_index: lane (r, q) loads chunk (h, q) of row r of each row
+  // block as 16 bytes at ((h * 4 + q) * M + r) * 4 within tile t (rows past M
+  // repeat the last), so a group of 16 lanes reads its rows of one chunk
+  // contiguously
+  const float* xb[MB];
 #pragma unroll
-  for (int j = 0; j < NPW; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < MB; ++b)
+    xb[b] = a.X + (size_t)t0 * TK * a.M + (size_t)(q * a.M + min(b * 16 + r, a.M - 1)) * 4;
+  floatx4 acc[MB][NPW];
+#pragma unroll
+  for (int b = 0; b < MB; ++b)
+#pragma unroll
+    for (int j = 0; j < NPW; ++j) acc[b][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   // DEPTH_ tiles in flight; past the end the last tile is re-read (never
   // consumed) so that the load sequence stays branch-free
   Raw w[DEPTH_][NPW];
-  f4v x[DEPTH_][E / 4];
+  f4v x[DEPTH_][MB][E / 4];
   auto issue = [&](int slot, int i) {
     const int ti = min(i, max(nt - 1, 0));
 #pragma unroll
     for (int j = 0; j < NPW; ++j) w[slot][j] = __builtin_nontemporal_load(wp[j] + (size_t)ti * 64);
 #pragma unroll
-    for (int h = 0; h < E / 4; ++h)
-      x[slot][h] = *reinterpret_cast<const f4v*>(xb + (size_t)ti * TK * a.M + h * 16 * a.M);
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+      for (int h = 0; h < E / 4; ++h)
+        x[slot][b][h] = *reinterpret_cast<const f4v*>(xb[b] + (size_t)ti * TK * a.M + h * 16 * a.M);
   };
   // one tile: acc += x . w over its TK inputs
   auto consume = [&](int d) {
@@ -218,49 +229,69 @@ __device__ __forceinline__ void bgemv_unit(const BgemvArgs& a, int g, int s, flo
       // exact in f32 and the MFMA accumulates in f32: the f32 GEMV up to
       // summation order (3 MFMAs per tile instead of 8 of 16x16x4 f32;
       // measured ~10% faster, with half the error against a float64 sum)
-      float xs[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) xs[e] = x[d][e >> 2][e & 3];
-      u4v xh, xm, xl;
-      split3(xs, xh, xm, xl);
+      for (int b = 0; b < MB; ++b) {
+        float xs[8];
 #pragma unroll
-      for (int j = 0; j < NPW; ++j) {
-        const bf16x8 wb = as_bf16x8(w[d][j]);
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xh), wb, acc[j], 0, 0, 0);
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xm), wb, acc[j], 0, 0, 0);
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xl), wb, acc[j], 0, 0, 0);
+        for (int e = 0; e < 8; ++e) xs[e] = x[d][b][e >> 2][e & 3];
+        u4v xh, xm, xl;
+        split3(xs, xh, xm, xl);
+#pragma unroll
+        for (int j = 0; j < NPW; ++j) {
+          const bf16x8 wb = as_bf16x8(w[d][j]);
+          acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xh), wb, acc[b][j], 0, 0, 0);
+          acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xm), wb, acc[b][j], 0, 0, 0);
+          acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xl), wb, acc[b][j], 0, 0, 0);
+        }
       }
     } else {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        const float xa = x[d][e >> 2][e & 3];
 #pragma unroll
-        for (int j = 0; j < NPW; ++j)
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, TL::get(w[d][j], e), acc[j], 0, 0, 0);
+        for (int b = 0; b < MB; ++b) {
+          const float xa = x[d][b][e >> 2][e & 3];
+#pragma unroll
+          for (int j = 0; j < NPW; ++j)
+            acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, TL::get(w[d][j], e), acc[b][j], 0, 0, 0);
+        }
       }
     }
   };
   // the input rows' LayerNorm statistics partials, loaded now and merged in
   // the epilogue (the kernel that wrote x left them)
-  float2 lnp[LNG_PER];
+  float2 lnp[MB][LNG_PER];
   if (nt > 0) {
 #pragma unroll
     for (int d = 0; d < DEPTH_; ++d) issue(d, d);
   }
   if constexpr (LNG) {
-    const int mrow = min((tid & 255) >> 4, a.M - 1), sub = tid & 15;
+    const int sub = tid & 15;
 #pragma unroll
-    for (int i = 0; i < LNG_PER; ++i) {
-      const int gg = min(sub + 16 * i, a.ln_groups - 1);
-      lnp[i] = *reinterpret_cast<const float2*>(a.ln_part + ((size_t)gg * 16 + mrow) * 2);
+    for (int b = 0; b < MB; ++b) {
+      const int mrow = min(b * 16 + ((tid & 255) >> 4), a.M - 1);
+#pragma unroll
+      for (int i = 0; i < LNG_PER; ++i) {
+        const int gg = min(sub + 16 * i, a.ln_groups - 1);
+        lnp[b][i] = *reinterpret_cast<const float2*>(a.ln_part + ((size_t)gg * kBgemvRows + mrow) * 2);
+      }
     }
   }
-  const int m = tid >> 4;
-  const bool early = a.epi == EPI_BIAS_RESID && !a.qkv.q;
-  EpiIn eo[NPW];
-  if (ep && early) {
+  EpiIn eo[MB][NPW];
+  float cin[MB], xcn[MB];
+  auto load_row = [&](int b) {
 #pragma unroll
-    for (int j = 0; j < NPW; ++j) eo[j] = load_epi(a, m, (g * NPW + j) * 16 + (tid & 15), LNG);
+    for (int j = 0; j < NPW; ++j)
+      eo[b][j] = load_epi(a, b * 16 + (tid >> 4), (g * NPW + j) * 16 + (tid & 15), LNG);
+  };
+  const int pos = a.qkv.q ? *a.qkv.pos_dev : 0;
+  if (ep) {
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+      load_row(b);
+      const int mr = min(b * 16 + (tid >> 4), a.M - 1);
+      cin[b] = LNG && a.cen_in ? a.cen_in[mr] : 0.f;
+      xcn[b] = a.xg_cen ? a.xg_cen[mr] : 0.f;
+    }
   }
   if (nt > 0) {
     if constexpr (ONESHOT) {
@@ -277,16 +308,20 @@ __device__ __forceinline__ void bgemv_unit(const BgemvArgs& a, int g, int s, flo
       }
     }
   }
-  // partial D of this wave: element (m = 4q + i, n = r) at m*16 + n
+  // partial D of this wave: element (m = 4q + i, n = r) of row block b, panel j
+  // at red[b * NPW + j][m * 16 + n]
+  constexpr int NB = MB * NPW;
 #pragma unroll
-  for (int j = 0; j < NPW; ++j)
+  for (int b = 0; b < MB; ++b)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][j][(4 * q + i) * 16 + r] = acc[j][i];
+    for (int j = 0; j < NPW; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[wave][b * NPW + j][(4 * q + i) * 16 + r] = acc[b][j][i];
   __syncthreads();
   // this workgroup's sum over its waves, in wave order; thread tid owns element tid
-  float v[NPW];
+  float v[NB];
 #pragma unroll
-  for (int j = 0; j < NPW; ++j) {
+  for (int j = 0; j < NB; ++j) {
     float t = 0.f;
     if (ep) {
       t = red[0][j][tid];
@@ -298,10 +333,10 @@ __device__ __forceinline__ void bgemv_unit(const BgemvArgs& a, int g, int s, flo
   if (a.S > 1) {
     // publish the workgroup partial (device-scope stores, complete before the
     // count), then the last of the S workgroups of this group sums them
-    float* pg = a.part + ((size_t)g * a.S + s) * NPW * 256;
+    float* pg = a.part + ((size_t)g * a.S + s) * NB * 256;
     if (ep) {
 #pragma unroll
-      for (int j = 0; j < NPW; ++j)
+      for (int j = 0; j < NB; ++j)
         __hip_atomic_store(pg + j * 256 + tid, v[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the stores have completed
@@ -316,18 +351,18 @@ __device__ __forceinline__ void bgemv_unit(const BgemvArgs& a, int g, int s, flo
     if (!is_last) return;
     // all S partials in flight together (device-scope round trips), then
     // summed in split order
-    const float* pb = a.part + (size_t)g * a.S * NPW * 256;
+    const float* pb = a.part + (size_t)g * a.S * NB * 256;
     if (ep) {
-      float pv[SMAX][NPW];
+      float pv[SMAX][NB];
 #pragma unroll
       for (int ss = 0; ss < SMAX; ++ss)
 #pragma unroll
-        for (int j = 0; j < NPW; ++j)
-          pv[ss][j] = ss < a.S ? __hip_atomic_load(const_cast<float*>(pb) + ((size_t)ss * NPW + j) * 256 + tid,
+        for (int j = 0; j < NB; ++j)
+          pv[ss][j] = ss < a.S ? __hip_atomic_load(const_cast<float*>(pb) + ((size_t)ss * NB + j) * 256 + tid,
                                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                                : 0.f;
 #pragma unroll
-      for (int j = 0; j < NPW; ++j) {
+      for (int j = 0; j < NB; ++j) {
         float t = pv[0][j];
 #pragma unroll
         for (int ss = 1; ss < SMAX; ++ss)
@@ -341,49 +376,48 @@ __device__ __forceinline__ void bgemv_unit(const BgemvArgs& a, int g, int s, flo
     __syncthreads();  // the LDS partials are free again once the epilogue threads read them
     return;
   }
-  float mean = 0.f, inv_std = 0.f, mc = 0.f;
-  if constexpr (LNG) {
-    row_stats_merge(a, lnp, mean, inv_std);
-    // the input was centred on cen_in[m]: only the drift of the mean remains
-    mc = mean - (a.cen_in && m < a.M ? a.cen_in[m] : 0.f);
-    if (a.cen_out && g == 0 && (tid & 15) == 0 && m < a.M) a.cen_out[m] = mean;
-  }
-  const float xc = a.xg_cen && m < a.M ? a.xg_cen[m] : 0.f;
-  if (!early) {
 #pragma unroll
-    for (int j = 0; j < NPW; ++j) eo[j] = load_epi(a, m, (g * NPW + j) * 16 + (tid & 15), LNG);
-  }
-  const int pos = a.qkv.q ? *a.qkv.pos_dev : 0;
-  float y[NPW];
-  bool valid[NPW];
-  u64 best = 0ull;
+  for (int b = 0; b < MB; ++b) {
+    const int m = b * 16 + (tid >> 4);
+    float mean = 0.f, inv_std = 0.f, mc = 0.f;
+    if constexpr (LNG) {
+      row_stats_merge(a, lnp[b], mean, inv_std);
+      // the input was centred on cen_in[m]: only the drift of the mean remains
+      mc = mean - cin[b];
+      if (a.cen_out && g == 0 && (tid & 15) == 0 && m < a.M) a.cen_out[m] = mean;
+    }
+    const float xc = xcn[b];
+    float y[NPW];
+    bool valid[NPW];
+    u64 best = 0ull;
 #pragma unroll
-  for (int j = 0; j < NPW; ++j) {
-    const int n = (g * NPW + j) * 16 + (tid & 15);
-    valid[j] = m < a.M && n < a.N;
-    y[j] = 0.f;
-    if (valid[j]) {
-      float t = v[j];
-      if constexpr (LNG) t = inv_std * (t - mc * eo[j].ln_s);
-      y[j] = store_out(a, m, n, t, eo[j], pos, TK);
-      if (a.xg) a.xg[xt_index(m, n, a.M, TK)] = (y[j] - xc) * eo[j].g_next;
-      if (a.keys) {
-        const u64 k = argmax_key(y[j], (uint32_t)n);
-        best = k > best ? k : best;
+    for (int j = 0; j < NPW; ++j) {
+      const int n = (g * NPW + j) * 16 + (tid & 15);
+      valid[j] = m < a.M && n < a.N;
+      y[j] = 0.f;
+      if (valid[j]) {
+        float t = v[b * NPW + j];
+        if constexpr (LNG) t = inv_std * (t - mc * eo[b][j].ln_s);
+        y[j] = store_out(a, m, n, t, eo[b][j], pos, TK);
+        if (a.xg) a.xg[xt_index(m, n, a.M, TK)] = (y[j] - xc) * eo[b][j].g_next;
+        if (a.keys) {
+          const u64 k = argmax_key(y[j], (uint32_t)n);
+          best = k > best ? k : best;
+        }
       }
     }
-  }
-  if (a.stats_part) row_stats_partial<NPW>(a, g, y, valid);
-  if (a.keys) {
-    // greedy argmax of the LM head: the row's best key over this unit, then
-    // one device-scope atomic max per row
+    if (a.stats_part) row_stats_partial<NPW>(a, g, m, y, valid);
+    if (a.keys) {
+      // greedy argmax of the LM head: the row's best key over this unit, then
+      // one device-scope atomic max per row
 #pragma unroll
-    for (int o = 8; o > 0; o >>= 1) {
-      const u64 other = __shfl_xor(best, o, 64);
-      best = other > best ? other : best;
+      for (int o = 8; o > 0; o >>= 1) {
+        const u64 other = __shfl_xor(best, o, 64);
+        best = other > best ? other : best;
+      }
+      if ((tid & 15) == 0 && m < a.M && best != 0ull)
+        __hip_atomic_fetch_max(a.keys + m, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if ((tid & 15) == 0 && m < a.M && best != 0ull)
-      __hip_atomic_fetch_max(a.keys + m, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
 }

@@ -98,7 +98,8 @@ struct BatchedWeights {
   std::vector<Layer> layers;
   const void* lm = nullptr;  // tiled wte (the tied LM head)
   const float *sl = nullptr, *cl = nullptr;  // ln_f into the LM head
-  BgemvPlan pq{}, pp{}, pf{}, pm{}, pl{};    // c_attn, attn c_proj, c_fc, mlp c_proj, LM head
+  BgemvPlan pq{}, pp{}, pf{}, pm{};          // c_attn, attn c_proj, c_fc, mlp c_proj
+  BgemvPlan pl[2]{};                         // LM head: up to 16 sequences, and more
   ~BatchedWeights() {
     if (arena) hipFree(arena);
   }
@@ -180,7 +181,7 @@ struct rtg_cache {
   float* bg_part = nullptr;
   unsigned* bg_cnt = nullptr;
   float* bg_spart = nullptr;
-  float* bg_cen = nullptr;  // [2][16]: per-row centres of the folded LayerNorms' inputs
+  float* bg_cen = nullptr;  // [2][kBgemvRows]: per-row centres of the folded LayerNorms' inputs
 };
 
 static void free_work(rtg_cache* c) {
@@ -407,11 +408,11 @@ static void enqueue_prefill(rtg_cache* c, const Work& w, const uint32_t* ids_dev
 // ---- batched decode step on the tile-ordered GEMV (bgemv.h) ----
 
 // The batched step needs every GEMV's K to be a whole number of k-tiles and at
-// most 16 sequences; other shapes keep the per-op kernels below.
+// most kBgemvRows sequences; other shapes keep the per-op kernels below.
 static bool batched_ok(const rtg_model* m, size_t B) {
   const size_t tk = m->wtype == W_F32 ? 16 : 32;
   // (the LayerNorm statistics of a row come in at most 128 panel groups)
-  return B >= 1 && B <= 16 && m->cfg.n_embd % tk == 0 && m->cfg.n_embd <= 2048;
+  return B >= 1 && B <= (size_t)kBgemvRows && m->cfg.n_embd % tk == 0 && m->cfg.n_embd <= 2048;
 }
 
 // Builds the model's tile-ordered weight copies and folded LayerNorm constants
@@ -466,7 +467,11 @@ static const BatchedWeights* ensure_batched(const rtg_model* mc) {
   bw->pp = bgemv_plan(d, d, wt);
   bw->pf = bgemv_plan(4 * d, d, wt);
   bw->pm = bgemv_plan(d, 4 * d, wt);
-  bw->pl = bgemv_plan(V, d, wt);
+  bw->pl[0] = bgemv_plan(V, d, wt);
+  // more than 16 rows: two panels per wave share each load of x (GPT-2 small
+  // f32, 24 sequences: 532 us per step against 550 with one and 539 with four;
+  // XL bf16: 508 against 516 with four)
+  bw->pl[1] = bgemv_plan(V, d, wt, 2);
   m->bw = std::move(bw);
   return m->bw.get();
 }
@@ -475,14 +480,14 @@ static const BatchedWeights* ensure_batched(const rtg_model* mc) {
 static void ensure_bg_work(rtg_cache* c, const BatchedWeights* bw) {
   if (c->bg_part) return;
   size_t part = 1, groups = 1;
-  for (const BgemvPlan* pl : {&bw->pq, &bw->pp, &bw->pf, &bw->pm, &bw->pl}) {
-    part = std::max(part, bgemv_work_floats(*pl));
+  for (const BgemvPlan* pl : {&bw->pq, &bw->pp, &bw->pf, &bw->pm, &bw->pl[c->batch > 16]}) {
+    part = std::max(part, bgemv_work_floats(*pl, (int)c->batch));
     groups = std::max(groups, (size_t)pl->groups);
   }
   HIPX(hipMalloc(&c->bg_part, part * 4));
   HIPX(hipMalloc(&c->bg_cnt, groups * 4));
-  HIPX(hipMalloc(&c->bg_spart, groups * 16 * 2 * 4));
-  HIPX(hipMalloc(&c->bg_cen, 2 * 16 * 4));
+  HIPX(hipMalloc(&c->bg_spart, groups * kBgemvRows * 2 * 4));
+  HIPX(hipMalloc(&c->bg_cen, 2 * kBgemvRows * 4));
   HIPX(hipMemsetAsync(c->bg_cnt, 0, groups * 4, c->stream));
   HIPX(hipStreamSynchronize(c->stream));
 }
@@ -527,7 +532,7 @@ static void enqueue_decode_step_batched(rtg_cache* c) {
   // epilogue after it centres the next input on that mean, so the fold only
   // ever subtracts the drift of the mean between two LayerNorms.
   float* cen_cur = c->bg_cen;
-  float* cen_next = c->bg_cen + 16;
+  float* cen_next = c->bg_cen + kBgemvRows;
   if (!launch_embed_stats(s, m->wte, m->wtype, m->wpe, c->token_dev, c->pos_dev, B, d, c->x, c->bg_spart,
                           NL ? m->layers[0].ln1w : m->lnfw, c->ln, cen_cur))
     throw HipError{"embed_stats launch failed"};
@@ -537,7 +542,7 @@ static void enqueue_decode_step_batched(rtg_cache* c) {
     a.ln_g = g; a.ln_s = sv; a.ln_part = c->bg_spart; a.ln_groups = st_groups; a.ln_cols = st_cols;
     a.cen_in = cen_cur;
     if (record) {
-      cen_next = cen_cur == c->bg_cen ? c->bg_cen + 16 : c->bg_cen;
+      cen_next = cen_cur == c->bg_cen ? c->bg_cen + kBgemvRows : c->bg_cen;
       a.cen_out = cen_next;
     }
   };
@@ -590,7 +595,7 @@ static void enqueue_decode_step_batched(rtg_cache* c) {
     a.X = c->ln; a.Wt = bw->lm; a.N = V; a.K = d; a.bias = bw->cl;
     ln_in(a, m->lnfw, bw->sl, false);
     a.C = c->logits; a.ldc = V; a.epi = EPI_BIAS;
-    run(bw->pl, a);
+    run(bw->pl[B > 16], a);
   }
   // (the argmax in the LM head's epilogue, a per-row atomic max per
   // workgroup, was measured slower than this separate kernel)
