@@ -20,7 +20,12 @@ LIB = os.path.join(LIBDIR, "librtgpu.so")
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # -packed-fp32-ops: keep the compiler from emitting packed fp32 VALU ops.
-DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# -amdgpu-kernarg-preload-count: a kernel's leading scalar arguments arrive in
+# SGPRs with the launch, so its first loads do not wait for a read of the
+# argument segment (the batched decode step's short kernels: 356 -> 348 us per
+# step of GPT-2 small f32 at 8 sequences, 385 -> 372 us of 8 XL bf16 layers at 16).
+DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm",
+                "-amdgpu-kernarg-preload-count=14"]
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function", f"-I{os.path.join(PKG, '..', 'include')}"]
 
 SOURCES = ["kernels.hip", "gemm_pair.hip", "decode_persistent.hip", "decode_persistent_inst_mini.hip",

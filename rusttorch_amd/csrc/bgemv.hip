@@ -56,8 +56,16 @@ __global__ void tile_weights_kernel(const void* __restrict__ src, int wtype, int
   reinterpret_cast<u4v*>(dst)[i] = v;
 }
 
+// (what the first loads need comes first and as scalars: preloaded into SGPRs)
 template <int WT, int NPW, bool LNG, int MB, int DEPTH, bool ONESHOT>
-__global__ __launch_bounds__(64 * BG_NW) void bgemv_kernel(BgemvArgs a) {
+__global__ __launch_bounds__(64 * BG_NW) void bgemv_kernel(const void* Wt, const float* X, int M, int N, int K, int ktc,
+                                                            BgemvArgs a) {
+  a.Wt = Wt;
+  a.X = X;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.ktc = ktc;
   __shared__ float red[BG_NW][MB * NPW][256];
   __shared__ unsigned last;
   bgc::bgemv_unit<WT, NPW, LNG, BG_NW, MB, DEPTH, ONESHOT>(a, blockIdx.x, blockIdx.y, red, &last);
@@ -72,17 +80,17 @@ void launch_depth(hipStream_t s, dim3 grid, const BgemvArgs& a) {
   const dim3 block(64 * BG_NW);
   if constexpr (per_tile * 8 <= 160) {
     if (a.ktc <= 8) {
-      bgemv_kernel<WT, NPW, LNG, MB, 8, true><<<grid, block, 0, s>>>(a);
+      bgemv_kernel<WT, NPW, LNG, MB, 8, true><<<grid, block, 0, s>>>(a.Wt, a.X, a.M, a.N, a.K, a.ktc, a);
       return;
     }
   }
   if constexpr (per_tile * 12 <= 160) {
     if (a.ktc <= 12) {
-      bgemv_kernel<WT, NPW, LNG, MB, 12, true><<<grid, block, 0, s>>>(a);
+      bgemv_kernel<WT, NPW, LNG, MB, 12, true><<<grid, block, 0, s>>>(a.Wt, a.X, a.M, a.N, a.K, a.ktc, a);
       return;
     }
   }
-  bgemv_kernel<WT, NPW, LNG, MB, 4, false><<<grid, block, 0, s>>>(a);
+  bgemv_kernel<WT, NPW, LNG, MB, 4, false><<<grid, block, 0, s>>>(a.Wt, a.X, a.M, a.N, a.K, a.ktc, a);
 }
 
 template <int WT, int NPW>
