@@ -181,6 +181,7 @@ struct rtg_cache {
   float* bg_part = nullptr;
   unsigned* bg_cnt = nullptr;
   float* bg_spart = nullptr;
+  void* sample_work = nullptr;  // of launch_sample, made for the first sampled token
   float* bg_cen = nullptr;  // [2][kBgemvRows]: per-row centres of the folded LayerNorms' inputs
 };
 
@@ -242,6 +243,10 @@ static void ensure_logits(rtg_cache* c, size_t rows) {
   size_t cap = std::max<size_t>(rows, 16);
   HIPX(hipMalloc(&c->logits, cap * c->m->cfg.vocab_size * 4));
   c->logit_rows_cap = cap;
+}
+
+static void ensure_sample_work(rtg_cache* c) {
+  if (!c->sample_work) HIPX(hipMalloc(&c->sample_work, sample_work_bytes((int)c->m->cfg.vocab_size)));
 }
 
 static rtg_cache* cache_create(const rtg_model* m, size_t batch) {
@@ -809,10 +814,12 @@ static void generate_greedy(const rtg_model* m, const uint32_t* prompts, size_t 
   const bool rows = rows_path(c, B, n);
   ensure_rows(c, B * n);
   ensure_logits(c, rows ? B * n : B);
+  if (sp) ensure_sample_work(c);
   hipStream_t s = c->stream;
   // overwrite the argmax token of the step just enqueued with the sampler's choice
   auto sample = [&](const float* row) {
-    if (sp && !launch_sample(s, row, (int)V, c->ids_in, (int)n, c->ids_dev, c->step_dev, *sp, c->token_dev))
+    if (sp && !launch_sample(s, row, (int)V, c->ids_in, (int)n, c->ids_dev, c->step_dev, *sp, c->token_dev,
+                             c->sample_work))
       throw HipError{"vocabulary too large for the device sampler"};
   };
   if (!c->pstate && persistent_supported(m->pplan, (int)B)) {
@@ -1309,7 +1316,8 @@ void rtg_cache_destroy(rtg_cache* c) {
   free_work(c);
   for (void* p : {(void*)c->k, (void*)c->v, (void*)c->pos_dev, (void*)c->step_dev, (void*)c->keys,
                   (void*)c->token_dev, (void*)c->ids_dev, (void*)c->ids_in, (void*)c->logits,
-                  (void*)c->bg_part, (void*)c->bg_cnt, (void*)c->bg_spart, (void*)c->bg_cen})
+                  (void*)c->bg_part, (void*)c->bg_cnt, (void*)c->bg_spart, (void*)c->bg_cen,
+                  c->sample_work})
     if (p) hipFree(p);
   for (auto e : c->ev)
     if (e) hipEventDestroy(e);
@@ -1566,6 +1574,7 @@ rtg_result rtg_generate(const rtg_model* model, const uint32_t* prompt, size_t n
     c->len = 0;
     ensure_rows(c, std::min(total - 1, P));
     ensure_logits(c, 1);
+    ensure_sample_work(c);
     // sample_with_temperature (gpt2.rs:996-1017); argmax for temperature <= 0.
     // Draw k of the seeded sequence goes to generation index k - 1.
     const SampleParams sp{temperature, 0, 1.0f, 1.0f, seed, 0};
@@ -1573,7 +1582,8 @@ rtg_result rtg_generate(const rtg_model* model, const uint32_t* prompt, size_t n
       const size_t len = n + i;
       const size_t start = len > P ? len - P : 0;
       enqueue_prefill(c, cache_work(c), toks + start, 1, len - start, 0, LOGITS_LAST);
-      if (!launch_sample(s, c->logits, (int)V, toks, (int)n, toks + n, steps + i, sp, c->token_dev))
+      if (!launch_sample(s, c->logits, (int)V, toks, (int)n, toks + n, steps + i, sp, c->token_dev,
+                         c->sample_work))
         throw HipError{"vocabulary too large for the device sampler"};
     }
     HIPX(hipMemcpyAsync(out, toks, total * 4, hipMemcpyDeviceToHost, s));

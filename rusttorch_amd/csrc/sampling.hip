@@ -4,7 +4,8 @@
 // repetition penalty (:872-880); and sample_with_temperature (:996-1017),
 // which is sample_logits without penalty and filters.
 //
-// One workgroup of 512 threads per sequence. Element i is held in a register
+// The general form (sample_whole): one workgroup of 512 threads per sequence.
+// Element i is held in a register
 // of thread i % 512 (row i / 512: the row index is the register index, so
 // the load is one coalesced sweep and every later pass works on registers).
 // The work is VALU-bound on the one CU, so every pass over the row is kept to
@@ -366,16 +367,13 @@ __device__ __forceinline__ void apply_penalty(float (&v)[NJ], const float* logit
   }
 }
 
-}  // namespace
-
+// The token of generation index g by passes over the whole row, on this
+// workgroup alone.
 template <int NJ>
-__global__ __launch_bounds__(ST) void sample_kernel(const float* __restrict__ logits, int V,
-                                                    const uint32_t* __restrict__ prompt, int n_prompt,
-                                                    uint32_t* __restrict__ ids, const int* __restrict__ step_dev,
-                                                    SampleParams sp, uint32_t* __restrict__ token) {
-  __shared__ SampleSmem sm;
+__device__ __forceinline__ uint32_t sample_whole(const float* __restrict__ logits, int V, const uint32_t* __restrict__ prompt,
+                                 int n_prompt, const uint32_t* __restrict__ ids, int g, const SampleParams& sp,
+                                 SampleSmem& sm) {
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const int g = *step_dev - 1;  // generation index of the token being chosen
   // v[j] = element j * ST + t ("row" j), in registers for all passes
   float v[NJ];
 #pragma unroll
@@ -598,23 +596,424 @@ __global__ __launch_bounds__(ST) void sample_kernel(const float* __restrict__ lo
       pick = sm.misc[4];
     }
   }
+  return pick;
+}
+
+// ---- the same choice over many workgroups and few candidates ----
+//
+// sample_segments_kernel: workgroup b takes 1024 consecutive logits, applies
+// the penalty and the temperature, and leaves the scaled logits y and, per
+// segment of 64 consecutive ones, their maximum and their sum of
+// exp(y - maximum). sample_pick_kernel, one workgroup, then reads the <= 1024
+// segment records and only the segments that matter:
+//  - top-k: a segment whose maximum is below k others' holds none of the k
+//    largest, so about k segments are read (those that reach a bound just
+//    below the k-th largest maximum); of these, values below the bound are
+//    dropped. What is left (about k values) is ranked by comparing all pairs, for top-k (fewer than k
+//    larger) and for top-p (the mass ranked before it below p, the rule of the
+//    histogram rounds above: masses are integers).
+//  - no filter: the segment where the running sum passes the draw.
+//  - greedy: the segments' best keys.
+// More candidates than fit (many ties), infinities and NaN take the passes
+// over the whole row above, in the same launch.
+// One workgroup's VALU and LDS atomics bounded the whole-row passes: GPT-2's
+// 50257 logits with top-k 50, top-p 0.95 and a penalty took 73 us per token, now
+// 5.3 (segments) + 17.3 (pick), most of the latter the latency of its own
+// instruction fetches and of the chain of LDS and memory round trips.
+constexpr int SEG = 64, SEGS_MAX = MAX_ROWS * ST / SEG;  // 1024
+constexpr int AT = 256, AW = 1024;                       // threads and logits of one segment workgroup
+constexpr int CREG = 16;                                 // candidate values per thread: 8192 in 128 segments
+constexpr int SURV = 512;                                // values ranked
+
+struct SampleWork {
+  float* y;                     // [V] scaled logits
+  float* segmax;                // [segments]
+  float* segsum;                // [segments]; NaN where the segment holds one
+  unsigned long long* segkey;   // [segments] greedy: best argmax key
+};
+
+__host__ __device__ inline size_t align256(size_t x) { return (x + 255) / 256 * 256; }
+__host__ __device__ inline SampleWork sample_work(void* mem, int V) {
+  char* p = static_cast<char*>(mem);
+  const size_t nseg = (size_t)(V + SEG - 1) / SEG;
+  SampleWork w;
+  w.y = reinterpret_cast<float*>(p);
+  p += align256((size_t)V * 4);
+  w.segmax = reinterpret_cast<float*>(p);
+  p += align256(nseg * 4);
+  w.segsum = reinterpret_cast<float*>(p);
+  p += align256(nseg * 4);
+  w.segkey = reinterpret_cast<unsigned long long*>(p);
+  return w;
+}
+
+__global__ __launch_bounds__(AT) void sample_segments_kernel(const float* __restrict__ logits, int V,
+                                                             const uint32_t* __restrict__ prompt, int n_prompt,
+                                                             const uint32_t* __restrict__ ids,
+                                                             const int* __restrict__ step_dev, float temperature,
+                                                             float penalty, SampleWork wk) {
+  __shared__ unsigned cnt[AW];
+  constexpr int R = AW / AT;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int base = blockIdx.x * AW, first = base + wave * (R * 64);
+  float x[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) x[r] = logits[min(first + r * 64 + lane, V - 1)];
+  if (penalty != 1.0f) {
+    // gpt2.rs:909-921, once per occurrence of a token in the history
+    const int nh = n_prompt + *step_dev - 1;
+#pragma unroll
+    for (int i = 0; i < R; ++i) cnt[t + i * AT] = 0u;
+    __syncthreads();
+    for (int q = t; q < nh; q += AT) {
+      const uint32_t off = hist_at(prompt, n_prompt, ids, q) - (uint32_t)base;
+      if (off < (uint32_t)AW) atomicAdd(&cnt[off], 1u);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      for (unsigned z = cnt[wave * (R * 64) + r * 64 + lane]; z > 0; --z)
+        x[r] = x[r] > 0.0f ? x[r] / penalty : x[r] * penalty;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = first + r * 64 + lane, seg = i / SEG;
+    if (first + r * 64 >= V) break;  // wave-uniform
+    if (temperature <= 0.0f) {
+      unsigned long long k = i < V ? argmax_key(x[r], (uint32_t)i) : 0ull;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long u = __shfl_xor(k, o, 64);
+        k = u > k ? u : k;
+      }
+      if (lane == 0) wk.segkey[seg] = k;
+      continue;
+    }
+    const float y = i < V ? x[r] / temperature : -INFINITY;
+    if (i < V) wk.y[i] = y;
+    const float m = wave_max_s(y);
+    float e = y > -INFINITY ? expf(y - m) : 0.f;
+    if (y != y) e = y;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
+    if (lane == 0) {
+      wk.segmax[seg] = m;
+      wk.segsum[seg] = e;
+    }
+  }
+}
+
+struct PickSmem {
+  float segmax[SEGS_MAX];
+  float seg[SEGS_MAX];     // sums in index order (segments, or survivors) and
+  float segpre[SEGS_MAX];  // their exclusive prefix
+  uint16_t cand[SEGS_MAX];
+  float val[SURV];
+  uint32_t idx[SURV];
+  unsigned mass[SURV];
+  float red[2 * SW];
+  unsigned wtot[SW];
+  float fmisc[2];
+  unsigned misc[2];
+};
+
+// Exclusive prefix over the block in thread order (as block_excl_scan).
+__device__ __forceinline__ unsigned pick_scan(unsigned x, PickSmem& sm, unsigned* total) {
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  unsigned incl = x;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned u = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += u;
+  }
+  __syncthreads();
+  if (lane == 63) sm.wtot[w] = incl;
+  __syncthreads();
+  unsigned base = 0, tot = 0;
+#pragma unroll
+  for (int i = 0; i < SW; ++i) {
+    if (i == w) base = tot;
+    tot += sm.wtot[i];
+  }
+  *total = tot;
+  return base + incl - x;
+}
+
+// The first of n (<= 1024) entries of sm.seg whose running sum exceeds
+// r * (their sum), r a uniform draw; NONE when none does. Every thread gets it
+// (and that entry's exclusive prefix in *before, the threshold in *rs).
+__device__ __forceinline__ uint32_t pick_entry(PickSmem& sm, int n, float r, float* before, float* rs) {
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __syncthreads();
+  if (w == 0) {
+    const float S = wave_excl_prefix(sm.seg, sm.segpre, n, lane);
+    const float lim = r * S;
+    const int per = (n + 63) / 64, b0 = lane * per, e0 = min(n, b0 + per);
+    int found = -1;
+    for (int i = b0; i < e0 && found < 0; ++i)
+      if (lim < sm.segpre[i] + sm.seg[i]) found = i;
+    const unsigned long long bal = __ballot(found >= 0);
+    const int f = bal ? __shfl(found, __builtin_ctzll(bal), 64) : -1;
+    if (lane == 0) {
+      sm.misc[0] = f < 0 ? NONE : (unsigned)f;
+      sm.fmisc[0] = f < 0 ? 0.f : sm.segpre[f];
+      sm.fmisc[1] = lim;
+    }
+  }
+  __syncthreads();
+  *before = sm.fmisc[0];
+  *rs = sm.fmisc[1];
+  return sm.misc[0];
+}
+
+// The pick from the segment records; false when the whole row is needed.
+__device__ __forceinline__ bool pick_from_segments(const SampleWork& wk, int V, int g, const SampleParams& sp, PickSmem& sm,
+                                   uint32_t* pick) {
+  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+  const int nseg = (V + SEG - 1) / SEG;
+  // segments 2t and 2t + 1 of this thread
+  float m2[2], s2[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int i = min(2 * t + q, nseg - 1);
+    m2[q] = wk.segmax[i];
+    s2[q] = wk.segsum[i];
+    if (2 * t + q >= nseg) {
+      m2[q] = -INFINITY;
+      s2[q] = 0.f;
+    }
+    sm.segmax[2 * t + q] = m2[q];
+  }
+  float mx = wave_max_s(fmaxf(m2[0], m2[1]));
+  const bool bad = __any(s2[0] != s2[0] || s2[1] != s2[1]);
+  if (lane == 0) {
+    sm.red[w] = mx;
+    sm.red[SW + w] = bad ? 1.f : 0.f;
+  }
+  __syncthreads();
+  float any_bad = 0.f;
+#pragma unroll
+  for (int i = 0; i < SW; ++i) {
+    mx = fmaxf(mx, sm.red[i]);
+    any_bad += sm.red[SW + i];
+  }
+  if (any_bad != 0.f || !(fabsf(mx) < INFINITY)) return false;
+  const float r =
+      (float)(splitmix_at(sp.seed, (uint64_t)sp.draw0 + (uint64_t)g + 1) >> 40) * (1.0f / 16777216.0f);
+  float before, rs;
+  if (sp.top_k <= 0 || sp.top_k >= V) {
+    // ---- temperature only: the segment, then the index inside it ----
+#pragma unroll
+    for (int q = 0; q < 2; ++q) sm.seg[2 * t + q] = s2[q] > 0.f ? s2[q] * expf(m2[q] - mx) : 0.f;
+    const uint32_t seg = pick_entry(sm, nseg, r, &before, &rs);
+    if (seg == NONE) {
+      *pick = (uint32_t)(V - 1);
+      return true;
+    }
+    const int i = (int)seg * SEG + lane;
+    const float y = i < V ? wk.y[i] : -INFINITY;
+    const float p = y > -INFINITY ? expf(y - mx) : 0.f;
+    float incl = p;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const float u = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += u;
+    }
+    const unsigned long long bal = __ballot(i < V && rs < before + incl);
+    // (the running sum may stop short of the segment's by rounding: then its
+    // last index of non-zero probability)
+    const unsigned long long nz = __ballot(p > 0.f);
+    *pick = bal ? seg * SEG + (uint32_t)__builtin_ctzll(bal)
+                : nz ? seg * SEG + 63u - (uint32_t)__builtin_clzll(nz) : (uint32_t)(V - 1);
+    return true;
+  }
+  // ---- top-k: a bound that at least k segments' maxima reach (the top 16
+  // bits of the k-th largest maximum's order key, bit by bit on one wave: all
+  // pairs of maxima took 10 us), and the segments that reach it ----
+  const int k = sp.top_k;
+  if (w == 0) {
+    uint32_t key[SEGS_MAX / 64];
+#pragma unroll
+    for (int j = 0; j < SEGS_MAX / 64; ++j) key[j] = order_key(sm.segmax[64 * j + lane]) >> 16;
+    uint32_t bound = 0;
+#pragma unroll 1
+    for (int bit = 15; bit >= 0; --bit) {
+      const uint32_t next = bound | 1u << bit;
+      int n = 0;
+#pragma unroll
+      for (int j = 0; j < SEGS_MAX / 64; ++j) n += __popcll(__ballot(key[j] >= next));
+      if (n >= k) bound = next;
+    }
+    if (lane == 0) sm.misc[0] = bound;
+  }
+  __syncthreads();
+  const uint32_t bound = sm.misc[0];
+  float low = from_order_key(bound << 16);
+  if (!(low > -INFINITY)) low = -INFINITY;  // (fewer than k finite maxima: they bound nothing)
+  unsigned nc;
+  const bool c0 = 2 * t < nseg && order_key(m2[0]) >> 16 >= bound;
+  const bool c1 = 2 * t + 1 < nseg && order_key(m2[1]) >> 16 >= bound;
+  unsigned at = pick_scan((c0 ? 1u : 0u) + (c1 ? 1u : 0u), sm, &nc);
+  if (c0) sm.cand[at++] = (uint16_t)(2 * t);
+  if (c1) sm.cand[at] = (uint16_t)(2 * t + 1);
+  __syncthreads();
+  if (nc > (unsigned)(CREG * SW)) return false;
+  // candidate c = CREG * wave + j: consecutive per wave, so that survivors
+  // gather in index order
+  float v[CREG];
+  unsigned mine = 0;
+#pragma unroll
+  for (int j = 0; j < CREG; ++j) {
+    const unsigned c = CREG * w + j;
+    v[j] = -INFINITY;
+    if (c < nc) {
+      const int i = (int)sm.cand[c] * SEG + lane;
+      if (i < V) v[j] = wk.y[i];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < CREG; ++j) mine += (unsigned)__popcll(__ballot(v[j] >= low && v[j] > -INFINITY));
+  __syncthreads();
+  if (lane == 0) sm.wtot[w] = mine;
+  __syncthreads();
+  unsigned pos = 0, ns = 0;
+#pragma unroll
+  for (int i = 0; i < SW; ++i) {
+    if (i == w) pos = ns;
+    ns += sm.wtot[i];
+  }
+  if (ns > (unsigned)SURV) return false;
+#pragma unroll
+  for (int j = 0; j < CREG; ++j) {
+    const unsigned long long bal = __ballot(v[j] >= low && v[j] > -INFINITY);
+    if ((bal >> lane) & 1ull) {
+      const unsigned p = pos + (unsigned)lanes_before(bal);
+      sm.val[p] = v[j];
+      sm.idx[p] = (uint32_t)sm.cand[CREG * w + j] * SEG + (uint32_t)lane;
+    }
+    pos += (unsigned)__popcll(bal);
+  }
+  __syncthreads();
+  // top-k over the survivors: all values with fewer than k larger ones
+  const bool have = (unsigned)t < ns;
+  const float yv = have ? sm.val[t] : -INFINITY;
+  int larger = 0;
+#pragma unroll 8
+  for (unsigned i = 0; i < ns; ++i) larger += sm.val[i] > yv;
+  float e = have && larger < k ? expf(yv - mx) : 0.f;
+  if (sp.top_p < 1.0f && sp.top_p > 0.0f) {
+    __syncthreads();
+    sm.seg[t] = e;
+    __syncthreads();
+    if (w == 0) {
+      const float S = wave_excl_prefix(sm.seg, sm.segpre, (int)ns, lane);
+      if (lane == 0) sm.fmisc[0] = S;
+    }
+    __syncthreads();
+    const float ms = 2147483648.0f / sm.fmisc[0];
+    const unsigned target = max(1u, (unsigned)(sp.top_p * 2147483648.0f));
+    if (have) sm.mass[t] = mass_of(e, ms);
+    __syncthreads();
+    unsigned before_mass = 0;
+#pragma unroll 8
+    for (unsigned i = 0; i < ns; ++i) {
+      const float o = sm.seg[i];
+      if (o > e || (o == e && i < (unsigned)t)) before_mass += sm.mass[i];
+    }
+    if (before_mass >= target) e = 0.f;
+    __syncthreads();
+  }
+  __syncthreads();
+  if (have) sm.seg[t] = e;
+  const uint32_t f = pick_entry(sm, (int)ns, r, &before, &rs);
+  *pick = f == NONE ? (uint32_t)(V - 1) : sm.idx[f];
+  return true;
+}
+
+template <int NJ>
+__global__ __launch_bounds__(ST) void sample_kernel(const float* __restrict__ logits, int V,
+                                                    const uint32_t* __restrict__ prompt, int n_prompt,
+                                                    uint32_t* __restrict__ ids, const int* __restrict__ step_dev,
+                                                    SampleParams sp, uint32_t* __restrict__ token) {
+  __shared__ SampleSmem sm;
+  const int g = *step_dev - 1;  // generation index of the token being chosen
+  const uint32_t pick = sample_whole<NJ>(logits, V, prompt, n_prompt, ids, g, sp, sm);
+  if (threadIdx.x == 0) {
+    token[0] = pick;
+    ids[g] = pick;
+  }
+}
+
+template <int NJ>
+__global__ __launch_bounds__(ST) void sample_pick_kernel(const float* __restrict__ logits, int V,
+                                                         const uint32_t* __restrict__ prompt, int n_prompt,
+                                                         uint32_t* __restrict__ ids,
+                                                         const int* __restrict__ step_dev, SampleParams sp,
+                                                         uint32_t* __restrict__ token, SampleWork wk) {
+  __shared__ __attribute__((aligned(16))) union {
+    SampleSmem whole;
+    PickSmem part;
+  } sm;
+  const int t = threadIdx.x, lane = t & 63;
+  const int g = *step_dev - 1;  // generation index of the token being chosen
+  uint32_t pick = 0;
+  if (sp.temperature <= 0.0f) {
+    const int nseg = (V + SEG - 1) / SEG;
+    unsigned long long k = 0ull;
+    for (int i = t; i < nseg; i += ST) k = wk.segkey[i] > k ? wk.segkey[i] : k;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const unsigned long long u = __shfl_xor(k, o, 64);
+      k = u > k ? u : k;
+    }
+    if (t == 0) sm.whole.key = 0ull;
+    __syncthreads();
+    if (lane == 0) atomicMax(&sm.whole.key, k);
+    __syncthreads();
+    pick = argmax_key_index(sm.whole.key);
+  } else if (!pick_from_segments(wk, V, g, sp, sm.part, &pick)) {
+    __syncthreads();
+    pick = sample_whole<NJ>(logits, V, prompt, n_prompt, ids, g, sp, sm.whole);
+  }
   if (t == 0) {
     token[0] = pick;
     ids[g] = pick;
   }
 }
 
+}  // namespace
+
+size_t sample_work_bytes(int V) {
+  const size_t nseg = (size_t)(V + SEG - 1) / SEG;
+  return align256((size_t)V * 4) + 2 * align256(nseg * 4) + align256(nseg * 8);
+}
+
 bool launch_sample(hipStream_t s, const float* logits, int V, const uint32_t* prompt, int n_prompt, uint32_t* ids,
-                   const int* step_dev, const SampleParams& sp, uint32_t* token) {
-#define RTG_SAMPLE(NJ) sample_kernel<NJ><<<1, ST, 0, s>>>(logits, V, prompt, n_prompt, ids, step_dev, sp, token)
-  if (V <= 0) return false;
+                   const int* step_dev, const SampleParams& sp, uint32_t* token, void* work) {
+  if (V <= 0 || V > MAX_ROWS * ST) return false;
+  // Segments for rows that one workgroup takes long over, unless top-p alone
+  // filters (its kept set is not small) or top-k keeps more than the ranking
+  // is made for.
+  const bool top_k = sp.top_k > 0 && sp.top_k < V, top_p = sp.top_p < 1.0f && sp.top_p > 0.0f;
+  const bool segments =
+      work != nullptr && V > 4 * ST && (sp.temperature <= 0.0f || (top_k ? sp.top_k <= SURV / 4 : !top_p));
+  const SampleWork wk = sample_work(work, V);
+  if (segments)
+    sample_segments_kernel<<<(V + AW - 1) / AW, AT, 0, s>>>(logits, V, prompt, n_prompt, ids, step_dev,
+                                                            sp.temperature, sp.penalty, wk);
+#define RTG_SAMPLE(NJ)                                                                                         \
+  do {                                                                                                         \
+    if (segments)                                                                                              \
+      sample_pick_kernel<NJ><<<1, ST, 0, s>>>(logits, V, prompt, n_prompt, ids, step_dev, sp, token, wk);      \
+    else                                                                                                       \
+      sample_kernel<NJ><<<1, ST, 0, s>>>(logits, V, prompt, n_prompt, ids, step_dev, sp, token);               \
+  } while (0)
   if (V <= 1 * ST) RTG_SAMPLE(1);
   else if (V <= 4 * ST) RTG_SAMPLE(4);
   else if (V <= 16 * ST) RTG_SAMPLE(16);
   else if (V <= 64 * ST) RTG_SAMPLE(64);
   else if (V <= 100 * ST) RTG_SAMPLE(100);  // GPT-2's 50257 tokens
-  else if (V <= 128 * ST) RTG_SAMPLE(128);
-  else return false;
+  else RTG_SAMPLE(128);
 #undef RTG_SAMPLE
   return true;
 }
