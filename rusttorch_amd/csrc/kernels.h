@@ -77,6 +77,16 @@ void launch_argmax(hipStream_t s, const float* logits, long ld, int rows, int V,
 // keys reset; *pos_dev += 1; *step_dev += 1; *epoch += 1 when given.
 void launch_finalize(hipStream_t s, int B, unsigned long long* keys, uint32_t* token, uint32_t* ids_out, int ld_ids,
                      int* pos_dev, int* step_dev, unsigned* epoch = nullptr);
+// Sets a step's inputs: token[b] = ids[b] for b < B (0: unchanged), *pos_dev =
+// pos, *step_dev = step, in one launch with the values as kernel arguments.
+constexpr int kStepIds = 32;
+struct StepIds {
+  uint32_t id[kStepIds];
+};
+void launch_set_step(hipStream_t s, uint32_t* token, int* pos_dev, int pos, int* step_dev, int step, int B = 0,
+                     const StepIds& ids = StepIds{});
+// Copies n words, then *extra (when given) to dst[n], by stores to host memory.
+void launch_copy_out(hipStream_t s, const uint32_t* src, size_t n, const unsigned* extra, uint32_t* dst);
 // Extract tokens from keys without touching counters (prefill).
 void launch_keys_to_tokens(hipStream_t s, int B, unsigned long long* keys, uint32_t* token);
 void launch_reset_keys(hipStream_t s, int B, unsigned long long* keys);

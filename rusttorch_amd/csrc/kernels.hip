@@ -10,6 +10,8 @@
 #include <stdint.h>
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include "argmax_key.h"
 #include "attn_core.h"
 #include "f16_pair.h"
@@ -565,6 +567,31 @@ __global__ __launch_bounds__(256) void finalize_kernel(int B, unsigned long long
     *step_dev = step + 1;
     if (epoch) *epoch = ep + 1u;
   }
+}
+
+__global__ __launch_bounds__(64) void set_step_kernel(uint32_t* token, int* pos_dev, int* step_dev, int pos, int step,
+                                                      int B, StepIds ids) {
+  const int t = threadIdx.x;
+  if (t == 0) {
+    *pos_dev = pos;
+    *step_dev = step;
+  }
+  if (t < B) token[t] = ids.id[t];
+}
+void launch_set_step(hipStream_t s, uint32_t* token, int* pos_dev, int pos, int* step_dev, int step, int B,
+                     const StepIds& ids) {
+  set_step_kernel<<<1, 64, 0, s>>>(token, pos_dev, step_dev, pos, step, B, ids);
+}
+
+__global__ __launch_bounds__(256) void copy_out_kernel(const uint32_t* __restrict__ src, size_t n,
+                                                       const unsigned* __restrict__ extra,
+                                                       uint32_t* __restrict__ dst) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = src[i];
+  if (extra != nullptr && blockIdx.x == 0 && threadIdx.x == 0) dst[n] = *extra;
+}
+void launch_copy_out(hipStream_t s, const uint32_t* src, size_t n, const unsigned* extra, uint32_t* dst) {
+  const size_t blocks = std::max<size_t>(1, std::min<size_t>((n + 255) / 256, 512));
+  copy_out_kernel<<<(unsigned)blocks, 256, 0, s>>>(src, n, extra, dst);
 }
 
 void launch_finalize(hipStream_t s, int B, unsigned long long* keys, uint32_t* token, uint32_t* ids_out, int ld_ids,
