@@ -28,7 +28,7 @@ DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-m
                 "-amdgpu-kernarg-preload-count=14"]
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function", f"-I{os.path.join(PKG, '..', 'include')}"]
 
-SOURCES = ["kernels.hip", "gemm_pair.hip", "decode_persistent.hip", "decode_persistent_inst_mini.hip",
+SOURCES = ["kernels.hip", "gemm_pair.hip", "attn_pair.hip", "decode_persistent.hip", "decode_persistent_inst_mini.hip",
            "decode_persistent_inst_small.hip", "decode_persistent_inst_medium.hip",
            "decode_persistent_inst_large.hip", "rtg_runtime.cpp", "safetensors_reader.cpp",
            "tokenizer.cpp", "sampling.hip", "bgemv.hip", "scratch.hip", "decode_tile.hip", "rows.hip"]

@@ -109,7 +109,8 @@ void launch_kv_append(hipStream_t s, const float* qkv, int S, int T, int past, K
 void launch_gemm_qkv(hipStream_t s, const float* A, int lda, const void* W, int wtype, const float* bias, float* C,
                      long ldc, int M, int K, int S, int T, int past, KvDst kv, float* ws = nullptr,
                      size_t ws_floats = 0);
-// Prefill causal attention for S sequences of T new tokens at offset past: f32
+// Prefill causal attention for S sequences of T new tokens at offset past, any
+// head_dim (attn_pair.h: head_dim 64 in the models the pair GEMM takes): f32
 // rows to out, or with pair set the pair GEMM's input (f16 pairs, scaled).
 void launch_attn_prefill(hipStream_t s, const float* qkv, int S, int T, int past, const float* kc, const float* vc,
                          int n_head, int n_pos, int d, float* out, uint16_t* pair = nullptr,

@@ -21,6 +21,7 @@
 
 #include "../../include/rtgpu.h"
 #include "decode_persistent.h"
+#include "attn_pair.h"
 #include "bgemv.h"
 #include "gemm_pair.h"
 #include "kernels.h"
@@ -279,7 +280,8 @@ struct PrefillWeights {
   void* arena = nullptr;
   struct Layer {
     PairWeights qkv, proj, fc, mproj;
-    const float *s1, *satt, *s2, *sh;  // input scales: LN1, attention output, LN2, gelu output
+    const float *s1, *s2, *sh;  // input scales: LN1, LN2, gelu output
+    AttnScales att;             // v: the attention output's scale too
   };
   std::vector<Layer> layers;
   PairWeights lm;              // wte
@@ -522,8 +524,11 @@ static void enqueue_prefill_pair(rtg_cache* c, const Work& w, const uint32_t* id
     a.kv_T = (int)T;
     a.kv_past = (int)past;
     launch_pair_gemm(s, P.qkv, a);
-    launch_attn_prefill(s, w.qkv, (int)S, (int)T, (int)past, kv.k, kv.v, kv.n_head, kv.n_pos, d, nullptr, att,
-                        P.satt);
+    if (m->hd == 64)
+      launch_attn_pair(s, w.qkv, (int)S, (int)T, (int)past, kv.k, kv.v, kv.n_head, kv.n_pos, d, P.att, att);
+    else
+      launch_attn_prefill(s, w.qkv, (int)S, (int)T, (int)past, kv.k, kv.v, kv.n_head, kv.n_pos, d, nullptr, att,
+                          P.att.v);
     launch_pair_gemm(s, P.proj, args(att, d, L.baproj, w.x, d, EPI_BIAS_RESID));
     launch_layernorm_pair(s, w.x, d, L.ln2w, L.ln2b, eps, M, d, P.s2, ln);
     a = args(ln, d, L.bfc, nullptr, 0, EPI_BIAS_GELU);
@@ -1131,7 +1136,8 @@ static void build_prefill_weights(rtg_model* m) {
   const Shape sh[4] = {{3 * d, d}, {d, d}, {4 * d, d}, {d, 4 * d}};
   size_t total = 256;  // the flag
   for (const Shape& x : sh) total += L * (align_up(pair_weight_bytes(x.N, x.K, wt), 256) + align_up(x.N * 4, 256));
-  total += L * (3 * align_up(d * 4, 256) + align_up(4 * d * 4, 256));
+  const int H = (int)m->cfg.n_head;
+  total += L * (2 * align_up(d * 4, 256) + align_up(3 * d * 4, 256) + align_up(4 * d * 4, 256) + align_up(2 * H * 4, 256));
   total += align_up(pair_weight_bytes(V, d, wt), 256) + align_up((size_t)V * 4, 256) + align_up(d * 4, 256);
   if (hipMalloc(&pw->arena, total) != hipSuccess) {
     hipGetLastError();
@@ -1157,22 +1163,21 @@ static void build_prefill_weights(rtg_model* m) {
     launch_pair_weights(s, W, wt, in_scale, w, bad);
     return w;
   };
-  const size_t wb = wt == W_BF16 ? 2 : 4;
   for (const LayerW& W : m->layers) {
     PrefillWeights::Layer l;
-    float *s1 = floats(d), *satt = floats(d), *s2 = floats(d), *sh4 = floats(4 * d);
+    float *s1 = floats(d), *sqkv = floats(3 * d), *s2 = floats(d), *sh4 = floats(4 * d), *heads = floats(2 * H);
     launch_pair_ln_scale(s, W.ln1w, W.ln1b, d, s1, bad);
     launch_pair_ln_scale(s, W.ln2w, W.ln2b, d, s2, bad);
-    // attention averages value rows: the bound of c_attn's v outputs
-    launch_pair_row_scale(s, static_cast<const char*>(W.wqkv) + 2 * (size_t)d * d * wb, wt, d, d, W.ln1w, W.ln1b,
-                          W.bqkv + 2 * d, satt, bad);
+    // attention averages value rows, so its output has the bound of c_attn's v
+    launch_pair_row_scale(s, W.wqkv, wt, 3 * d, d, W.ln1w, W.ln1b, W.bqkv, sqkv, bad);
+    if (m->hd == 64) launch_head_scale(s, sqkv, H, heads, heads + H);
+    l.att = AttnScales{heads, heads + H, sqkv + 2 * d};
     launch_pair_row_scale(s, W.wfc, wt, 4 * d, d, W.ln2w, W.ln2b, W.bfc, sh4, bad);
     l.s1 = s1;
-    l.satt = satt;
     l.s2 = s2;
     l.sh = sh4;
     l.qkv = weights(W.wqkv, 3 * d, d, s1);
-    l.proj = weights(W.waproj, d, d, satt);
+    l.proj = weights(W.waproj, d, d, l.att.v);
     l.fc = weights(W.wfc, 4 * d, d, s2);
     l.mproj = weights(W.wmproj, d, 4 * d, sh4);
     pw->layers.push_back(l);

@@ -1,5 +1,5 @@
-"""The prefill on f16-pair GEMMs (gemm_pair.hip) through forward_cached, against
-float64 (tests/ref64.py).
+"""The prefill on f16-pair GEMMs and attention (gemm_pair.hip, attn_pair.hip)
+through forward_cached, against float64 (tests/ref64.py).
 
 The bar is the CPU oracle's own distance from float64 on the same model and
 ids (f32 throughout, sums in k order): the library may be at most twice as far
@@ -58,6 +58,8 @@ def check(oracle_lib, sh, sd, m, chunks, batch=1):
     (192, 3, 301, 1, (33,)),          # 32 x 64 tiles, split
     (192, 6, 301, 3, (17,)),          # head_dim 32, 51 rows
     (192, 3, 301, 5, (131, 7)),       # 655 rows, then 35 behind 131 cached
+    (192, 3, 301, 1, (520, 40)),      # attention's keys over 8 waves, then behind 520 cached
+    (192, 3, 301, 90, (33, 34)),      # 64 and 32 queries per attention workgroup
     (768, 12, 515, 1, (65,)),
     (768, 12, 515, 2, (161,)),
     (768, 12, 515, 9, (129,)),        # 64 x 64 and 64 x 128 tiles
