@@ -278,6 +278,7 @@ struct BatchedWeights {
 // scales of the inputs they multiply; built with the model.
 struct PrefillWeights {
   void* arena = nullptr;
+  size_t bytes = 0;
   struct Layer {
     PairWeights qkv, proj, fc, mproj;
     const float *s1, *s2, *sh;  // input scales: LN1, LN2, gelu output
@@ -1122,13 +1123,13 @@ static void generate_greedy(const rtg_model* m, const uint32_t* prompts, size_t 
 // Model construction (gpt2.rs:214-263)
 // ---------------------------------------------------------------------------
 
-// Builds the model's PrefillWeights. Left null where the pair GEMM does not
-// apply (n_embd not a multiple of 64, a negative epsilon), where a weight or a
-// bound of an activation is not finite, or where the copy does not fit the
-// device: the f32-MFMA GEMMs then run the prefill.
-static void build_prefill_weights(rtg_model* m) {
-  const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, L = (int)m->layers.size(), wt = m->wtype;
-  if (d % 64 != 0 || !(m->cfg.layer_norm_epsilon >= 0.f)) return;
+// Memory for the model's PrefillWeights (cfg, wtype and the layer count set).
+// Null where the pair GEMM does not apply (n_embd not a multiple of 64, a
+// negative epsilon) or where the copy does not fit the device: the f32-MFMA
+// GEMMs then run the prefill.
+static std::unique_ptr<PrefillWeights> alloc_prefill_weights(const rtg_model* m) {
+  const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, L = (int)m->cfg.n_layer, wt = m->wtype;
+  if (d % 64 != 0 || !(m->cfg.layer_norm_epsilon >= 0.f)) return nullptr;
   std::unique_ptr<PrefillWeights> pw(new PrefillWeights());
   struct Shape {
     int N, K;
@@ -1140,9 +1141,18 @@ static void build_prefill_weights(rtg_model* m) {
   total += L * (2 * align_up(d * 4, 256) + align_up(3 * d * 4, 256) + align_up(4 * d * 4, 256) + align_up(2 * H * 4, 256));
   total += align_up(pair_weight_bytes(V, d, wt), 256) + align_up((size_t)V * 4, 256) + align_up(d * 4, 256);
   if (hipMalloc(&pw->arena, total) != hipSuccess) {
-    hipGetLastError();
-    return;
+    (void)hipGetLastError();
+    return nullptr;
   }
+  pw->bytes = total;
+  return pw;
+}
+
+// Fills and keeps them, unless a weight or a bound of an activation is not
+// finite.
+static void build_prefill_weights(rtg_model* m, std::unique_ptr<PrefillWeights> pw) {
+  if (!pw) return;
+  const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, H = (int)m->cfg.n_head, wt = m->wtype;
   char* p = static_cast<char*>(pw->arena);
   auto take = [&](size_t n) {
     char* r = p;
@@ -1289,12 +1299,24 @@ rtg_result build_model(const rtg_config* cfg, Lookup& lk, rtg_storage storage, r
   }
   const size_t o_wte = take(V * d * wb), o_wpe = take(P * d * 4), o_lnfw = take(d * 4), o_lnfb = take(d * 4);
   float* staging = nullptr;
+  bool own_staging = false;
+  std::unique_ptr<PrefillWeights> pw;
   try {
     HIPX(hipMalloc(&m->arena, cur));
     m->arena_bytes = cur;
     char* A = reinterpret_cast<char*>(m->arena);
-    size_t stage_max = std::max({V * d, P * d, 4 * d * d});
-    HIPX(hipMalloc(&staging, stage_max * 4));
+    // (uploads pass through the memory of the prefill weights, which are made
+    // last, where it is large enough: allocating 0.26 GB takes ~10 ms)
+    const size_t stage_max = std::max({V * d, P * d, 4 * d * d}) * 4;
+    pw = alloc_prefill_weights(m.get());
+    own_staging = !pw || pw->bytes < stage_max;
+    if (own_staging) {
+      if (hipMalloc(&staging, stage_max) != hipSuccess) {
+        (void)hipGetLastError();
+        pw.reset();  // the load needs the staging, the prefill can do without its copy
+        HIPX(hipMalloc(&staging, stage_max));
+      }
+    } else staging = static_cast<float*>(pw->arena);
     hipStream_t s = nullptr;
     // Tensors go to the device in their own element type; widening,
     // narrowing to the storage type and the transpose run there.
@@ -1360,13 +1382,14 @@ rtg_result build_model(const rtg_config* cfg, Lookup& lk, rtg_storage storage, r
     m->wpe = reinterpret_cast<float*>(A + o_wpe);
     m->lnfw = reinterpret_cast<float*>(A + o_lnfw);
     m->lnfb = reinterpret_cast<float*>(A + o_lnfb);
-    HIPX(hipFree(staging));
-    staging = nullptr;
-    build_prefill_weights(m.get());
+    if (own_staging) HIPX(hipFree(staging));
+    own_staging = false;
+    build_prefill_weights(m.get(), std::move(pw));
   } catch (const HipError& he) {
-    if (staging) hipFree(staging);
-    return err(he.msg);  } catch (const std::exception& ex) {
-    if (staging) hipFree(staging);
+    if (own_staging && staging) hipFree(staging);
+    return err(he.msg);
+  } catch (const std::exception& ex) {
+    if (own_staging && staging) hipFree(staging);
     return err_internal(ex);
   }
   size_t np = V * d + P * d + 2 * d;
