@@ -17,8 +17,9 @@
 // attention output's own, so O / (2^14 l) is the pair GEMM's input as it is.
 // K and V are read from the f32 cache and split while a block is staged in LDS:
 // K rows of 64 hi + 64 lo (256 bytes), V^T rows (one per dim) of 32 hi + 32 lo
-// in the key order above (128 bytes), 16-byte chunks XOR-swizzled so that the
-// operand reads hit distinct banks.
+// in the key order above (128 bytes), 16-byte chunks XOR-swizzled so that the 16
+// lanes of an LDS read cycle cover its 64 banks (K by row % 16: by row % 8 its
+// reads took twice their cycles, 6.20e6 against 6.08e6 in all at 32 x 1024).
 //
 // What bounds it: the vector work around the MFMAs (masks, exponentials,
 // splitting P, K and V), about 1250 cycles per block and wave against 768 of
@@ -83,8 +84,8 @@ struct Stage {
         split2(k[u][r].x * ak, k[u][r].y * ak, &h.x, &l.x);
         split2(k[u][r].z * ak, k[u][r].w * ak, &h.y, &l.y);
         char* p = Ks + row * 256 + (d4 & 4) * 2;
-        *reinterpret_cast<uint2*>(p + (((d4 >> 3) ^ (row & 7)) << 4)) = h;
-        *reinterpret_cast<uint2*>(p + (((8 + (d4 >> 3)) ^ (row & 7)) << 4)) = l;
+        *reinterpret_cast<uint2*>(p + (((d4 >> 3) ^ (row & 15)) << 4)) = h;
+        *reinterpret_cast<uint2*>(p + (((8 + (d4 >> 3)) ^ (row & 15)) << 4)) = l;
       }
       // V^T: the key pair's word in chunk (t, half) of four dims' rows
       const int c = (key >> 4) * 2 + ((key >> 2) & 1), in = ((key >> 3) & 1) * 8 + (key & 3) * 2;
@@ -134,8 +135,8 @@ struct State {
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
       const char* row = Ks + c * 256;
-      const f16x8 kh = *reinterpret_cast<const f16x8*>(row + (((2 * st + hh) ^ (c & 7)) << 4));
-      const f16x8 kl = *reinterpret_cast<const f16x8*>(row + (((8 + 2 * st + hh) ^ (c & 7)) << 4));
+      const f16x8 kh = *reinterpret_cast<const f16x8*>(row + (((2 * st + hh) ^ (c & 15)) << 4));
+      const f16x8 kl = *reinterpret_cast<const f16x8*>(row + (((8 + 2 * st + hh) ^ (c & 15)) << 4));
       s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[st], s, 0, 0, 0);
       s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[st], s, 0, 0, 0);
       s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[st], s, 0, 0, 0);

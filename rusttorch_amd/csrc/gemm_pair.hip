@@ -18,8 +18,12 @@
 //
 // A workgroup computes BM x BN outputs from k-tiles of 32: LDS rows of 128
 // bytes [32 hi][32 lo] (64 bytes for one-plane weights), filled by LDS-direct
-// loads in a ring of NS stages, 16-byte chunks XOR-swizzled by the row so that
-// a wave's operand reads hit distinct banks.
+// loads in a ring of NS stages, 16-byte chunks XOR-swizzled so that the 16 lanes
+// of an LDS read cycle (consecutive rows) cover its 64 banks: two 128-byte
+// rows span them, so the swizzle is row / 2 (row / 4 for 64-byte rows). By the
+// row itself every read took twice its cycles (SQ_LDS_BANK_CONFLICT 6.9e7 per
+// dispatch of 32768 x 1280 x 3840-5120, now 0): 1.66e7 -> 1.64e7 cycles, the
+// 128 x 128 tiles 1.28e7 -> 1.26e7; the MFMAs' power sets the time.
 #include "gemm_pair.h"
 
 #include <algorithm>
@@ -248,14 +252,15 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void pair_gemm_kernel(const uint
 #pragma unroll
   for (int q = 0; q < T::LD; ++q) {
     const int g = min(wave * T::LD + q, T::G - 1);
+    const int swz = (g & 1) << 2 | lane >> 4;  // (row / 2) % 8 of row 8 g + lane / 8 (GA is even)
     if (g < T::GA)
-      off[q] = (unsigned)min(g * 8 + (lane >> 3), M - 1 - m0) * (unsigned)(lda * 2) + (((lane & 7) ^ (lane >> 3)) << 4);
+      off[q] = (unsigned)min(g * 8 + (lane >> 3), M - 1 - m0) * (unsigned)(lda * 2) + (((lane & 7) ^ swz) << 4);
     else if (PW == 2)
       off[q] = (unsigned)min((g - T::GA) * 8 + (lane >> 3), N - 1 - n0) * (unsigned)(K * 4) +
-               (((lane & 7) ^ (lane >> 3)) << 4);
+               (((lane & 7) ^ swz) << 4);
     else
       off[q] = (unsigned)min((g - T::GA) * 16 + (lane >> 2), N - 1 - n0) * (unsigned)(K * 2) +
-               (((lane & 3) ^ ((lane >> 3) & 3)) << 4);
+               (((lane & 3) ^ (lane >> 4)) << 4);
   }
   const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
   auto issue = [&](int kt, int st) {
@@ -276,13 +281,13 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void pair_gemm_kernel(const uint
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int s = 0; s < 2; ++s) ard[p][s] = (wm + r31) * 128 + (((p * 4 + s * 2 + h) ^ (lane & 7)) << 4);
+    for (int s = 0; s < 2; ++s) ard[p][s] = (wm + r31) * 128 + (((p * 4 + s * 2 + h) ^ ((lane >> 1) & 7)) << 4);
 #pragma unroll
   for (int p = 0; p < PW; ++p)
 #pragma unroll
     for (int s = 0; s < 2; ++s)
-      wrd[p][s] = T::A_BYTES + (PW == 2 ? (wn + r31) * 128 + (((p * 4 + s * 2 + h) ^ (lane & 7)) << 4)
-                                        : (wn + r31) * 64 + (((s * 2 + h) ^ ((lane >> 1) & 3)) << 4));
+      wrd[p][s] = T::A_BYTES + (PW == 2 ? (wn + r31) * 128 + (((p * 4 + s * 2 + h) ^ ((lane >> 1) & 7)) << 4)
+                                        : (wn + r31) * 64 + (((s * 2 + h) ^ ((lane >> 2) & 3)) << 4));
 
   int arz[2], wrz[PW];  // those of this wave's half (KW = 2)
 #pragma unroll
