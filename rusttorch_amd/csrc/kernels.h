@@ -91,7 +91,9 @@ void launch_copy_out(hipStream_t s, const uint32_t* src, size_t n, const unsigne
 void launch_keys_to_tokens(hipStream_t s, int B, unsigned long long* keys, uint32_t* token);
 void launch_reset_keys(hipStream_t s, int B, unsigned long long* keys);
 
-// GEMM on f32 MFMA, for the models the pair GEMM (gemm_pair.h) does not take: C[M][N] = epi(A[M][K] * W[N][K]^T); C row stride ldc.
+// Prefill GEMM on f32 MFMA (bf16 weights: three bf16 parts of A), for prompts
+// that are drawn from and for the models the pair GEMM (gemm_pair.h) does not
+// take: C[M][N] = epi(A[M][K] * W[N][K]^T); C row stride ldc.
 // ws (ws_floats floats, may be null) holds split-k partial tiles: shapes with
 // too few output tiles to fill the GPU split k when it is large enough
 // (gemm_splitk_ws_floats), otherwise they run unsplit.
@@ -105,13 +107,15 @@ void launch_kv_append(hipStream_t s, const float* qkv, int S, int T, int past, K
 // Prefill c_attn: C = A W^T + bias with the k/v columns ([d, 3d)) of row
 // s*T + t written into the cache at position past + t instead of C (the
 // append of LayerKVCache::append, gpt2.rs:500-514, in the GEMM's epilogue).
-// Falls back to launch_gemm + launch_kv_append where no k split does that.
+// Falls back to launch_gemm + launch_kv_append where the fused kernels do not
+// apply (they need K % 64 == 0, 16-byte aligned operands, head_dim 64 and more
+// than 64 rows, or fewer with a k split; f32 or bf16 weights).
 void launch_gemm_qkv(hipStream_t s, const float* A, int lda, const void* W, int wtype, const float* bias, float* C,
                      long ldc, int M, int K, int S, int T, int past, KvDst kv, float* ws = nullptr,
                      size_t ws_floats = 0);
 // Prefill causal attention for S sequences of T new tokens at offset past, any
-// head_dim (attn_pair.h: head_dim 64 in the models the pair GEMM takes): f32
-// rows to out, or with pair set the pair GEMM's input (f16 pairs, scaled).
+// head_dim: f32 rows to out, or with pair set the pair GEMM's input (f16 pairs,
+// scaled; head_dim 64 takes attn_pair.h there).
 void launch_attn_prefill(hipStream_t s, const float* qkv, int S, int T, int past, const float* kc, const float* vc,
                          int n_head, int n_pos, int d, float* out, uint16_t* pair = nullptr,
                          const float* scale = nullptr);

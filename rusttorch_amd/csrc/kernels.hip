@@ -14,6 +14,7 @@
 
 #include "argmax_key.h"
 #include "attn_core.h"
+#include "bf16_split.h"
 #include "f16_pair.h"
 #include "gelu.h"
 #include "kernels.h"
@@ -769,9 +770,19 @@ __global__ __launch_bounds__(256) void gemm_kernel(const float* __restrict__ A, 
   }
 }
 
-// LDS-direct loads in a ring of GL_NS stages (gemm_skinny_lds_kernel): rows of
-// 16 k (64 bytes), 16-byte chunks XOR-swizzled so that the operand reads hit
-// distinct banks.
+// Prefill GEMM for f32 weights, K % 64 == 0: the same 128x128 tile and MFMA
+// arrangement, fed by LDS-direct loads (global_load_lds_dwordx4) through a
+// GL_NS-stage LDS ring, so no registers hold tiles in flight and three k-tiles
+// are in flight while one is computed.
+// - A stage holds the A and W tiles as 8 + 8 groups of 16 rows x 16 k (1 KiB,
+//   one load instruction each: lane i fills bytes [16i, 16i + 16) of its
+//   group). Lane i loads row r = i / 4 of the group, 4-float chunk
+//   c = (i % 4) ^ gl_swz(row): an XOR swizzle that makes the operand reads
+//   below conflict-free.
+// - k is permuted inside a tile: MFMA step s of lane half h (lane / 32) uses
+//   k = 8h + s, so a lane reads its 8 values of a row with two ds_read_b128.
+//   A and W use the same permutation, so the products are those of the plain
+//   order (the sum is taken over all 16 k of the tile either way).
 constexpr int GL_NS = 4;
 __device__ __forceinline__ int gl_swz(int row) { return (row >> 2) & 3; }
 
@@ -789,6 +800,411 @@ __device__ __forceinline__ void gl_dma16(const float* src, const float* lds_dst)
 template <int N>
 __device__ __forceinline__ void gl_wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// One k-tile step of gemm_lds_kernel on stage ST. Each stage is its own LDS
+// array and the loop is unrolled over the four stages, so every LDS address
+// is a base plus an immediate offset (about 1% faster than one array indexed
+// by kt % 4).
+template <int ST>
+__device__ __forceinline__ void gl_step(int kt, int nk, float (&lds)[2][GBM * 16], float (&nxt)[2][GBM * 16],
+                                        const float* const (&asrc)[2], const float* const (&wsrc)[2], int wave,
+                                        const int (&aoff)[2][2], const int (&woff)[2][2], floatx16 (&acc)[2][2]) {
+  // tile kt has landed once at most the loads of the GL_NS - 2 later tiles
+  // (4 instructions each) are still outstanding; after the barrier every
+  // wave's loads of tile kt are in and no wave reads tile kt - 1 any more
+  if (kt + GL_NS - 2 < nk) gl_wait_barrier<(GL_NS - 2) * 4>();
+  else gl_wait_barrier<0>();
+  if (kt + GL_NS - 1 < nk) {
+    const int k = (kt + GL_NS - 1) * 16;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int g = 2 * wave + q;
+      gl_dma16(asrc[q] + k, &nxt[0][g * 256]);
+      gl_dma16(wsrc[q] + k, &nxt[1][g * 256]);
+    }
+  }
+  float4 a[2][2], b[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      a[i][c] = *reinterpret_cast<const float4*>(&lds[0][aoff[i][c]]);
+      b[i][c] = *reinterpret_cast<const float4*>(&lds[1][woff[i][c]]);
+    }
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float4& av = a[i][s >> 2];
+        const float4& bv = b[j][s >> 2];
+        const int e = s & 3;
+        const float x = e == 0 ? av.x : e == 1 ? av.y : e == 2 ? av.z : av.w;
+        const float y = e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[i][j], 0, 0, 0);
+      }
+  }
+}
+
+// Epilogue of the 128x128 tile kernels: wave tile (wm, wn) of block (m0, n0)
+// in acc[i][j] (32x32 blocks, MFMA output layout), to ws[z] as a raw partial
+// tile when ws is set, else with the epilogue (bias, gelu, residual; with kv
+// set, c_attn's k / v columns go into the cache at (sequence, head, past + t)).
+template <int I = 2, int J = 2>
+__device__ __forceinline__ void gl_epilogue(const floatx16 (&acc)[I][J], int lane, int m0, int n0, int wm, int wn,
+                                            int z, const float* __restrict__ bias, float* __restrict__ C, long ldc,
+                                            int M, int N, int epi, const KvDst& kv, int kv_T, int kv_past,
+                                            float* __restrict__ ws) {
+  if (ws != nullptr) {
+    float* wz = ws + (size_t)z * M * N;
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        const int n = n0 + wn + j * 32 + (lane & 31);
+        if (n >= N) continue;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int m = m0 + wm + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          if (m < M) wz[(size_t)m * N + n] = acc[i][j][e];
+        }
+      }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < I; ++i) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int n = n0 + wn + j * 32 + (lane & 31);
+      if (n >= N) continue;
+      const float bv = bias ? bias[n] : 0.f;
+      if (kv.k != nullptr && n >= kv.d) {
+        // k / v column of c_attn: into the cache at (sequence, head, past + t)
+        const int which = n >= 2 * kv.d, cc = n - kv.d - which * kv.d;
+        float* base = (which ? kv.v : kv.k) + (size_t)(cc >> 6) * kv.n_pos * 64 + (cc & 63);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int m = m0 + wm + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          if (m < M) {
+            const int sq = m / kv_T, t = m - sq * kv_T;
+            base[((size_t)sq * kv.n_head * kv.n_pos + kv_past + t) * 64] = acc[i][j][e] + bv;
+          }
+        }
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = m0 + wm + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+        if (m < M) {
+          float* cp = C + (size_t)m * ldc + n;
+          const float v = acc[i][j][e];
+          if (epi == EPI_BIAS) *cp = v + bv;
+          else if (epi == EPI_BIAS_GELU) *cp = gelu_new(v + bv);
+          else if (epi == EPI_BIAS_RESID) *cp = *cp + (v + bv);
+          else *cp = v;
+        }
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void gemm_lds_kernel(const float* __restrict__ A, int lda,
+                                                       const float* __restrict__ W, const float* __restrict__ bias,
+                                                       float* __restrict__ C, long ldc, int M, int N, int K, int epi,
+                                                       int m_fast, KvDst kv, int kv_T, int kv_past, int ks,
+                                                       float* __restrict__ ws) {
+  __shared__ __attribute__((aligned(16))) float st0[2][GBM * 16];
+  __shared__ __attribute__((aligned(16))) float st1[2][GBM * 16];
+  __shared__ __attribute__((aligned(16))) float st2[2][GBM * 16];
+  __shared__ __attribute__((aligned(16))) float st3[2][GBM * 16];
+  static_assert(GL_NS == 4, "four stage arrays");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+  // block order: with m_fast the row blocks of one W column block are
+  // consecutive (W read once while A cycles through the cache), else the
+  // column blocks of one A row block (A read once while W cycles)
+  // with ks > 1 the k range is split: block b handles tile b % (nmb * nnb)
+  // over k-split z = b / (nmb * nnb) and stores its raw partial tile to
+  // ws[z] (summed and finished by splitk_reduce_kernel)
+  const int nmb = (M + GBM - 1) / GBM, nnb = (N + GBN - 1) / GBN;
+  const int bid = blockIdx.x % (nmb * nnb), z = blockIdx.x / (nmb * nnb);
+  const int m0 = (m_fast ? bid % nmb : bid / nnb) * GBM, n0 = (m_fast ? bid / nmb : bid % nnb) * GBN;
+  const int nk = K / 16 / ks;  // k-tiles of this split, a multiple of GL_NS
+
+  // this lane's load sources: groups 2*wave and 2*wave + 1 of A and of W
+  const int lr = lane >> 2;
+  const float* asrc[2];
+  const float* wsrc[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int row = (2 * wave + q) * 16 + lr;
+    const int c = (lane & 3) ^ gl_swz(row);
+    asrc[q] = A + (size_t)min(m0 + row, M - 1) * lda + c * 4 + (size_t)z * nk * 16;
+    wsrc[q] = W + (size_t)min(n0 + row, N - 1) * K + c * 4 + (size_t)z * nk * 16;
+  }
+  auto issue = [&](int kt, float (&st)[2][GBM * 16]) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int g = 2 * wave + q;
+      gl_dma16(asrc[q] + kt * 16, &st[0][g * 256]);
+      gl_dma16(wsrc[q] + kt * 16, &st[1][g * 256]);
+    }
+  };
+
+  // operand read offsets (floats within a stage's A or W tile): rows
+  // wm + 32i + lane % 32 (A) and wn + 32j + lane % 32 (W), chunks 2h, 2h + 1
+  const int h = lane >> 5;
+  int aoff[2][2], woff[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int ra = wm + 32 * i + (lane & 31), rw = wn + 32 * i + (lane & 31);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      aoff[i][c] = ra * 16 + (((2 * h + c) ^ gl_swz(ra)) * 4);
+      woff[i][c] = rw * 16 + (((2 * h + c) ^ gl_swz(rw)) * 4);
+    }
+  }
+
+  floatx16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  issue(0, st0);
+  issue(1, st1);
+  issue(2, st2);
+  for (int kt = 0; kt < nk; kt += GL_NS) {
+    gl_step<0>(kt, nk, st0, st3, asrc, wsrc, wave, aoff, woff, acc);
+    gl_step<1>(kt + 1, nk, st1, st0, asrc, wsrc, wave, aoff, woff, acc);
+    gl_step<2>(kt + 2, nk, st2, st1, asrc, wsrc, wave, aoff, woff, acc);
+    gl_step<3>(kt + 3, nk, st3, st2, asrc, wsrc, wave, aoff, woff, acc);
+  }
+
+  gl_epilogue(acc, lane, m0, n0, wm, wn, z, bias, C, ldc, M, N, epi, kv, kv_T, kv_past, ws);
+}
+
+// gemm_lds_kernel with 64 x 128 workgroup tiles (each wave 32 x 64, one A
+// group of 16 rows and two W groups per stage), for f32 GEMMs of at most 1024
+// rows: twice the workgroups of the 128 x 128 tiles, so fewer k splits and
+// reductions (c3's 512-row and c2's 1024-row prefill GEMMs: 5-25% faster
+// each, the split-k reduction included).
+constexpr int G64M = 64;
+template <int ST>
+__device__ __forceinline__ void g64_step(int kt, int nk, float (&la)[G64M * 16], float (&lw)[GBN * 16],
+                                         float (&na)[G64M * 16], float (&nw)[GBN * 16], const float* asrc,
+                                         const float* const (&wsrc)[2], int wave, const int (&aoff)[2],
+                                         const int (&woff)[2][2], floatx16 (&acc)[1][2]) {
+  if (kt + GL_NS - 2 < nk) gl_wait_barrier<(GL_NS - 2) * 3>();
+  else gl_wait_barrier<0>();
+  if (kt + GL_NS - 1 < nk) {
+    const int k = (kt + GL_NS - 1) * 16;
+    gl_dma16(asrc + k, &na[wave * 256]);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) gl_dma16(wsrc[q] + k, &nw[(2 * wave + q) * 256]);
+  }
+  float4 a[2], b[2][2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    a[c] = *reinterpret_cast<const float4*>(&la[aoff[c]]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) b[j][c] = *reinterpret_cast<const float4*>(&lw[woff[j][c]]);
+  }
+#pragma unroll
+  for (int st = 0; st < 8; ++st) {
+    const float4& av = a[st >> 2];
+    const int e = st & 3;
+    const float x = e == 0 ? av.x : e == 1 ? av.y : e == 2 ? av.z : av.w;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float4& bv = b[j][st >> 2];
+      const float y = e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w;
+      acc[0][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[0][j], 0, 0, 0);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void gemm_lds64_kernel(const float* __restrict__ A, int lda,
+                                                         const float* __restrict__ W, const float* __restrict__ bias,
+                                                         float* __restrict__ C, long ldc, int M, int N, int K, int epi,
+                                                         int m_fast, KvDst kv, int kv_T, int kv_past, int ks,
+                                                         float* __restrict__ ws) {
+  __shared__ __attribute__((aligned(16))) float a0[G64M * 16], a1[G64M * 16], a2[G64M * 16], a3[G64M * 16];
+  __shared__ __attribute__((aligned(16))) float w0[GBN * 16], w1[GBN * 16], w2[GBN * 16], w3[GBN * 16];
+  static_assert(GL_NS == 4, "four stage arrays");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
+  const int nmb = (M + G64M - 1) / G64M, nnb = (N + GBN - 1) / GBN;
+  const int bid = blockIdx.x % (nmb * nnb), z = blockIdx.x / (nmb * nnb);
+  const int m0 = (m_fast ? bid % nmb : bid / nnb) * G64M, n0 = (m_fast ? bid / nmb : bid % nnb) * GBN;
+  const int nk = K / 16 / ks;
+  const int lr = lane >> 2;
+  const float* asrc;
+  {
+    const int row = wave * 16 + lr;
+    const int c = (lane & 3) ^ gl_swz(row);
+    asrc = A + (size_t)min(m0 + row, M - 1) * lda + c * 4 + (size_t)z * nk * 16;
+  }
+  const float* wsrc[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int row = (2 * wave + q) * 16 + lr;
+    const int c = (lane & 3) ^ gl_swz(row);
+    wsrc[q] = W + (size_t)min(n0 + row, N - 1) * K + c * 4 + (size_t)z * nk * 16;
+  }
+  auto issue = [&](int kt, float (&la)[G64M * 16], float (&lw)[GBN * 16]) {
+    gl_dma16(asrc + kt * 16, &la[wave * 256]);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) gl_dma16(wsrc[q] + kt * 16, &lw[(2 * wave + q) * 256]);
+  };
+  const int h = lane >> 5;
+  int aoff[2], woff[2][2];
+  {
+    const int ra = wm + (lane & 31);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) aoff[c] = ra * 16 + (((2 * h + c) ^ gl_swz(ra)) * 4);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int rw = wn + 32 * j + (lane & 31);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) woff[j][c] = rw * 16 + (((2 * h + c) ^ gl_swz(rw)) * 4);
+    }
+  }
+  floatx16 acc[1][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[0][j][e] = 0.f;
+  issue(0, a0, w0);
+  issue(1, a1, w1);
+  issue(2, a2, w2);
+  for (int kt = 0; kt < nk; kt += GL_NS) {
+    g64_step<0>(kt, nk, a0, w0, a3, w3, asrc, wsrc, wave, aoff, woff, acc);
+    g64_step<1>(kt + 1, nk, a1, w1, a0, w0, asrc, wsrc, wave, aoff, woff, acc);
+    g64_step<2>(kt + 2, nk, a2, w2, a1, w1, asrc, wsrc, wave, aoff, woff, acc);
+    g64_step<3>(kt + 3, nk, a3, w3, a2, w2, asrc, wsrc, wave, aoff, woff, acc);
+  }
+  gl_epilogue<1, 2>(acc, lane, m0, n0, wm, wn, z, bias, C, ldc, M, N, epi, kv, kv_T, kv_past, ws);
+}
+
+// gemm_lds_kernel for bf16 weights (the f32 activations times W stored as
+// bf16, gpt2.rs Conv1D with bf16-rounded weights upcast in the product): the
+// same 128x128 tiles, k-tiles of 16 and LDS-direct stage ring, with W's tile
+// as 128 rows of 32 bytes (one load instruction per wave: lane i fills row
+// 32 * wave + i / 2, 16-byte chunk (i % 2) ^ ((row >> 3) & 1)). Each lane's 8
+// A values of a 32-row block enter v_mfma_f32_32x32x16_bf16 as three exact
+// bf16 parts (split3), so every product is exact in f32 and the MFMA
+// accumulates in f32: the f32 GEMM up to summation order, at the bf16 rate.
+// Lane l holds A[row l % 32][k 8 (l / 32) .. + 8) and W[col l % 32][the same
+// k] of a tile, the A reads of gemm_lds_kernel.
+template <int ST>
+__device__ __forceinline__ void glb_step(int kt, int nk, float (&la)[GBM * 16], float (&lw)[GBM * 8],
+                                         float (&na)[GBM * 16], float (&nw)[GBM * 8], const float* const (&asrc)[2],
+                                         const uint16_t* wsrc, int wave, const int (&aoff)[2][2], const int (&woff)[2],
+                                         floatx16 (&acc)[2][2]) {
+  // tile kt has landed once at most the loads of the GL_NS - 2 later tiles
+  // (3 instructions each) are outstanding
+  if (kt + GL_NS - 2 < nk) gl_wait_barrier<(GL_NS - 2) * 3>();
+  else gl_wait_barrier<0>();
+  if (kt + GL_NS - 1 < nk) {
+    const int k = (kt + GL_NS - 1) * 16;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) gl_dma16(asrc[q] + k, &na[(2 * wave + q) * 256]);
+    gl_dma16(reinterpret_cast<const float*>(wsrc + k), &nw[wave * 256]);
+  }
+  u4v b[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const u4v*>(&lw[woff[j]]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float4 a0 = *reinterpret_cast<const float4*>(&la[aoff[i][0]]);
+    const float4 a1 = *reinterpret_cast<const float4*>(&la[aoff[i][1]]);
+    const float xs[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+    u4v xh, xm, xl;
+    split3(xs, xh, xm, xl);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const bf16x8 wb = as_bf16x8(b[j]);
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xh), wb, acc[i][j], 0, 0, 0);
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xm), wb, acc[i][j], 0, 0, 0);
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xl), wb, acc[i][j], 0, 0, 0);
+    }
+  }
+}
+
+__device__ __forceinline__ int glb_swz(int row) { return (row >> 3) & 1; }
+
+__global__ __launch_bounds__(256) void gemm_lds_bf16_kernel(const float* __restrict__ A, int lda,
+                                                            const uint16_t* __restrict__ W,
+                                                            const float* __restrict__ bias, float* __restrict__ C,
+                                                            long ldc, int M, int N, int K, int epi, int m_fast,
+                                                            KvDst kv, int kv_T, int kv_past, int ks,
+                                                            float* __restrict__ ws) {
+  __shared__ __attribute__((aligned(16))) float a0[GBM * 16], a1[GBM * 16], a2[GBM * 16], a3[GBM * 16];
+  __shared__ __attribute__((aligned(16))) float w0[GBM * 8], w1[GBM * 8], w2[GBM * 8], w3[GBM * 8];
+  static_assert(GL_NS == 4, "four stage arrays");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+  const int nmb = (M + GBM - 1) / GBM, nnb = (N + GBN - 1) / GBN;
+  const int bid = blockIdx.x % (nmb * nnb), z = blockIdx.x / (nmb * nnb);
+  const int m0 = (m_fast ? bid % nmb : bid / nnb) * GBM, n0 = (m_fast ? bid / nmb : bid % nnb) * GBN;
+  const int nk = K / 16 / ks;  // k-tiles of this split, a multiple of GL_NS
+
+  // load sources: A groups 2*wave and 2*wave + 1 (as gemm_lds_kernel), W rows
+  // 32*wave + lane / 2
+  const int lr = lane >> 2;
+  const float* asrc[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int row = (2 * wave + q) * 16 + lr;
+    const int c = (lane & 3) ^ gl_swz(row);
+    asrc[q] = A + (size_t)min(m0 + row, M - 1) * lda + c * 4 + (size_t)z * nk * 16;
+  }
+  const uint16_t* wsrc;
+  {
+    const int row = 32 * wave + (lane >> 1);
+    const int c = (lane & 1) ^ glb_swz(row);
+    wsrc = W + (size_t)min(n0 + row, N - 1) * K + c * 8 + (size_t)z * nk * 16;
+  }
+  auto issue = [&](int kt, float (&la)[GBM * 16], float (&lw)[GBM * 8]) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) gl_dma16(asrc[q] + kt * 16, &la[(2 * wave + q) * 256]);
+    gl_dma16(reinterpret_cast<const float*>(wsrc + kt * 16), &lw[wave * 256]);
+  };
+  // operand reads: A rows wm + 32i + lane % 32, chunks 2h and 2h + 1 (floats);
+  // W rows wn + 32j + lane % 32, chunk h (8 bf16 = 4 floats' bytes)
+  const int h = lane >> 5;
+  int aoff[2][2], woff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int ra = wm + 32 * i + (lane & 31), rw = wn + 32 * i + (lane & 31);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) aoff[i][c] = ra * 16 + (((2 * h + c) ^ gl_swz(ra)) * 4);
+    woff[i] = rw * 8 + ((h ^ glb_swz(rw)) * 4);
+  }
+
+  floatx16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  issue(0, a0, w0);
+  issue(1, a1, w1);
+  issue(2, a2, w2);
+  for (int kt = 0; kt < nk; kt += GL_NS) {
+    glb_step<0>(kt, nk, a0, w0, a3, w3, asrc, wsrc, wave, aoff, woff, acc);
+    glb_step<1>(kt + 1, nk, a1, w1, a0, w0, asrc, wsrc, wave, aoff, woff, acc);
+    glb_step<2>(kt + 2, nk, a2, w2, a1, w1, asrc, wsrc, wave, aoff, woff, acc);
+    glb_step<3>(kt + 3, nk, a3, w3, a2, w2, asrc, wsrc, wave, aoff, woff, acc);
+  }
+  gl_epilogue(acc, lane, m0, n0, wm, wn, z, bias, C, ldc, M, N, epi, kv, kv_T, kv_past, ws);
 }
 
 // Skinny GEMM for few rows (a short prompt): the 128x128 tile kernel would
@@ -981,7 +1397,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny16_kernel(const float* __r
   }
 }
 
-// GEMM for 17..32 rows with f32 weights, K % 64 == 0, on an
+// Prompt GEMM for 17..32 rows with f32 weights, K % 64 == 0: gemm_lds_kernel's
 // LDS-direct ring (4 stages, XOR-swizzled 16-byte chunks, k permuted inside a
 // tile) with a 32 x 128 tile: the 32 rows of A and 128 rows of W (output
 // columns) per 16-k stage, wave w computing columns [32w, 32w + 32) with one
@@ -1194,8 +1610,8 @@ static bool launch_skinny(hipStream_t s, const float* A, int lda, const void* W,
   return true;
 }
 
-// Sum of the ks split-k partial tiles of a GEMM (ws[z][m][n], in z order) and
-// the epilogue the kernel applies without a split (bias, gelu,
+// Sum of the ks split-k partial tiles of gemm_lds_kernel (ws[z][m][n], in z
+// order) and the epilogue that kernel applies without a split (bias, gelu,
 // residual; with kv set, the k / v columns of c_attn go into the cache).
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ ws, int ks, int M, int N,
                                                             const float* __restrict__ bias, float* __restrict__ C,
@@ -1238,18 +1654,37 @@ static void splitk_reduce(hipStream_t s, const float* ws, int ks, int M, int N, 
                                                                       kv_past);
 }
 
-// k-splits of gemm_kernel for an M x N x K GEMM: 1 when the output tiles
+// k-splits of gemm_lds_kernel for an M x N x K GEMM: 1 when the output tiles
 // alone give enough workgroups (>= 192) or M < 128, else the smallest split
-// that gives >= 240 workgroups, or the largest valid one up to 16.
-static int gemm_splitk_factor(int M, int N, int K) {
+// that gives >= 240 workgroups (each split a multiple of 4 k-tiles), or the
+// largest valid one up to 16. (Prefills of a few hundred rows otherwise run
+// their d-wide GEMMs on 32-48 of the 256 CUs.)
+// granule: k-tiles of 16 a split must hold a multiple of (GL_NS for
+// gemm_lds_kernel's stage ring, 1 for gemm_kernel).
+int gemm_splitk_factor(int M, int N, int K, int granule) {
   const int tiles = ((M + GBM - 1) / GBM) * ((N + GBN - 1) / GBN);
-  if (M < 128 || tiles >= 192 || K % 16 != 0) return 1;
+  if (M < 128 || tiles >= 192 || K % (16 * granule) != 0) return 1;
   const int nk = K / 16;
   int best = 1;
   for (int s = 2; s <= 16; ++s) {
-    if (nk % s != 0) continue;
+    if (nk % (granule * s) != 0) continue;
     best = s;
     if (tiles * s >= 240) break;
+  }
+  return best;
+}
+
+// k-splits of gemm_lds64_kernel (M <= 1024): as gemm_splitk_factor, over its
+// 64 x 128 output tiles (and, as there, none below 128 rows).
+static int gemm64_splitk_factor(int M, int N, int K) {
+  const int tiles = ((N + GBN - 1) / GBN) * ((M + G64M - 1) / G64M);
+  if (M < 128 || M > 1024 || tiles >= 192 || K % (16 * GL_NS) != 0) return 1;
+  const int nkt = K / 16;
+  int best = 1;
+  for (int sp = 2; sp <= 16; ++sp) {
+    if (nkt % (GL_NS * sp) != 0) continue;
+    best = sp;
+    if (tiles * sp >= 240) break;
   }
   return best;
 }
@@ -1257,26 +1692,74 @@ static int gemm_splitk_factor(int M, int N, int K) {
 size_t gemm_splitk_ws_floats(int M, int N, int K) {
   // the largest of the kernels' needs (which one runs depends on the weight
   // type, the row count and alignment)
-  const int ks = std::max(gemm_splitk_factor(M, N, K),
-                          std::max(skinny_splitk_factor(M, N, K), skinny_lds_splitk_factor(M, N, K)));
+  const int ks = std::max(std::max(std::max(gemm_splitk_factor(M, N, K, GL_NS), gemm_splitk_factor(M, N, K, 1)),
+                                   std::max(skinny_splitk_factor(M, N, K), skinny_lds_splitk_factor(M, N, K))),
+                          gemm64_splitk_factor(M, N, K));
   return ks > 1 ? (size_t)ks * M * N : 0;
+}
+
+static bool gemm_lds_ok(const float* A, int lda, const void* W, int wtype, int K) {
+  return K % 64 == 0 && lda % 4 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
+         (reinterpret_cast<uintptr_t>(W) & 15) == 0;
+}
+
+// gemm_lds_kernel (f32 W) or gemm_lds_bf16_kernel (bf16 W), split over k
+// when that fills the GPU and ws holds the partial tiles (ws_floats of them),
+// then the split-k reduction.
+static void launch_gemm_lds(hipStream_t s, const float* A, int lda, const void* W, int wtype, const float* bias,
+                            float* C, long ldc, int M, int N, int K, int epi, KvDst kv, int kv_T, int kv_past,
+                            float* ws, size_t ws_floats) {
+  const int nb = ((N + GBN - 1) / GBN) * ((M + GBM - 1) / GBM);
+  int ks = gemm_splitk_factor(M, N, K, GL_NS);
+  if (ks > 1 && (ws == nullptr || (size_t)ks * M * N > ws_floats)) ks = 1;
+  if (wtype == W_F32 && M <= 1024) {
+    // 64 x 128 tiles (gemm_lds64_kernel)
+    const int nb64 = ((N + GBN - 1) / GBN) * ((M + G64M - 1) / G64M);
+    int ks64 = gemm64_splitk_factor(M, N, K);
+    if (ks64 > 1 && (ws == nullptr || (size_t)ks64 * M * N > ws_floats)) ks64 = 1;
+    gemm_lds64_kernel<<<nb64 * ks64, 256, 0, s>>>(A, lda, static_cast<const float*>(W), bias, C, ldc, M, N, K, epi,
+                                                  N > M ? 1 : 0, kv, kv_T, kv_past, ks64, ks64 > 1 ? ws : nullptr);
+    if (ks64 > 1) splitk_reduce(s, ws, ks64, M, N, bias, C, ldc, epi, kv, kv_T, kv_past);
+    return;
+  }
+  float* wsk = ks > 1 ? ws : nullptr;
+  if (wtype == W_F32)
+    gemm_lds_kernel<<<nb * ks, 256, 0, s>>>(A, lda, static_cast<const float*>(W), bias, C, ldc, M, N, K, epi,
+                                            N > M ? 1 : 0, kv, kv_T, kv_past, ks, wsk);
+  else
+    gemm_lds_bf16_kernel<<<nb * ks, 256, 0, s>>>(A, lda, static_cast<const uint16_t*>(W), bias, C, ldc, M, N, K,
+                                                 epi, N > M ? 1 : 0, kv, kv_T, kv_past, ks, wsk);
+  if (ks > 1) splitk_reduce(s, ws, ks, M, N, bias, C, ldc, epi, kv, kv_T, kv_past);
 }
 
 void launch_gemm(hipStream_t s, const float* A, int lda, const void* W, int wtype, const float* bias, float* C,
                  long ldc, int M, int N, int K, int epi, float* ws, size_t ws_floats) {
   if (launch_skinny(s, A, lda, W, wtype, bias, C, ldc, M, N, K, epi, SkinnyQkv{}, ws, ws_floats)) return;
-  int ks = gemm_splitk_factor(M, N, K);
-  if (ks > 1 && (ws == nullptr || (size_t)ks * M * N > ws_floats)) ks = 1;
-  const dim3 grid((N + GBN - 1) / GBN, (M + GBM - 1) / GBM, ks);
-  float* wsk = ks > 1 ? ws : nullptr;
-  if (wtype == W_F32) gemm_kernel<W_F32><<<grid, 256, 0, s>>>(A, lda, W, bias, C, ldc, M, N, K, epi, ks, wsk);
-  else gemm_kernel<W_BF16><<<grid, 256, 0, s>>>(A, lda, W, bias, C, ldc, M, N, K, epi, ks, wsk);
-  if (ks > 1) splitk_reduce(s, ws, ks, M, N, bias, C, ldc, epi, KvDst{}, 1, 0);
+  dim3 grid((N + GBN - 1) / GBN, (M + GBM - 1) / GBM);
+  if (gemm_lds_ok(A, lda, W, wtype, K))
+    // (256 x 128 tiles with 3 stages, bounded to two waves per SIMD, were 2-4%
+    // faster on the c4 shapes without an epilogue but made the c4 prefill
+    // slower, 70.7k against 72.5k tokens/s; 3 stages at three waves per SIMD
+    // and 2 stages at four were no faster than this kernel)
+    launch_gemm_lds(s, A, lda, W, wtype, bias, C, ldc, M, N, K, epi, KvDst{}, 1, 0, ws, ws_floats);
+  else {
+    int ks = gemm_splitk_factor(M, N, K, 1);
+    if (ks > 1 && (ws == nullptr || (size_t)ks * M * N > ws_floats)) ks = 1;
+    grid.z = ks;
+    float* wsk = ks > 1 ? ws : nullptr;
+    if (wtype == W_F32) gemm_kernel<W_F32><<<grid, 256, 0, s>>>(A, lda, W, bias, C, ldc, M, N, K, epi, ks, wsk);
+    else gemm_kernel<W_BF16><<<grid, 256, 0, s>>>(A, lda, W, bias, C, ldc, M, N, K, epi, ks, wsk);
+    if (ks > 1) splitk_reduce(s, ws, ks, M, N, bias, C, ldc, epi, KvDst{}, 1, 0);
+  }
 }
 
 void launch_gemm_qkv(hipStream_t s, const float* A, int lda, const void* W, int wtype, const float* bias, float* C,
                      long ldc, int M, int K, int S, int T, int past, KvDst kv, float* ws, size_t ws_floats) {
   const int N = 3 * kv.d;
+  if (M > 64 && gemm_lds_ok(A, lda, W, wtype, K) && kv.d == 64 * kv.n_head) {
+    launch_gemm_lds(s, A, lda, W, wtype, bias, C, ldc, M, N, K, EPI_BIAS, kv, T, past, ws, ws_floats);
+    return;
+  }
   // a prompt of at most 64 rows: the split skinny GEMM's reduction writes the
   // k / v columns into the cache itself (head_dim 64)
   if (kv.d == 64 * kv.n_head &&
@@ -1407,11 +1890,367 @@ __global__ __launch_bounds__(64) void attn_prefill_kernel(const float* __restric
   }
 }
 
+// ---------------------------------------------------------------------------
+// Prefill causal attention for head_dim 64 on fp32 MFMA (flash-attention
+// form of multi_head_attention_cached, gpt2.rs:772-834). A workgroup of FW
+// waves takes 32 * FW queries of one (sequence, head); each wave owns 32. Key
+// blocks of 32 rows are staged in LDS (K row-major, V transposed), the next
+// block's rows are loaded into registers while the current one is used.
+//
+// Per key block a wave computes S^T = K Q^T (32 keys x 32 queries, 32
+// v_mfma_f32_32x32x2f32 steps over the 64 dims: step kk pairs dims kk and
+// kk + 32), so accumulator i of lane l holds the score of query l % 32 with
+// key r(i, l) = (i/4)*8 + (l/32)*4 + i%4. The softmax statistics of a query
+// are therefore lane-local (16 values) plus one exchange between the two
+// lane halves, and the rescale of the output is lane-local.
+// O^T += V^T P^T runs 16 steps per 32-dim output tile; step kk takes key
+// r(kk, l) in lane half l/32, which is exactly accumulator kk of the lane,
+// so P feeds the MFMA from registers. Online softmax with running max m and
+// per-half partial sums l (combined at the end), as the scalar kernel.
+// ---------------------------------------------------------------------------
+
+constexpr int FA_QW = 32;         // queries per wave
+constexpr int FA_K = 32;          // keys per block
+constexpr int FA_KP = 64 + 4;     // padded K row (floats)
+constexpr int FA_VP = FA_K + 4;   // padded V^T row (floats)
+
+template <int FW>
+__global__ __launch_bounds__(64 * FW) void attn_prefill_mfma_kernel(
+    const float* __restrict__ qkv, int T, int past, const float* __restrict__ kc, const float* __restrict__ vc,
+    int H, int P, int d, int nqb, float* __restrict__ out) {
+  constexpr int NT = 64 * FW, U = 512 / NT;  // threads; float4 of K (and of V) a thread stages per block
+  __shared__ __attribute__((aligned(16))) float Ks[FA_K][FA_KP];
+  __shared__ __attribute__((aligned(16))) float Vt[64][FA_VP];
+  // the query block is the slowest grid dimension, longest (last) blocks
+  // first: every (sequence, head)'s longest block is dispatched before any
+  // shorter one, which keeps the tail of the grid short
+  const int qb = nqb - 1 - (int)blockIdx.z;
+  const int h = blockIdx.x, sidx = blockIdx.y;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int c = lane & 31, hh = lane >> 5;
+  const int qi = qb * FA_QW * FW + wave * FA_QW + c;  // this lane's query (0..T-1 when valid)
+  const bool qvalid = qi < T;
+  const int qpos = past + qi;
+  const size_t head_off = ((size_t)sidx * H + h) * (size_t)P * 64;
+  const float* Kh = kc + head_off;
+  const float* Vh = vc + head_off;
+  // this lane's half of its query row: dims [32*hh, 32*hh + 32)
+  float q[32];
+  {
+    const float* qrow = qkv + ((size_t)sidx * T + min(qi, T - 1)) * 3 * d + h * 64 + 32 * hh;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float4 v = reinterpret_cast<const float4*>(qrow)[j];
+      q[4 * j] = v.x;
+      q[4 * j + 1] = v.y;
+      q[4 * j + 2] = v.z;
+      q[4 * j + 3] = v.w;
+    }
+  }
+  const int kmax = past + min(T, (qb + 1) * FA_QW * FW) - 1;  // last key any query here attends
+  const int nkb = kmax / FA_K + 1;
+  // staging: 512 float4 of K and of V per block, U each per thread
+  float4 kr[U], vr[U];
+  auto load_block = [&](int kb) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = tid + u * NT;
+      const int r = e >> 4, c4 = (e & 15) * 4, j = kb * FA_K + r;
+      const bool ok = j <= kmax;
+      kr[u] = ok ? *reinterpret_cast<const float4*>(Kh + (size_t)j * 64 + c4) : make_float4(0.f, 0.f, 0.f, 0.f);
+      vr[u] = ok ? *reinterpret_cast<const float4*>(Vh + (size_t)j * 64 + c4) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  float m = -INFINITY, l = 0.f;
+  floatx16 o0, o1;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    o0[i] = 0.f;
+    o1[i] = 0.f;
+  }
+  load_block(0);
+  for (int kb = 0; kb < nkb; ++kb) {
+    __syncthreads();  // every wave is done with the previous block
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = tid + u * NT;
+      const int r = e >> 4, c4 = (e & 15) * 4;
+      *reinterpret_cast<float4*>(&Ks[r][c4]) = kr[u];
+      Vt[c4][r] = vr[u].x;
+      Vt[c4 + 1][r] = vr[u].y;
+      Vt[c4 + 2][r] = vr[u].z;
+      Vt[c4 + 3][r] = vr[u].w;
+    }
+    __syncthreads();
+    if (kb + 1 < nkb) load_block(kb + 1);
+    // S^T = K Q^T
+    floatx16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float4 a = *reinterpret_cast<const float4*>(&Ks[c][32 * hh + 4 * j]);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, q[4 * j], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, q[4 * j + 1], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, q[4 * j + 2], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, q[4 * j + 3], s, 0, 0, 0);
+    }
+    // causal mask (key j <= query position), scale 1/sqrt(64), online softmax
+    const int j0 = kb * FA_K;
+    float bm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int j = j0 + (i / 4) * 8 + hh * 4 + (i % 4);
+      s[i] = j <= qpos ? s[i] * 0.125f : -INFINITY;
+      bm = fmaxf(bm, s[i]);
+    }
+    bm = xor32_max_k(bm);
+    const float mn = fmaxf(m, bm);
+    const float corr = m == -INFINITY ? 0.f : fexp_a(m - mn);
+    float ps = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = s[i] == -INFINITY ? 0.f : fexp_a(s[i] - mn);
+      ps += s[i];
+    }
+    l = l * corr + ps;
+    m = mn;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      o0[i] *= corr;
+      o1[i] *= corr;
+    }
+    // O^T += V^T P^T
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 v0 = *reinterpret_cast<const float4*>(&Vt[c][8 * g + 4 * hh]);
+      const float4 v1 = *reinterpret_cast<const float4*>(&Vt[32 + c][8 * g + 4 * hh]);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v0.x, s[4 * g], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1.x, s[4 * g], o1, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v0.y, s[4 * g + 1], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1.y, s[4 * g + 1], o1, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v0.z, s[4 * g + 2], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1.z, s[4 * g + 2], o1, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v0.w, s[4 * g + 3], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1.w, s[4 * g + 3], o1, 0, 0, 0);
+    }
+  }
+  l = xor32_sum_k(l);
+  if (qvalid) {
+    const float inv = 1.0f / l;
+    float* orow = out + ((size_t)sidx * T + qi) * d + h * 64;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = (i / 4) * 8 + hh * 4 + (i % 4);
+      orow[r] = o0[i] * inv;
+      orow[32 + r] = o1[i] * inv;
+    }
+  }
+}
+
+// attn_prefill_mfma_kernel with the key range split over the waves: a
+// workgroup of KS waves takes 32 queries of one (sequence, head) and wave w
+// the key blocks w, w + KS, ... (each staged in the wave's own LDS region, so
+// no workgroup barrier per block); the waves' (m, l, O) merge in LDS at the
+// end (out = sum_w O_w e^(m_w - M) / sum_w l_w e^(m_w - M)). For a few long
+// prompts the causal chain of the last query block (T / 32 key blocks, one
+// after the other on one wave) is otherwise the whole kernel.
+template <int KS>
+__global__ __launch_bounds__(64 * KS) void attn_prefill_ks_kernel(const float* __restrict__ qkv, int T, int past,
+                                                                  const float* __restrict__ kc,
+                                                                  const float* __restrict__ vc, int H, int P, int d,
+                                                                  int nqb, float* __restrict__ out) {
+  constexpr int REG = FA_K * FA_KP + 64 * FA_VP;  // floats of one wave's K block and V^T block
+  constexpr int MW = 64 + 2;                      // merge record of one query: m, l, O[64]
+  static_assert(FA_QW * MW <= REG, "merge records fit the staging region");
+  __shared__ __attribute__((aligned(16))) float sm[KS][REG];
+  const int qb = nqb - 1 - (int)blockIdx.z;  // longest query blocks first
+  const int h = blockIdx.x, sidx = blockIdx.y;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int c = lane & 31, hh = lane >> 5;
+  const int qi = qb * FA_QW + c;
+  const bool qvalid = qi < T;
+  const int qpos = past + qi;
+  const size_t head_off = ((size_t)sidx * H + h) * (size_t)P * 64;
+  const float* Kh = kc + head_off;
+  const float* Vh = vc + head_off;
+  float(*Ks)[FA_KP] = reinterpret_cast<float(*)[FA_KP]>(&sm[wave][0]);
+  float(*Vt)[FA_VP] = reinterpret_cast<float(*)[FA_VP]>(&sm[wave][FA_K * FA_KP]);
+  float q[32];
+  {
+    const float* qrow = qkv + ((size_t)sidx * T + min(qi, T - 1)) * 3 * d + h * 64 + 32 * hh;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float4 v = reinterpret_cast<const float4*>(qrow)[j];
+      q[4 * j] = v.x;
+      q[4 * j + 1] = v.y;
+      q[4 * j + 2] = v.z;
+      q[4 * j + 3] = v.w;
+    }
+  }
+  const int kmax = past + min(T, (qb + 1) * FA_QW) - 1;
+  const int nkb = kmax / FA_K + 1;
+  float4 kr[8], vr[8];
+  auto load_block = [&](int kb) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = lane + u * 64;
+      const int r = e >> 4, c4 = (e & 15) * 4, j = kb * FA_K + r;
+      const bool ok = j <= kmax;
+      kr[u] = ok ? *reinterpret_cast<const float4*>(Kh + (size_t)j * 64 + c4) : make_float4(0.f, 0.f, 0.f, 0.f);
+      vr[u] = ok ? *reinterpret_cast<const float4*>(Vh + (size_t)j * 64 + c4) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  float m = -INFINITY, l = 0.f;
+  floatx16 o0, o1;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    o0[i] = 0.f;
+    o1[i] = 0.f;
+  }
+  if (wave < nkb) load_block(wave);
+  for (int kb = wave; kb < nkb; kb += KS) {
+    // this wave's region only: LDS accesses of one wave are ordered, the
+    // wave's previous reads are complete before its writes below
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = lane + u * 64;
+      const int r = e >> 4, c4 = (e & 15) * 4;
+      *reinterpret_cast<float4*>(&Ks[r][c4]) = kr[u];
+      Vt[c4][r] = vr[u].x;
+      Vt[c4 + 1][r] = vr[u].y;
+      Vt[c4 + 2][r] = vr[u].z;
+      Vt[c4 + 3][r] = vr[u].w;
+    }
+    if (kb + KS < nkb) load_block(kb + KS);
+    floatx16 sc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float4 a = *reinterpret_cast<const float4*>(&Ks[c][32 * hh + 4 * j]);
+      sc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, q[4 * j], sc, 0, 0, 0);
+      sc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, q[4 * j + 1], sc, 0, 0, 0);
+      sc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, q[4 * j + 2], sc, 0, 0, 0);
+      sc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, q[4 * j + 3], sc, 0, 0, 0);
+    }
+    const int j0 = kb * FA_K;
+    float bm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int j = j0 + (i / 4) * 8 + hh * 4 + (i % 4);
+      sc[i] = j <= qpos ? sc[i] * 0.125f : -INFINITY;
+      bm = fmaxf(bm, sc[i]);
+    }
+    bm = xor32_max_k(bm);
+    const float mn = fmaxf(m, bm);
+    const float corr = m == -INFINITY ? 0.f : fexp_a(m - mn);
+    float ps = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      sc[i] = sc[i] == -INFINITY ? 0.f : fexp_a(sc[i] - mn);
+      ps += sc[i];
+    }
+    l = l * corr + ps;
+    m = mn;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      o0[i] *= corr;
+      o1[i] *= corr;
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 v0 = *reinterpret_cast<const float4*>(&Vt[c][8 * g + 4 * hh]);
+      const float4 v1 = *reinterpret_cast<const float4*>(&Vt[32 + c][8 * g + 4 * hh]);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v0.x, sc[4 * g], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1.x, sc[4 * g], o1, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v0.y, sc[4 * g + 1], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1.y, sc[4 * g + 1], o1, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v0.z, sc[4 * g + 2], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1.z, sc[4 * g + 2], o1, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(v0.w, sc[4 * g + 3], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(v1.w, sc[4 * g + 3], o1, 0, 0, 0);
+    }
+  }
+  l = xor32_sum_k(l);
+  // merge records: query c of wave w at sm[w][c * MW]: m, l, O[64]
+  __syncthreads();  // every wave is done with its staging region
+  float* rec = &sm[wave][c * MW];
+  if (hh == 0) {
+    rec[0] = m;
+    rec[1] = l;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int r = (i / 4) * 8 + hh * 4 + (i % 4);
+    rec[2 + r] = o0[i];
+    rec[2 + 32 + r] = o1[i];
+  }
+  __syncthreads();
+  // wave 0 lane (c, hh) merges the 32 dims it holds for query c
+  if (wave == 0 && qvalid) {
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < KS; ++w) M = fmaxf(M, sm[w][c * MW]);
+    float L = 0.f, f[KS];
+#pragma unroll
+    for (int w = 0; w < KS; ++w) {
+      const float mw = sm[w][c * MW];
+      f[w] = mw == -INFINITY ? 0.f : fexp_a(mw - M);
+      L += sm[w][c * MW + 1] * f[w];
+    }
+    const float inv = 1.0f / L;
+    float* orow = out + ((size_t)sidx * T + qi) * d + h * 64;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = (i / 4) * 8 + hh * 4 + (i % 4);
+      float a = 0.f, b = 0.f;
+#pragma unroll
+      for (int w = 0; w < KS; ++w) {
+        a += sm[w][c * MW + 2 + r] * f[w];
+        b += sm[w][c * MW + 2 + 32 + r] * f[w];
+      }
+      orow[r] = a * inv;
+      orow[32 + r] = b * inv;
+    }
+  }
+}
+
 void launch_attn_prefill(hipStream_t s, const float* qkv, int S, int T, int past, const float* kc, const float* vc,
-                         int n_head, int n_pos, int d, float* out_rows, uint16_t* pair, const float* scale) {
-  const AttnOut out{out_rows, pair, scale};
+                         int n_head, int n_pos, int d, float* out, uint16_t* pair, const float* scale) {
+  // (the pair GEMM's models take attn_pair.hip at head_dim 64)
+  const bool mfma = d / n_head == 64 && pair == nullptr;
+  if (mfma && (long)n_head * S < 256 && T + past >= 4 * FA_K) {
+    // few (sequence, head) pairs with long key ranges: split the keys over 4
+    // waves, 8 from 16 key blocks on (c3, 512 tokens of GPT-2 medium: 85.4k
+    // -> 96.9k tokens/s with 4, 5.25 -> 5.10-5.23 ms with 8; c2, 8 x 128
+    // tokens: 3.885 -> 3.82 ms with 4)
+    const int nqb = (T + FA_QW - 1) / FA_QW;
+    const dim3 grid(n_head, S, nqb);
+    if (T + past >= 16 * FA_K)
+      attn_prefill_ks_kernel<8><<<grid, 512, 0, s>>>(qkv, T, past, kc, vc, n_head, n_pos, d, nqb, out);
+    else
+      attn_prefill_ks_kernel<4><<<grid, 256, 0, s>>>(qkv, T, past, kc, vc, n_head, n_pos, d, nqb, out);
+    return;
+  }
+  if (mfma) {
+    // 128 queries per workgroup where that gives two workgroups per CU, else
+    // 64 or 32 (a short batch of prompts would otherwise leave most CUs idle)
+    int fw = 4;
+    while (fw > 1 && (long)n_head * S * ((T + FA_QW * fw - 1) / (FA_QW * fw)) < 512) fw >>= 1;
+    const int nqb = (T + FA_QW * fw - 1) / (FA_QW * fw);
+    dim3 grid(n_head, S, nqb);
+    if (fw == 4)
+      attn_prefill_mfma_kernel<4><<<grid, 256, 0, s>>>(qkv, T, past, kc, vc, n_head, n_pos, d, nqb, out);
+    else if (fw == 2)
+      attn_prefill_mfma_kernel<2><<<grid, 128, 0, s>>>(qkv, T, past, kc, vc, n_head, n_pos, d, nqb, out);
+    else
+      attn_prefill_mfma_kernel<1><<<grid, 64, 0, s>>>(qkv, T, past, kc, vc, n_head, n_pos, d, nqb, out);
+    return;
+  }
   dim3 grid((T + PQ - 1) / PQ, n_head, S);
-  attn_prefill_kernel<<<grid, PQ, 0, s>>>(qkv, T, past, kc, vc, n_head, n_pos, d, d / n_head, out);
+  attn_prefill_kernel<<<grid, PQ, 0, s>>>(qkv, T, past, kc, vc, n_head, n_pos, d, d / n_head,
+                                          AttnOut{out, pair, scale});
 }
 
 // ---------------------------------------------------------------------------

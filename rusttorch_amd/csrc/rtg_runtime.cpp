@@ -373,14 +373,15 @@ static void destroy_graph(rtg_cache* c) {
   c->graph = nullptr;
 }
 
-// Floats the layer GEMMs of a prefill over M rows use to split over k.
-static size_t prefill_ws_floats(const rtg_model* m, size_t M) {
+// Floats the layer GEMMs of a prefill over M rows use to split over k, on the
+// pair GEMMs or on the f32-MFMA ones.
+static size_t prefill_ws_floats(const rtg_model* m, size_t M, bool pair) {
   const int d = (int)m->cfg.n_embd, planes = m->wtype == W_F32 ? 2 : 1;
   size_t ws = 0;
   for (const auto& nk : {std::make_pair(3 * d, d), std::make_pair(d, d), std::make_pair(4 * d, d),
                          std::make_pair(d, 4 * d)})
-    ws = std::max(ws, m->pw ? pair_gemm_ws_floats((int)M, nk.first, nk.second, planes)
-                            : gemm_splitk_ws_floats((int)M, nk.first, nk.second));
+    ws = std::max(ws, pair ? pair_gemm_ws_floats((int)M, nk.first, nk.second, planes)
+                           : gemm_splitk_ws_floats((int)M, nk.first, nk.second));
   return ws;
 }
 
@@ -398,8 +399,10 @@ static void ensure_rows(rtg_cache* c, size_t rows) {
   // the split-k workspace for the largest need of the four layer GEMMs at
   // any row count up to cap (the split depends on the row blocks)
   size_t ws = 0;
-  for (size_t r = 32; r < cap + 128; r += (c->m->pw || r < 128 ? 32 : 128))
-    ws = std::max(ws, prefill_ws_floats(c->m, std::min(r, cap)));
+  for (size_t r = 32; r < cap + 128; r += (r < 128 ? 32 : 128))
+    ws = std::max(ws, prefill_ws_floats(c->m, std::min(r, cap), false));
+  for (size_t r = 32; c->m->pw && r < cap + 32; r += 32)
+    ws = std::max(ws, prefill_ws_floats(c->m, std::min(r, cap), true));
   if (ws) HIPX(hipMalloc(&c->ws, ws * 4));
   c->ws_floats = ws;
   c->rows_cap = cap;
@@ -552,11 +555,16 @@ static void enqueue_prefill_pair(rtg_cache* c, const Work& w, const uint32_t* id
 }
 
 // forward_cached body for S sequences x T new tokens (gpt2.rs:376-396) on the
-// MFMA prefill path, on the activation buffers w. ids_dev holds S*T ids.
+// MFMA prefill path, on the activation buffers w. ids_dev holds S*T ids. for_draws:
+// the logits go to the seeded sampler, which keeps the f32-MFMA GEMMs and the
+// attention that go with them for every model. The pair GEMMs' logits are as
+// close to 64 bits or closer, but differ by up to 1e-6; over a flat distribution
+// (45000 kept tokens of 2e-5) that moves one draw in a few hundred to the next
+// token, and the text behind a seed changes from there on.
 static void enqueue_prefill(rtg_cache* c, const Work& w, const uint32_t* ids_dev, size_t S, size_t T, size_t past,
-                            LogitRows logit_rows) {
+                            LogitRows logit_rows, bool for_draws = false) {
   const rtg_model* m = c->m;
-  if (m->pw) return enqueue_prefill_pair(c, w, ids_dev, S, T, past, logit_rows);
+  if (m->pw && !for_draws) return enqueue_prefill_pair(c, w, ids_dev, S, T, past, logit_rows);
   const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, M = (int)(S * T);
   const float eps = m->cfg.layer_norm_epsilon;
   hipStream_t s = c->stream;
@@ -1003,8 +1011,11 @@ static void generate_greedy(const rtg_model* m, const uint32_t* prompts, size_t 
   const size_t V = m->cfg.vocab_size, P = m->cfg.n_positions;
   const size_t steps = max_new > 0 ? max_new : 1;  // first token comes from prefill
   const bool rows = rows_path(c, B, n);
+  // Draws read the last row of an LM head over all rows (as the f32-MFMA GEMM
+  // sums it for that many; see enqueue_prefill).
+  const bool draws = sp && sp->temperature > 0.0f, all = rows || draws;
   ensure_rows(c, B * n);
-  ensure_logits(c, rows ? B * n : B);
+  ensure_logits(c, all ? B * n : B);
   if (sp) ensure_sample_work(c);
   hipStream_t s = c->stream;
   // overwrite the argmax token of the step just enqueued with the sampler's choice
@@ -1040,11 +1051,11 @@ static void generate_greedy(const rtg_model* m, const uint32_t* prompts, size_t 
     enqueue_rows(c, c->ids_in, B, n, 0, c->logits, nullptr, &fin);
   } else {
     // argmax of the last row of each sequence (extract_row(logits, n-1))
-    enqueue_prefill(c, cache_work(c), c->ids_in, B, n, 0, LOGITS_LAST);
-    launch_argmax(s, c->logits, (long)V, (int)B, (int)V, c->keys);
+    enqueue_prefill(c, cache_work(c), c->ids_in, B, n, 0, all ? LOGITS_ALL : LOGITS_LAST, draws);
+    launch_argmax(s, c->logits + (all ? (n - 1) * V : 0), (long)(all ? n * V : V), (int)B, (int)V, c->keys);
     launch_finalize(s, (int)B, c->keys, c->token_dev, c->ids_dev, (int)P, c->pos_dev, c->step_dev);
   }
-  sample(rows ? c->logits + (n - 1) * V : c->logits);
+  sample(all ? c->logits + (n - 1) * V : c->logits);
   HIPX(hipEventRecord(c->ev[1], s));
   // The persistent step (one kernel) is launched directly: replaying it as a
   // one-node graph was measured to leave ~8 us between launches instead of ~1.
@@ -1629,7 +1640,7 @@ rtg_result rtg_forward_cached_noalloc(const rtg_model* model, rtg_cache* cache, 
   const size_t pv = align_up(n * V, 64);
   // the split-k partial tiles the pass's GEMMs use at n rows (as much as the
   // cache's own workspace would hold for them, so the same kernels run)
-  size_t pw = prefill_ws_floats(model, n);
+  size_t pw = prefill_ws_floats(model, n, model->pw != nullptr);
   pw = align_up(pw, 64);
   const size_t need = 3 * pd + p3 + p4 + pv;
   if (need > kScratchFloats)
@@ -1797,7 +1808,7 @@ rtg_result rtg_generate(const rtg_model* model, const uint32_t* prompt, size_t n
     for (size_t i = 0; i < max_new; ++i) {
       const size_t len = n + i;
       const size_t start = len > P ? len - P : 0;
-      enqueue_prefill(c, cache_work(c), toks + start, 1, len - start, 0, LOGITS_LAST);
+      enqueue_prefill(c, cache_work(c), toks + start, 1, len - start, 0, LOGITS_LAST, temperature > 0.0f);
       if (!launch_sample(s, c->logits, (int)V, toks, (int)n, toks + n, steps + i, sp, c->token_dev,
                          c->sample_work))
         throw HipError{"vocabulary too large for the device sampler"};
