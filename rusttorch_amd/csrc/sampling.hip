@@ -603,23 +603,31 @@ __device__ __forceinline__ uint32_t sample_whole(const float* __restrict__ logit
 //
 // sample_segments_kernel: workgroup b takes 1024 consecutive logits, applies
 // the penalty and the temperature, and leaves the scaled logits y and, per
-// segment of 64 consecutive ones, their maximum and their sum of
-// exp(y - maximum). sample_pick_kernel, one workgroup, then reads the <= 1024
-// segment records and only the segments that matter:
+// segment of 64 consecutive ones, their maximum. sample_pick_kernel, one
+// workgroup, then reads the <= 1024 segment records and only the segments that
+// matter:
 //  - top-k: a segment whose maximum is below k others' holds none of the k
 //    largest, so about k segments are read (those that reach a bound just
 //    below the k-th largest maximum); of these, values below the bound are
 //    dropped. What is left (about k values) is ranked by comparing all pairs, for top-k (fewer than k
 //    larger) and for top-p (the mass ranked before it below p, the rule of the
 //    histogram rounds above: masses are integers).
-//  - no filter: the segment where the running sum passes the draw.
+//  - no filter: sample_sums_kernel, between the two, adds up every segment's
+//    exp(y - maximum of the row); then the segment where the running sum passes
+//    the draw.
 //  - greedy: the segments' best keys.
+// The segments are the (row, wave) segments of the passes above, summed by the
+// same tree, and their prefix runs over the same entries, so that every sum and
+// with it every pick is the whole row's, bit for bit: with sums in another
+// order one draw in a few thousand over a flat row fell on the next token.
 // More candidates than fit (many ties), infinities and NaN take the passes
 // over the whole row above, in the same launch.
 // One workgroup's VALU and LDS atomics bounded the whole-row passes: GPT-2's
 // 50257 logits with top-k 50, top-p 0.95 and a penalty took 73 us per token, now
-// 5.3 (segments) + 17.3 (pick), most of the latter the latency of its own
-// instruction fetches and of the chain of LDS and memory round trips.
+// 4.9 (segments) + 22.7 (pick; 14.9 without top-p), most of the latter the
+// latency of its own instruction fetches and of the chain of LDS and memory round
+// trips (17.3 with sums over the survivors alone, in another order);
+// temperature alone 23.5 us, now 4.8 + 4.9 (sums) + 6.0.
 constexpr int SEG = 64, SEGS_MAX = MAX_ROWS * ST / SEG;  // 1024
 constexpr int AT = 256, AW = 1024;                       // threads and logits of one segment workgroup
 constexpr int CREG = 16;                                 // candidate values per thread: 8192 in 128 segments
@@ -627,8 +635,8 @@ constexpr int SURV = 512;                                // values ranked
 
 struct SampleWork {
   float* y;                     // [V] scaled logits
-  float* segmax;                // [segments]
-  float* segsum;                // [segments]; NaN where the segment holds one
+  float* segmax;                // [segments]; NaN where the segment holds one
+  float* segsum;                // [segments] no filter: sum of exp(y - maximum of the row)
   unsigned long long* segkey;   // [segments] greedy: best argmax key
 };
 
@@ -692,24 +700,44 @@ __global__ __launch_bounds__(AT) void sample_segments_kernel(const float* __rest
     const float y = i < V ? x[r] / temperature : -INFINITY;
     if (i < V) wk.y[i] = y;
     const float m = wave_max_s(y);
-    float e = y > -INFINITY ? expf(y - m) : 0.f;
-    if (y != y) e = y;
+    const bool nan = __any(y != y);
+    if (lane == 0) wk.segmax[seg] = nan ? NAN : m;
+  }
+}
+
+// segsum of the 16 segments of a workgroup, each added up as seg_sums does.
+__global__ __launch_bounds__(AT) void sample_sums_kernel(int V, SampleWork wk) {
+  __shared__ float red[AT / 64];
+  constexpr int R = AW / AT;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nseg = (V + SEG - 1) / SEG;
+  const int first = blockIdx.x * AW + wave * (R * 64);
+  float y[R], m = -INFINITY;
+#pragma unroll
+  for (int r = 0; r < R; ++r) y[r] = wk.y[min(first + r * 64 + lane, V - 1)];
+#pragma unroll
+  for (int r = 0; r < SEGS_MAX / AT; ++r) m = fmaxf(m, wk.segmax[min(t + r * AT, nseg - 1)]);
+  m = wave_max_s(m);
+  if (lane == 0) red[wave] = m;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < AT / 64; ++i) m = fmaxf(m, red[i]);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = first + r * 64 + lane;
+    if (first + r * 64 >= V) break;  // wave-uniform
+    float e = i < V && y[r] > -INFINITY ? expf(y[r] - m) : 0.f;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
-    if (lane == 0) {
-      wk.segmax[seg] = m;
-      wk.segsum[seg] = e;
-    }
+    if (lane == 0) wk.segsum[i / SEG] = e;
   }
 }
 
 struct PickSmem {
   float segmax[SEGS_MAX];
-  float seg[SEGS_MAX];     // sums in index order (segments, or survivors) and
+  float seg[SEGS_MAX];     // sums per segment and
   float segpre[SEGS_MAX];  // their exclusive prefix
   uint16_t cand[SEGS_MAX];
-  float val[SURV];
-  uint32_t idx[SURV];
+  float val[SURV];         // survivors: scaled logits, then exp(y - maximum)
   unsigned mass[SURV];
   float red[2 * SW];
   unsigned wtot[SW];
@@ -739,9 +767,9 @@ __device__ __forceinline__ unsigned pick_scan(unsigned x, PickSmem& sm, unsigned
   return base + incl - x;
 }
 
-// The first of n (<= 1024) entries of sm.seg whose running sum exceeds
-// r * (their sum), r a uniform draw; NONE when none does. Every thread gets it
-// (and that entry's exclusive prefix in *before, the threshold in *rs).
+// The first of n (<= 1024) segments whose running sum exceeds r * (the sum of
+// all), r a uniform draw; NONE when none does. Every thread gets it (and that
+// segment's exclusive prefix in *before, the threshold in *rs).
 __device__ __forceinline__ uint32_t pick_entry(PickSmem& sm, int n, float r, float* before, float* rs) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   __syncthreads();
@@ -766,26 +794,49 @@ __device__ __forceinline__ uint32_t pick_entry(PickSmem& sm, int n, float r, flo
   return sm.misc[0];
 }
 
-// The pick from the segment records; false when the whole row is needed.
+// One wave, its lanes holding segment seg's p = exp(y - maximum) (0: removed),
+// before the running sum up to it: the index where it passes rs. Should the
+// running sum stop short of the segment's (a tree) by rounding, its last index
+// of non-zero probability.
+__device__ __forceinline__ uint32_t pick_in_segment(float p, uint32_t seg, float before, float rs, int V, int lane) {
+  float incl = p;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const float u = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += u;
+  }
+  const unsigned long long bal = __ballot((int)seg * SEG + lane < V && rs < before + incl);
+  const unsigned long long nz = __ballot(p > 0.f);
+  return bal ? seg * SEG + (uint32_t)__builtin_ctzll(bal)
+             : nz ? seg * SEG + 63u - (uint32_t)__builtin_clzll(nz) : (uint32_t)(V - 1);
+}
+
+// The pick from the segment records; false when the whole row is needed. NJ:
+// registers per thread of sample_whole's row, whose NJ * SW segments the sums
+// run over.
+template <int NJ>
 __device__ __forceinline__ bool pick_from_segments(const SampleWork& wk, int V, int g, const SampleParams& sp, PickSmem& sm,
                                    uint32_t* pick) {
   const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+  constexpr int NS = NJ * SW;  // >= nseg; the segments past the row are empty
   const int nseg = (V + SEG - 1) / SEG;
+  const bool top_k = sp.top_k > 0 && sp.top_k < V;
   // segments 2t and 2t + 1 of this thread
-  float m2[2], s2[2];
+  float m2[2];
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     const int i = min(2 * t + q, nseg - 1);
     m2[q] = wk.segmax[i];
-    s2[q] = wk.segsum[i];
+    float s = top_k ? 0.f : wk.segsum[i];
     if (2 * t + q >= nseg) {
       m2[q] = -INFINITY;
-      s2[q] = 0.f;
+      s = 0.f;
     }
     sm.segmax[2 * t + q] = m2[q];
+    sm.seg[2 * t + q] = s;
   }
   float mx = wave_max_s(fmaxf(m2[0], m2[1]));
-  const bool bad = __any(s2[0] != s2[0] || s2[1] != s2[1]);
+  const bool bad = __any(m2[0] != m2[0] || m2[1] != m2[1]);
   if (lane == 0) {
     sm.red[w] = mx;
     sm.red[SW + w] = bad ? 1.f : 0.f;
@@ -801,30 +852,16 @@ __device__ __forceinline__ bool pick_from_segments(const SampleWork& wk, int V, 
   const float r =
       (float)(splitmix_at(sp.seed, (uint64_t)sp.draw0 + (uint64_t)g + 1) >> 40) * (1.0f / 16777216.0f);
   float before, rs;
-  if (sp.top_k <= 0 || sp.top_k >= V) {
+  if (!top_k) {
     // ---- temperature only: the segment, then the index inside it ----
-#pragma unroll
-    for (int q = 0; q < 2; ++q) sm.seg[2 * t + q] = s2[q] > 0.f ? s2[q] * expf(m2[q] - mx) : 0.f;
-    const uint32_t seg = pick_entry(sm, nseg, r, &before, &rs);
+    const uint32_t seg = pick_entry(sm, NS, r, &before, &rs);
     if (seg == NONE) {
       *pick = (uint32_t)(V - 1);
       return true;
     }
     const int i = (int)seg * SEG + lane;
     const float y = i < V ? wk.y[i] : -INFINITY;
-    const float p = y > -INFINITY ? expf(y - mx) : 0.f;
-    float incl = p;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const float u = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += u;
-    }
-    const unsigned long long bal = __ballot(i < V && rs < before + incl);
-    // (the running sum may stop short of the segment's by rounding: then its
-    // last index of non-zero probability)
-    const unsigned long long nz = __ballot(p > 0.f);
-    *pick = bal ? seg * SEG + (uint32_t)__builtin_ctzll(bal)
-                : nz ? seg * SEG + 63u - (uint32_t)__builtin_clzll(nz) : (uint32_t)(V - 1);
+    *pick = pick_in_segment(y > -INFINITY ? expf(y - mx) : 0.f, seg, before, rs, V, lane);
     return true;
   }
   // ---- top-k: a bound that at least k segments' maxima reach (the top 16
@@ -859,7 +896,7 @@ __device__ __forceinline__ bool pick_from_segments(const SampleWork& wk, int V, 
   __syncthreads();
   if (nc > (unsigned)(CREG * SW)) return false;
   // candidate c = CREG * wave + j: consecutive per wave, so that survivors
-  // gather in index order
+  // gather in index order, lane l holding index l of the segment
   float v[CREG];
   unsigned mine = 0;
 #pragma unroll
@@ -883,14 +920,12 @@ __device__ __forceinline__ bool pick_from_segments(const SampleWork& wk, int V, 
     ns += sm.wtot[i];
   }
   if (ns > (unsigned)SURV) return false;
+  int at_val[CREG];  // this lane's survivor of candidate j, or -1
 #pragma unroll
   for (int j = 0; j < CREG; ++j) {
     const unsigned long long bal = __ballot(v[j] >= low && v[j] > -INFINITY);
-    if ((bal >> lane) & 1ull) {
-      const unsigned p = pos + (unsigned)lanes_before(bal);
-      sm.val[p] = v[j];
-      sm.idx[p] = (uint32_t)sm.cand[CREG * w + j] * SEG + (uint32_t)lane;
-    }
+    at_val[j] = (bal >> lane) & 1ull ? (int)pos + lanes_before(bal) : -1;
+    if (at_val[j] >= 0) sm.val[at_val[j]] = v[j];
     pos += (unsigned)__popcll(bal);
   }
   __syncthreads();
@@ -901,12 +936,29 @@ __device__ __forceinline__ bool pick_from_segments(const SampleWork& wk, int V, 
 #pragma unroll 8
   for (unsigned i = 0; i < ns; ++i) larger += sm.val[i] > yv;
   float e = have && larger < k ? expf(yv - mx) : 0.f;
+  // segment sums of the e in sm.val, by seg_sums' tree
+  static_assert(CREG == 16, "the transposing butterfly's chunk");
+  auto sums = [&]() {
+    __syncthreads();  // every thread is done with sm.val and sm.seg
+    if (have) sm.val[t] = e;
+    __syncthreads();
+    float a[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) a[j] = at_val[j] >= 0 ? sm.val[at_val[j]] : 0.f;
+    tr_stage<16, 32>(a, lane);
+    tr_stage<8, 16>(a, lane);
+    tr_stage<4, 8>(a, lane);
+    tr_stage<2, 4>(a, lane);
+    a[0] += __shfl_xor(a[0], 2, 64);
+    a[0] += __shfl_xor(a[0], 1, 64);
+    const unsigned c = CREG * w + (lane >> 2);
+    if ((lane & 3) == 0 && c < nc) sm.seg[sm.cand[c]] = a[0];
+    __syncthreads();
+  };
+  sums();
   if (sp.top_p < 1.0f && sp.top_p > 0.0f) {
-    __syncthreads();
-    sm.seg[t] = e;
-    __syncthreads();
     if (w == 0) {
-      const float S = wave_excl_prefix(sm.seg, sm.segpre, (int)ns, lane);
+      const float S = wave_excl_prefix(sm.seg, sm.segpre, NS, lane);
       if (lane == 0) sm.fmisc[0] = S;
     }
     __syncthreads();
@@ -917,16 +969,26 @@ __device__ __forceinline__ bool pick_from_segments(const SampleWork& wk, int V, 
     unsigned before_mass = 0;
 #pragma unroll 8
     for (unsigned i = 0; i < ns; ++i) {
-      const float o = sm.seg[i];
+      const float o = sm.val[i];
       if (o > e || (o == e && i < (unsigned)t)) before_mass += sm.mass[i];
     }
     if (before_mass >= target) e = 0.f;
-    __syncthreads();
+    sums();
   }
+  const uint32_t seg = pick_entry(sm, NS, r, &before, &rs);
+  if (seg == NONE) {
+    *pick = (uint32_t)(V - 1);
+    return true;
+  }
+  // (the wave that holds the segment; each is a candidate once)
+#pragma unroll
+  for (int j = 0; j < CREG; ++j)
+    if (CREG * w + j < (int)nc && sm.cand[CREG * w + j] == seg) {  // wave-uniform
+      const uint32_t i = pick_in_segment(at_val[j] >= 0 ? sm.val[at_val[j]] : 0.f, seg, before, rs, V, lane);
+      if (lane == 0) sm.misc[1] = i;
+    }
   __syncthreads();
-  if (have) sm.seg[t] = e;
-  const uint32_t f = pick_entry(sm, (int)ns, r, &before, &rs);
-  *pick = f == NONE ? (uint32_t)(V - 1) : sm.idx[f];
+  *pick = sm.misc[1];
   return true;
 }
 
@@ -971,7 +1033,7 @@ __global__ __launch_bounds__(ST) void sample_pick_kernel(const float* __restrict
     if (lane == 0) atomicMax(&sm.whole.key, k);
     __syncthreads();
     pick = argmax_key_index(sm.whole.key);
-  } else if (!pick_from_segments(wk, V, g, sp, sm.part, &pick)) {
+  } else if (!pick_from_segments<NJ>(wk, V, g, sp, sm.part, &pick)) {
     __syncthreads();
     pick = sample_whole<NJ>(logits, V, prompt, n_prompt, ids, g, sp, sm.whole);
   }
@@ -992,7 +1054,7 @@ bool launch_sample(hipStream_t s, const float* logits, int V, const uint32_t* pr
                    const int* step_dev, const SampleParams& sp, uint32_t* token, void* work) {
   if (V <= 0 || V > MAX_ROWS * ST) return false;
   // Segments for rows that one workgroup takes long over, unless top-p alone
-  // filters (its kept set is not small) or top-k keeps more than the ranking
+  // filters (its kept set is most of a flat row) or top-k keeps more than the ranking
   // is made for.
   const bool top_k = sp.top_k > 0 && sp.top_k < V, top_p = sp.top_p < 1.0f && sp.top_p > 0.0f;
   const bool segments =
@@ -1001,6 +1063,8 @@ bool launch_sample(hipStream_t s, const float* logits, int V, const uint32_t* pr
   if (segments)
     sample_segments_kernel<<<(V + AW - 1) / AW, AT, 0, s>>>(logits, V, prompt, n_prompt, ids, step_dev,
                                                             sp.temperature, sp.penalty, wk);
+  if (segments && !top_k && sp.temperature > 0.0f)
+    sample_sums_kernel<<<(V + AW - 1) / AW, AT, 0, s>>>(V, wk);
 #define RTG_SAMPLE(NJ)                                                                                         \
   do {                                                                                                         \
     if (segments)                                                                                              \

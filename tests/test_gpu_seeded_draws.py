@@ -5,9 +5,10 @@ and the whole-row sampler for every model.
 The models' distributions are nearly flat (random weights: tens of thousands of
 kept tokens of 2e-5 each), where a change of the logits or of the running sums
 by 1e-6 moves about one draw in a few hundred to the next token. The recorded
-cases are ones that came out differently with the prompt on the f16-pair GEMMs,
-one for every kind of GEMM that a prompt meets: up to 32 and 64 rows, more, f32
-and bf16 weights, and the uncached loop. Ids are whole numbers: equal."""
+cases are ones that came out differently: "topp" and "uncached" with the prompt
+on the f16-pair GEMMs, one for every kind of GEMM that a prompt meets (up to 32
+and 64 rows, more, f32 and bf16 weights, the uncached loop); "temp" with segment
+sums in another order than the whole row's. Ids are whole numbers: equal."""
 import pytest
 
 from rusttorch_amd import synth
@@ -53,6 +54,22 @@ IDS = {
         36916, 5871, 18238, 4188, 39400, 48142, 23945, 28681, 12518, 26470, 45479, 46562,
         40780, 43876, 39174, 37608, 27750, 28550, 22122, 29018, 28629, 17568, 27265, 1522,
         29727, 18656, 6210, 21173, 35697, 5110, 21307, 37133],
+    ("small", "f32", 45, "temp", 20): [
+        10638, 961, 12674, 18128, 5136, 8648, 41604, 15630, 4011, 17558, 6226, 38943,
+        18533, 26529, 33253, 33690, 1486, 22114, 38017, 40084, 2379, 10593, 26949, 13096,
+        48074, 26700, 35747, 400, 37502, 23136, 12985, 11538],
+    ("small", "bf16", 45, "temp", 31): [
+        42266, 37071, 25295, 27165, 29937, 16461, 19855, 30785, 13810, 38021, 39756, 15159,
+        32775, 8863, 17261, 10060, 7633, 17290, 47044, 9713, 8506, 42861, 7061, 38799,
+        22561, 17018, 26119, 795, 47672, 5540, 12150, 12771],
+    ("small", "bf16", 100, "temp", 18): [
+        3355, 35866, 21592, 35294, 6024, 46137, 49253, 6607, 35695, 26125, 19523, 43338,
+        41650, 1323, 43295, 13206, 2731, 9708, 50237, 22400, 30768, 35837, 23408, 26335,
+        4891, 11517, 4929, 29602, 22809, 33105, 41395, 6059],
+    ("wide", "bf16", 20, "temp", 38): [
+        46123, 410, 4021, 11210, 16475, 46531, 16519, 40052, 23112, 1670, 21127, 46281,
+        29316, 10920, 34562, 11729, 39491, 24780, 22625, 24052, 43012, 2052, 49071, 3666,
+        22267, 5004, 3875, 23808, 26848, 43249, 16256, 14703],
 }
 
 
