@@ -12,8 +12,9 @@ struct AttnScales {
   const float* k;
   const float* v;
 };
-// q[h], k[h] from the scales col[2 d] of c_attn's q and k columns.
-void launch_head_scale(hipStream_t s, const float* col, int H, float* q, float* k);
+// q[h], k[h] from the scales col[2 d] of c_attn's q and k columns, their product
+// between 2^-100 and 2^110; *bad is set nonzero where it would be smaller.
+void launch_head_scale(hipStream_t s, const float* col, int H, float* q, float* k, int* bad);
 
 // S sequences of T new tokens at offset past: qkv rows [S * T][3 d] (q columns
 // read), the cache of positions [0, past + T); out: pair matrix [S * T][d]

@@ -190,7 +190,8 @@ struct State {
   }
 };
 
-// score = (K . Q) / 8 (1 / sqrt(64)), in units of log2 e, of the scaled operands
+// score = (K . Q) / 8 (1 / sqrt(64)), in units of log2 e, of the scaled operands;
+// finite and not zero (head_scale_kernel), so that a masked score stays -inf
 __device__ __forceinline__ float score_factor(float aq, float ak) {
   return 0.125f * 1.4426950408889634f / (aq * ak);
 }
@@ -329,20 +330,32 @@ __global__ __launch_bounds__(64 * KS, 2) void attn_pair_ks_kernel(const float* _
   }
 }
 
-// The smallest scale of a head's 64 columns, for q (blocks [0, H)) and k.
+// A head's scales: the smallest of its 64 columns, for q and for k. Each may be
+// up to 2^80; where their product exceeds 2^110 the head's scores are below
+// 2^-77 (64 products of 2^30 over 2^110, over 8), the softmax is uniform
+// whatever they are, and a smaller q scale keeps the score factor from becoming
+// 0, whose product with a masked score is NaN. A product below 2^-100 (scores
+// that may pass f32's range) is left to the f32 attention.
 __global__ __launch_bounds__(64) void head_scale_kernel(const float* __restrict__ col, int H, float* __restrict__ q,
-                                                        float* __restrict__ k) {
-  const int b = blockIdx.x;
-  float v = col[b * 64 + threadIdx.x];
+                                                        float* __restrict__ k, int* bad) {
+  const int h = blockIdx.x;
+  float a = col[h * 64 + threadIdx.x], b = col[(H + h) * 64 + threadIdx.x];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
-  if (threadIdx.x == 0) (b < H ? q[b] : k[b - H]) = v;
+  for (int o = 32; o > 0; o >>= 1) {
+    a = fminf(a, __shfl_xor(a, o, 64));
+    b = fminf(b, __shfl_xor(b, o, 64));
+  }
+  if (threadIdx.x != 0) return;
+  const int e = ilogbf(a) + ilogbf(b);
+  if (e < -100) *bad = 1;
+  q[h] = ldexpf(a, min(110 - e, 0));
+  k[h] = b;
 }
 
 }  // namespace
 
-void launch_head_scale(hipStream_t s, const float* col, int H, float* q, float* k) {
-  head_scale_kernel<<<2 * H, 64, 0, s>>>(col, H, q, k);
+void launch_head_scale(hipStream_t s, const float* col, int H, float* q, float* k, int* bad) {
+  head_scale_kernel<<<H, 64, 0, s>>>(col, H, q, k, bad);
 }
 
 void launch_attn_pair(hipStream_t s, const float* qkv, int S, int T, int past, const float* kc, const float* vc,

@@ -1191,7 +1191,7 @@ static void build_prefill_weights(rtg_model* m, std::unique_ptr<PrefillWeights> 
     launch_pair_ln_scale(s, W.ln2w, W.ln2b, d, s2, bad);
     // attention averages value rows, so its output has the bound of c_attn's v
     launch_pair_row_scale(s, W.wqkv, wt, 3 * d, d, W.ln1w, W.ln1b, W.bqkv, sqkv, bad);
-    if (m->hd == 64) launch_head_scale(s, sqkv, H, heads, heads + H);
+    if (m->hd == 64) launch_head_scale(s, sqkv, H, heads, heads + H, bad);
     l.att = AttnScales{heads, heads + H, sqkv + 2 * d};
     launch_pair_row_scale(s, W.wfc, wt, 4 * d, d, W.ln2w, W.ln2b, W.bfc, sh4, bad);
     l.s1 = s1;

@@ -106,6 +106,22 @@ def test_spread_magnitudes(oracle_lib):
     m.close()
 
 
+@pytest.mark.parametrize("chunks", [(77,), (200,)])  # a wave of keys per workgroup, and the keys split over waves
+@pytest.mark.parametrize("what", ["collapsed head", "collapsed keys"])
+def test_score_range(oracle_lib, what, chunks):
+    """A head whose queries and keys are 1e-20 (its scores are 0: uniform
+    attention), and one whose keys alone are."""
+    def change(sd):
+        w, b = sd["h.0.attn.c_attn.weight"], sd["h.0.attn.c_attn.bias"]
+        for first in (64, 192 + 64) if what == "collapsed head" else (192 + 64,):
+            w[:, first:first + 64] *= 1e-20
+            b[first:first + 64] *= 1e-20
+    sh = synth.ModelShape(301, 256, 192, 1, 3)
+    sd, m = build(sh, change=change)
+    check(oracle_lib, sh, sd, m, chunks)
+    m.close()
+
+
 @pytest.mark.parametrize("what", ["nan bias", "inf weight", "negative epsilon"])
 def test_models_outside_the_bounds(oracle_lib, what):
     """No finite bound, or an epsilon for which it does not hold: the f32 GEMMs
