@@ -28,7 +28,7 @@ size_t pair_weight_bytes(int N, int K, int wtype);
 // of anything no larger: averages over rows, gelu), by Cauchy-Schwarz at most
 // sqrt(K) |W[n] * g|_2 + |W[n] . b + bias[n]|. Each value times its scale is
 // at most 2^15 in magnitude, half of f16's range. *bad is set nonzero where a
-// bound is not finite.
+// bound is 2^95 or more, or not a number.
 void launch_pair_ln_scale(hipStream_t s, const float* g, const float* b, int d, float* scale, int* bad);
 void launch_pair_row_scale(hipStream_t s, const void* W, int wtype, int N, int K, const float* g, const float* b,
                            const float* bias, float* scale, int* bad);

@@ -40,16 +40,18 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 // ---- scales and weights, once per model ----
 
-// The power of two that brings a bound below 2^15 (1 for a zero bound).
+// The power of two that brings a bound below 2^15 (1 for a zero bound), at most
+// 2^80. A bound of 2^95 or more (or none) sets *bad: no scale down to 2^-80
+// keeps such values in f16.
 __device__ __forceinline__ float scale_of(double bound, int* bad) {
-  if (!(bound < 1e30)) {
+  if (!(bound < 0x1p95)) {
     *bad = 1;
     return 1.f;
   }
   if (bound == 0.0) return 1.f;
   int e;
-  frexp(bound, &e);  // bound < 2^e
-  return (float)ldexp(1.0, min(max(15 - e, -80), 80));
+  frexp(bound, &e);  // bound < 2^e <= 2^95
+  return (float)ldexp(1.0, min(15 - e, 80));
 }
 
 __global__ __launch_bounds__(256) void pair_ln_scale_kernel(const float* __restrict__ g, const float* __restrict__ b,

@@ -107,12 +107,17 @@ def test_spread_magnitudes(oracle_lib):
 
 
 @pytest.mark.parametrize("chunks", [(77,), (200,)])  # a wave of keys per workgroup, and the keys split over waves
-@pytest.mark.parametrize("what", ["collapsed head", "collapsed keys"])
+@pytest.mark.parametrize("what", ["collapsed head", "collapsed keys", "large value"])
 def test_score_range(oracle_lib, what, chunks):
     """A head whose queries and keys are 1e-20 (its scores are 0: uniform
-    attention), and one whose keys alone are."""
+    attention), one whose keys alone are, and a value column of 1e29 that c_proj
+    brings back to 1 (past the bounds: the f32 kernels run)."""
     def change(sd):
         w, b = sd["h.0.attn.c_attn.weight"], sd["h.0.attn.c_attn.bias"]
+        if what == "large value":
+            b[2 * 192 + 64] = 1e29
+            sd["h.0.attn.c_proj.weight"][64] *= 1e-29
+            return
         for first in (64, 192 + 64) if what == "collapsed head" else (192 + 64,):
             w[:, first:first + 64] *= 1e-20
             b[first:first + 64] *= 1e-20
