@@ -149,9 +149,12 @@ __global__ __launch_bounds__(256) void pair_weights_kernel(const void* __restric
 __device__ __forceinline__ void dma16(unsigned voff, const void* base, unsigned lds) {
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds) : "memory", "m0");
 }
+// At most N of this wave's loads outstanding and its LDS reads complete, then
+// the barrier. (The reads' results may be used behind it: nothing but this wait
+// keeps another wave's load from overwriting a stage still being read.)
 template <int N>
 __device__ __forceinline__ void wait_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 __device__ __forceinline__ f16x8 lds_frag(const char* p) { return *reinterpret_cast<const f16x8*>(p); }

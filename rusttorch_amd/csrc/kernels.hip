@@ -796,10 +796,12 @@ __device__ __forceinline__ void gl_dma16(const float* src, const float* lds_dst)
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0v) : "memory", "m0");
 }
 // Wait until at most N of this wave's vector memory operations are
-// outstanding, then a workgroup barrier; memory accesses do not move across.
+// outstanding and its LDS reads are complete (another wave's load may overwrite
+// their stage behind the barrier, and their results may be used only there),
+// then a workgroup barrier; memory accesses do not move across.
 template <int N>
 __device__ __forceinline__ void gl_wait_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
 // One k-tile step of gemm_lds_kernel on stage ST. Each stage is its own LDS
