@@ -385,6 +385,20 @@ static size_t prefill_ws_floats(const rtg_model* m, size_t M, bool pair) {
   return ws;
 }
 
+// The split-k workspace for the largest need of the four layer GEMMs at any row
+// count up to cap (the split depends on the row blocks).
+static void ensure_ws(rtg_cache* c, size_t cap, bool pair) {
+  size_t ws = 0;
+  for (size_t r = 32; r < cap + 128; r += (pair || r < 128 ? 32 : 128))
+    ws = std::max(ws, prefill_ws_floats(c->m, std::min(r, cap), pair));
+  if (ws <= c->ws_floats) return;
+  if (c->ws) hipFree(c->ws);
+  c->ws = nullptr;
+  c->ws_floats = 0;
+  HIPX(hipMalloc(&c->ws, ws * 4));
+  c->ws_floats = ws;
+}
+
 static void ensure_rows(rtg_cache* c, size_t rows) {
   if (rows <= c->rows_cap) return;
   destroy_graph(c);
@@ -396,15 +410,7 @@ static void ensure_rows(rtg_cache* c, size_t rows) {
   HIPX(hipMalloc(&c->qkv, cap * 3 * d * 4));
   HIPX(hipMalloc(&c->att, cap * d * 4));
   HIPX(hipMalloc(&c->h, cap * 4 * d * 4));
-  // the split-k workspace for the largest need of the four layer GEMMs at
-  // any row count up to cap (the split depends on the row blocks)
-  size_t ws = 0;
-  for (size_t r = 32; r < cap + 128; r += (r < 128 ? 32 : 128))
-    ws = std::max(ws, prefill_ws_floats(c->m, std::min(r, cap), false));
-  for (size_t r = 32; c->m->pw && r < cap + 32; r += 32)
-    ws = std::max(ws, prefill_ws_floats(c->m, std::min(r, cap), true));
-  if (ws) HIPX(hipMalloc(&c->ws, ws * 4));
-  c->ws_floats = ws;
+  ensure_ws(c, cap, c->m->pw != nullptr);
   c->rows_cap = cap;
 }
 
@@ -1015,6 +1021,7 @@ static void generate_greedy(const rtg_model* m, const uint32_t* prompts, size_t 
   // sums it for that many; see enqueue_prefill).
   const bool draws = sp && sp->temperature > 0.0f, all = rows || draws;
   ensure_rows(c, B * n);
+  if (draws && !rows) ensure_ws(c, B * n, false);
   ensure_logits(c, all ? B * n : B);
   if (sp) ensure_sample_work(c);
   hipStream_t s = c->stream;
@@ -1800,6 +1807,7 @@ rtg_result rtg_generate(const rtg_model* model, const uint32_t* prompt, size_t n
     HIPX(hipMemcpyAsync(steps, step_no.data(), max_new * 4, hipMemcpyHostToDevice, s));
     c->len = 0;
     ensure_rows(c, std::min(total - 1, P));
+    if (temperature > 0.0f) ensure_ws(c, std::min(total - 1, P), false);
     ensure_logits(c, 1);
     ensure_sample_work(c);
     // sample_with_temperature (gpt2.rs:996-1017); argmax for temperature <= 0.
