@@ -140,7 +140,9 @@ void rtg_cache_destroy(rtg_cache* cache);
  * counterpart (the reference's LayerKVCache fields are private). */
 rtg_result rtg_cache_read(const rtg_cache* cache, size_t layer, size_t head, size_t seq, int values, float* out);
 
-/* Gpt2Model::forward, gpt2.rs:269-304: logits_out[n * vocab_size]. */
+/* Gpt2Model::forward, gpt2.rs:269-304: logits_out[n * vocab_size]. Here and
+ * below, a call that returns an error leaves logits_out as it was, or with part
+ * or all of what it had computed when the error was found. */
 rtg_result rtg_forward(const rtg_model* model, const uint32_t* ids, size_t n, float* logits_out);
 /* Gpt2Model::forward_cached, gpt2.rs:358-399: logits_out[n * vocab_size]
  * (may be NULL: nothing is copied, and a prompt of more than one token runs

@@ -10,19 +10,18 @@
 #include <string.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "../../include/rtgpu.h"
 #include "decode_persistent.h"
 #include "attn_pair.h"
 #include "bgemv.h"
+#include "copy_team.h"
 #include "gemm_pair.h"
 #include "kernels.h"
 #include "rows.h"
@@ -83,9 +82,9 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 // A call's results reach the caller's pageable memory through page-locked
 // staging buffers of the library's own: a small one (a token's logits) by one
 // kernel that also carries the launch's error word, a large one in chunks, the
-// next chunk's transfer running while helper threads copy this one out; they
-// first touch the destination's pages while the GPU computes (first writes to
-// fresh memory were most of that time). Through the runtime's own staging, one
+// next chunk's transfer running while helper threads copy this one out
+// (copy_team.h); they first touch the destination's pages while the GPU computes
+// (first writes to fresh memory were most of that time). Through the runtime's own staging, one
 // batch-1 token of GPT-2 small took 259 us with its logits (a 205 us step) and
 // a 333-token forward 4.9 ms with its 67 MB; now 235 us and 2.7 ms (3.0 without
 // the early touch).
@@ -133,71 +132,6 @@ HostStages& host_stages() {
   return *s;
 }
 
-// Copies dst[0, bytes) from chunks that the main thread announces, each chunk
-// split between the main thread and kHelpers threads.
-struct CopyTeam {
-  static constexpr int kHelpers = 3;
-  char* dst;
-  size_t bytes, chunk;
-  const char* buf[2];
-  std::atomic<size_t> ready{0}, done{0};
-  std::atomic<bool> stop{false};
-  std::vector<std::thread> threads;
-  CopyTeam(char* d, size_t n, size_t c, const char* b0, const char* b1) : dst(d), bytes(n), chunk(c), buf{b0, b1} {
-    try {
-      for (int i = 0; i < kHelpers; ++i) threads.emplace_back([this, i] { helper(i); });
-    } catch (const std::system_error&) {
-      // no more threads to be had: those that started share the work
-    }
-  }
-  ~CopyTeam() {
-    stop.store(true, std::memory_order_release);
-    for (auto& t : threads) t.join();
-  }
-  size_t count() const { return (bytes + chunk - 1) / chunk; }
-  size_t size(size_t i) const { return std::min(chunk, bytes - i * chunk); }
-  // Part `which` of chunk i: its range of dst.
-  void range(size_t i, size_t which, size_t* a, size_t* b) const {
-    const size_t n = size(i), each = align_up((n + kHelpers) / (kHelpers + 1), 4096);
-    *a = std::min(n, which * each);
-    *b = std::min(n, *a + each);
-  }
-  void part(size_t i, size_t which) {
-    size_t a, b;
-    range(i, which, &a, &b);
-    memcpy(dst + i * chunk + a, buf[i & 1] + a, b - a);
-  }
-  // Writes to every page of part `which` of all chunks, which makes fresh
-  // memory present while the GPU still computes what will be copied there.
-  void touch(size_t which) {
-    for (size_t i = 0; i < count(); ++i) {
-      size_t a, b;
-      range(i, which, &a, &b);
-      for (; a < b; a += 4096) *const_cast<volatile char*>(dst + i * chunk + a) = 0;
-    }
-  }
-  void helper(int which) {
-    // (the number of parts is fixed by kHelpers; threads that did not start
-    // leave theirs to the main thread)
-    touch(which + 1);
-    for (size_t i = 0; i < count(); ++i) {
-      while (ready.load(std::memory_order_acquire) <= i) {
-        if (stop.load(std::memory_order_acquire)) return;
-        std::this_thread::yield();
-      }
-      part(i, which + 1);
-      done.fetch_add(1, std::memory_order_acq_rel);
-    }
-  }
-  // Main thread: chunk i has arrived in buf[i & 1]; returns once it is in dst.
-  void copy(size_t i) {
-    ready.store(i + 1, std::memory_order_release);
-    part(i, 0);
-    for (size_t h = threads.size(); h < kHelpers; ++h) part(i, h + 1);
-    while (done.load(std::memory_order_acquire) < (i + 1) * threads.size()) std::this_thread::yield();
-  }
-};
-
 // After the work enqueued on s: bytes (a multiple of 4) from device memory src
 // to dst, and the value of the device word err (null: 0 is returned). The
 // stream has drained when it returns.
@@ -227,7 +161,7 @@ unsigned copy_out(hipStream_t s, int device, void* dst, const void* src, size_t 
       if (err) launch_copy_out(s, nullptr, 0, err, word);
       fetch(0);
       if (team.count() > 1) fetch(1);
-      team.touch(0);
+      team.touch();
       for (size_t i = 0; i < team.count(); ++i) {
         HIPX(hipEventSynchronize(st->ev[i & 1]));
         team.copy(i);
