@@ -30,7 +30,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function", f"-I{os
 
 SOURCES = ["kernels.hip", "gemm_pair.hip", "attn_pair.hip", "decode_persistent.hip", "decode_persistent_inst_mini.hip",
            "decode_persistent_inst_small.hip", "decode_persistent_inst_medium.hip",
-           "decode_persistent_inst_large.hip", "rtg_runtime.cpp", "safetensors_reader.cpp",
+           "decode_persistent_inst_large.hip", "rtg_runtime.cpp", "device_memory.cpp", "safetensors_reader.cpp",
            "tokenizer.cpp", "sampling.hip", "bgemv.hip", "scratch.hip", "decode_tile.hip", "rows.hip"]
 
 

@@ -12,6 +12,7 @@
 #include "decode_persistent.h"
 #include "decode_persistent_kernel.h"
 #include "decode_tile.h"
+#include "device_memory.h"
 
 namespace rtg {
 namespace pk {
@@ -112,7 +113,7 @@ PersistentPlan* persistent_plan_create(const PersistentWeights& w) {
   // folded constants: per layer sq, cq [3d] and sf, cf [4d]; then sl, cl [V]
   const size_t per_layer = 2 * (size_t)(3 * d) + 2 * (size_t)(4 * d);
   const size_t fold_floats = per_layer * L + 2 * (size_t)V;
-  if (hipDeviceSynchronize() != hipSuccess || hipMalloc(&pl->fold, fold_floats * 4) != hipSuccess) return pl;
+  if (hipDeviceSynchronize() != hipSuccess || device_malloc(&pl->fold, fold_floats * 4) != hipSuccess) return pl;
   std::vector<pk::LayerPtrs> lp(L);
   for (int i = 0; i < L; ++i) {
     const PersistentLayer& s = w.layers[i];
@@ -128,10 +129,10 @@ PersistentPlan* persistent_plan_create(const PersistentWeights& w) {
   float* cl = sl + V;
   if (!ln_fold(w.wte, w.wtype, V, d, w.lnfw, w.lnfb, nullptr, sl, cl) || hipDeviceSynchronize() != hipSuccess)
     return pl;
-  if (hipMalloc(&pl->layers_dev, sizeof(pk::LayerPtrs) * L) != hipSuccess) return pl;
+  if (device_malloc(&pl->layers_dev, sizeof(pk::LayerPtrs) * L) != hipSuccess) return pl;
   if (hipMemcpy(pl->layers_dev, lp.data(), sizeof(pk::LayerPtrs) * L, hipMemcpyHostToDevice) != hipSuccess)
     return pl;
-  if (hipMalloc(&pl->zeros, 4096) != hipSuccess || hipMemset(pl->zeros, 0, 4096) != hipSuccess) return pl;
+  if (device_malloc(&pl->zeros, 4096) != hipSuccess || hipMemset(pl->zeros, 0, 4096) != hipSuccess) return pl;
   pk::Params& p = pl->base;
   p.dummy = pl->zeros;
   p.layers = pl->layers_dev;
@@ -189,8 +190,8 @@ PersistentState* persistent_state_create(PersistentPlan* pl, float* kcache, floa
   s->p = pl->base;
   pk::Params& p = s->p;
   const size_t words = (size_t)p.lw * p.L;
-  if (hipMalloc(&s->tags, words * 8) != hipSuccess || hipMalloc(&s->epoch, 256) != hipSuccess ||
-      hipMalloc(&s->err, 256) != hipSuccess || hipMalloc(&s->done, 256) != hipSuccess) {
+  if (device_malloc(&s->tags, words * 8) != hipSuccess || device_malloc(&s->epoch, 256) != hipSuccess ||
+      device_malloc(&s->err, 256) != hipSuccess || device_malloc(&s->done, 256) != hipSuccess) {
     persistent_state_destroy(s);
     return nullptr;
   }
@@ -212,7 +213,7 @@ PersistentState* persistent_state_create(PersistentPlan* pl, float* kcache, floa
   if (const char* tf = getenv("RTG_TRACE_FILE")) {
     // per-workgroup phase timestamps of the latest step, written on request
     const size_t tbytes = (size_t)pk::G * pk::TRACE_STRIDE * 8;
-    if (tf[0] && hipMalloc(&s->trace, tbytes) == hipSuccess && hipMemset(s->trace, 0, tbytes) == hipSuccess)
+    if (tf[0] && device_malloc(&s->trace, tbytes) == hipSuccess && hipMemset(s->trace, 0, tbytes) == hipSuccess)
       p.trace = s->trace;
   }
   p.kc = kcache;
@@ -227,7 +228,7 @@ PersistentState* persistent_state_create(PersistentPlan* pl, float* kcache, floa
   if (const TilePlan* tp = pl->tile) {
     // the tiled step shares the decode state (token, position, epoch, keys,
     // error word) and has its own exchange words; tag 0 never matches
-    if (hipMalloc(&s->ttags, tp->tag_words * 8) != hipSuccess ||
+    if (device_malloc(&s->ttags, tp->tag_words * 8) != hipSuccess ||
         hipMemset(s->ttags, 0, tp->tag_words * 8) != hipSuccess) {
       persistent_state_destroy(s);
       return nullptr;

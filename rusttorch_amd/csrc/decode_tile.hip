@@ -20,6 +20,7 @@
 
 #include "decode_tile.h"
 #include "decode_tile_kernel.h"
+#include "device_memory.h"
 
 namespace rtg {
 
@@ -130,7 +131,7 @@ TilePlan* tile_plan_create(const PersistentWeights& w) {
   const long per_layer4 = nq + np + nf + nm;  // float4
   const long fold_floats = (long)(3 * d) * (tk::GS + 1) + (long)(4 * d) * (tk::GS + 1);
   const size_t bytes = (size_t)per_layer4 * 16 * L + (size_t)fold_floats * 4 * L + (size_t)V * 4 + 4096;
-  if (hipDeviceSynchronize() != hipSuccess || hipMalloc(&tp->arena, bytes) != hipSuccess) {
+  if (hipDeviceSynchronize() != hipSuccess || device_malloc(&tp->arena, bytes) != hipSuccess) {
     tile_plan_destroy(tp);
     return nullptr;
   }
@@ -164,7 +165,7 @@ TilePlan* tile_plan_create(const PersistentWeights& w) {
   hipLaunchKernelGGL(tile_lm_const_kernel, dim3((V + 255) / 256), dim3(256), 0, 0, static_cast<const float*>(w.wte),
                      V, d, w.lnfb, cl);
   ok = ok && hipGetLastError() == hipSuccess && hipDeviceSynchronize() == hipSuccess;
-  if (ok) ok = hipMalloc(&tp->layers_dev, sizeof(tk::TLayer) * L) == hipSuccess;
+  if (ok) ok = device_malloc(&tp->layers_dev, sizeof(tk::TLayer) * L) == hipSuccess;
   if (ok) ok = hipMemcpy(tp->layers_dev, lay.data(), sizeof(tk::TLayer) * L, hipMemcpyHostToDevice) == hipSuccess;
   if (!ok) {
     tile_plan_destroy(tp);

@@ -8,6 +8,7 @@
 
 #include <vector>
 
+#include "device_memory.h"
 #include "kernels.h"
 #include "rows.h"
 #include "rows_kernel.h"
@@ -81,7 +82,7 @@ RowsPlan* rows_plan_create(const PersistentWeights& w, int cus) {
               static_cast<const float*>(s.wfc), static_cast<const float*>(s.wmproj), s.bqkv, s.baproj, s.bfc,
               s.bmproj, s.ln1w, s.ln1b, s.ln2w, s.ln2b};
   }
-  if (hipMalloc(&pl->layers_dev, sizeof(rk::RLayer) * pl->L) != hipSuccess ||
+  if (device_malloc(&pl->layers_dev, sizeof(rk::RLayer) * pl->L) != hipSuccess ||
       hipMemcpy(pl->layers_dev, lay.data(), sizeof(rk::RLayer) * pl->L, hipMemcpyHostToDevice) != hipSuccess) {
     rows_plan_destroy(pl);
     return nullptr;
@@ -121,7 +122,7 @@ unsigned* head_err(void* mem) { return reinterpret_cast<unsigned*>(static_cast<c
 
 RowsState* rows_state_create(const RowsPlan* p) {
   void* mem = nullptr;
-  if (hipMalloc(&mem, rows_state_bytes(p, true)) != hipSuccess) return nullptr;
+  if (device_malloc(&mem, rows_state_bytes(p, true)) != hipSuccess) return nullptr;
   const rk::u64 one = 1;
   if (hipMemset(mem, 0, kHead) != hipSuccess ||
       hipMemcpy(head_epoch(mem), &one, sizeof(one), hipMemcpyHostToDevice) != hipSuccess) {
@@ -150,7 +151,7 @@ rk::u64* trace_buf() {
   if (!tried) {
     tried = true;
     const char* f = getenv("RTG_ROWS_TRACE");
-    if (f && f[0] && hipMalloc(&buf, (size_t)rk::G * rk::TRACE_WORDS * 8) != hipSuccess) buf = nullptr;
+    if (f && f[0] && device_malloc(&buf, (size_t)rk::G * rk::TRACE_WORDS * 8) != hipSuccess) buf = nullptr;
   }
   return buf;
 }

@@ -10,11 +10,13 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/rtgpu.h"
@@ -22,6 +24,7 @@
 #include "attn_pair.h"
 #include "bgemv.h"
 #include "copy_team.h"
+#include "device_memory.h"
 #include "gemm_pair.h"
 #include "kernels.h"
 #include "rows.h"
@@ -226,6 +229,46 @@ struct PrefillWeights {
   }
 };
 
+// A model's PrefillWeights, as long as their memory is not needed for something
+// that cannot be done without: every allocation that fails takes them back
+// (device_memory.h) and the model's prefill runs the f32-MFMA GEMMs from then
+// on. A pass holds them while it is being enqueued; freeing them waits for the
+// device, and so for the passes enqueued.
+class PrefillHolder final : public SpareMemory {
+ public:
+  PrefillHolder() { register_spare(this); }
+  ~PrefillHolder() { unregister_spare(this); }
+  PrefillHolder(const PrefillHolder&) = delete;
+  PrefillHolder& operator=(const PrefillHolder&) = delete;
+  std::shared_ptr<const PrefillWeights> get() const {
+    std::lock_guard<std::mutex> g(mu_);
+    return pw_;
+  }
+  void set(std::unique_ptr<PrefillWeights> pw, int device) {
+    std::lock_guard<std::mutex> g(mu_);
+    pw_ = std::move(pw);
+    device_ = device;
+  }
+  bool give_back(int device) override {
+    std::weak_ptr<const PrefillWeights> left;
+    {
+      std::shared_ptr<const PrefillWeights> pw;
+      std::lock_guard<std::mutex> g(mu_);
+      if (!pw_ || device != device_) return false;
+      pw.swap(pw_);
+      left = pw;
+    }
+    // passes that are being enqueued on other threads (milliseconds) let go
+    for (int i = 0; i < 2000 && !left.expired(); ++i) std::this_thread::sleep_for(std::chrono::milliseconds(1));
+    return true;
+  }
+
+ private:
+  mutable std::mutex mu_;
+  std::shared_ptr<const PrefillWeights> pw_;
+  int device_ = -1;
+};
+
 struct rtg_model {
   rtg_config cfg;
   int hd = 0;
@@ -240,7 +283,7 @@ struct rtg_model {
   size_t nparams = 0;
   PersistentPlan* pplan = nullptr;
   RowsPlan* rplan = nullptr;  // multi-row forward (short prompts), null where unsupported
-  std::unique_ptr<PrefillWeights> pw;  // null where the f32-MFMA GEMMs run the prefill
+  PrefillHolder pw;           // empty where the f32-MFMA GEMMs run the prefill
   std::mutex bw_mu;
   std::unique_ptr<BatchedWeights> bw;
   // Pool of caches reused by the generate entry points (keyed by batch).
@@ -329,7 +372,7 @@ static void ensure_ws(rtg_cache* c, size_t cap, bool pair) {
   if (c->ws) hipFree(c->ws);
   c->ws = nullptr;
   c->ws_floats = 0;
-  HIPX(hipMalloc(&c->ws, ws * 4));
+  HIPX(device_malloc(&c->ws, ws * 4));
   c->ws_floats = ws;
 }
 
@@ -339,12 +382,12 @@ static void ensure_rows(rtg_cache* c, size_t rows) {
   free_work(c);
   const size_t d = c->m->cfg.n_embd;
   size_t cap = std::max<size_t>(rows, 16);
-  HIPX(hipMalloc(&c->x, cap * d * 4));
-  HIPX(hipMalloc(&c->ln, cap * d * 4));
-  HIPX(hipMalloc(&c->qkv, cap * 3 * d * 4));
-  HIPX(hipMalloc(&c->att, cap * d * 4));
-  HIPX(hipMalloc(&c->h, cap * 4 * d * 4));
-  ensure_ws(c, cap, c->m->pw != nullptr);
+  HIPX(device_malloc(&c->x, cap * d * 4));
+  HIPX(device_malloc(&c->ln, cap * d * 4));
+  HIPX(device_malloc(&c->qkv, cap * 3 * d * 4));
+  HIPX(device_malloc(&c->att, cap * d * 4));
+  HIPX(device_malloc(&c->h, cap * 4 * d * 4));
+  ensure_ws(c, cap, c->m->pw.get() != nullptr);
   c->rows_cap = cap;
 }
 
@@ -356,12 +399,12 @@ static void ensure_logits(rtg_cache* c, size_t rows) {
   if (c->logits) hipFree(c->logits);
   c->logits = nullptr;
   size_t cap = std::max<size_t>(rows, 16);
-  HIPX(hipMalloc(&c->logits, cap * c->m->cfg.vocab_size * 4));
+  HIPX(device_malloc(&c->logits, cap * c->m->cfg.vocab_size * 4));
   c->logit_rows_cap = cap;
 }
 
 static void ensure_sample_work(rtg_cache* c) {
-  if (!c->sample_work) HIPX(hipMalloc(&c->sample_work, sample_work_bytes((int)c->m->cfg.vocab_size)));
+  if (!c->sample_work) HIPX(device_malloc(&c->sample_work, sample_work_bytes((int)c->m->cfg.vocab_size)));
 }
 
 static rtg_cache* cache_create(const rtg_model* m, size_t batch) {
@@ -372,14 +415,14 @@ static rtg_cache* cache_create(const rtg_model* m, size_t batch) {
   c->layer_stride = batch * H * P * hd;
   try {
     HIPX(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    HIPX(hipMalloc(&c->k, std::max<size_t>(L * c->layer_stride, 1) * 4));
-    HIPX(hipMalloc(&c->v, std::max<size_t>(L * c->layer_stride, 1) * 4));
-    HIPX(hipMalloc(&c->pos_dev, 256));
-    HIPX(hipMalloc(&c->step_dev, 256));
-    HIPX(hipMalloc(&c->keys, std::max<size_t>(batch, 1) * 8));
-    HIPX(hipMalloc(&c->token_dev, std::max<size_t>(batch, 1) * 4));
-    HIPX(hipMalloc(&c->ids_dev, std::max<size_t>(batch * P, 1) * 4));
-    HIPX(hipMalloc(&c->ids_in, std::max<size_t>(batch * P, 1) * 4));
+    HIPX(device_malloc(&c->k, std::max<size_t>(L * c->layer_stride, 1) * 4));
+    HIPX(device_malloc(&c->v, std::max<size_t>(L * c->layer_stride, 1) * 4));
+    HIPX(device_malloc(&c->pos_dev, 256));
+    HIPX(device_malloc(&c->step_dev, 256));
+    HIPX(device_malloc(&c->keys, std::max<size_t>(batch, 1) * 8));
+    HIPX(device_malloc(&c->token_dev, std::max<size_t>(batch, 1) * 4));
+    HIPX(device_malloc(&c->ids_dev, std::max<size_t>(batch * P, 1) * 4));
+    HIPX(device_malloc(&c->ids_in, std::max<size_t>(batch * P, 1) * 4));
     for (auto& e : c->ev) HIPX(hipEventCreate(&e));
     HIPX(hipMemsetAsync(c->pos_dev, 0, 256, c->stream));
     HIPX(hipMemsetAsync(c->step_dev, 0, 256, c->stream));
@@ -435,10 +478,9 @@ enum LogitRows { LOGITS_ALL, LOGITS_LAST, LOGITS_NONE };
 // forward_cached body for S sequences x T new tokens (gpt2.rs:376-396) on the
 // pair GEMMs (gemm_pair.h): w.ln, w.att and w.h hold f16 pairs, 4 bytes per
 // element like the f32 rows they replace.
-static void enqueue_prefill_pair(rtg_cache* c, const Work& w, const uint32_t* ids_dev, size_t S, size_t T, size_t past,
-                                 LogitRows logit_rows) {
+static void enqueue_prefill_pair(rtg_cache* c, const PrefillWeights& pw, const Work& w, const uint32_t* ids_dev,
+                                 size_t S, size_t T, size_t past, LogitRows logit_rows) {
   const rtg_model* m = c->m;
-  const PrefillWeights& pw = *m->pw;
   const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, M = (int)(S * T);
   const float eps = m->cfg.layer_norm_epsilon;
   hipStream_t s = c->stream;
@@ -504,7 +546,8 @@ static void enqueue_prefill_pair(rtg_cache* c, const Work& w, const uint32_t* id
 static void enqueue_prefill(rtg_cache* c, const Work& w, const uint32_t* ids_dev, size_t S, size_t T, size_t past,
                             LogitRows logit_rows, bool for_draws = false) {
   const rtg_model* m = c->m;
-  if (m->pw && !for_draws) return enqueue_prefill_pair(c, w, ids_dev, S, T, past, logit_rows);
+  if (!for_draws)
+    if (const auto pw = m->pw.get()) return enqueue_prefill_pair(c, *pw, w, ids_dev, S, T, past, logit_rows);
   const int d = (int)m->cfg.n_embd, V = (int)m->cfg.vocab_size, M = (int)(S * T);
   const float eps = m->cfg.layer_norm_epsilon;
   hipStream_t s = c->stream;
@@ -558,7 +601,7 @@ static const BatchedWeights* ensure_batched(const rtg_model* mc) {
   const size_t fold_layer = (size_t)(2 * 3 * d + 2 * 4 * d) * 4;
   const size_t total = per_layer * L + align_up(tl, 256) + align_up(fold_layer, 256) * L + align_up((size_t)2 * V * 4, 256);
   HIPX(hipDeviceSynchronize());
-  HIPX(hipMalloc(&bw->arena, total));
+  HIPX(device_malloc(&bw->arena, total));
   char* p = static_cast<char*>(bw->arena);
   auto take = [&](size_t n) {
     char* r = p;
@@ -612,10 +655,10 @@ static void ensure_bg_work(rtg_cache* c, const BatchedWeights* bw) {
     part = std::max(part, bgemv_work_floats(*pl, (int)c->batch));
     groups = std::max(groups, (size_t)pl->groups);
   }
-  HIPX(hipMalloc(&c->bg_part, part * 4));
-  HIPX(hipMalloc(&c->bg_cnt, groups * 4));
-  HIPX(hipMalloc(&c->bg_spart, groups * kBgemvRows * 2 * 4));
-  HIPX(hipMalloc(&c->bg_cen, 2 * kBgemvRows * 4));
+  HIPX(device_malloc(&c->bg_part, part * 4));
+  HIPX(device_malloc(&c->bg_cnt, groups * 4));
+  HIPX(device_malloc(&c->bg_spart, groups * kBgemvRows * 2 * 4));
+  HIPX(device_malloc(&c->bg_cen, 2 * kBgemvRows * 4));
   HIPX(hipMemsetAsync(c->bg_cnt, 0, groups * 4, c->stream));
   HIPX(hipStreamSynchronize(c->stream));
 }
@@ -1151,7 +1194,7 @@ static void build_prefill_weights(rtg_model* m, std::unique_ptr<PrefillWeights> 
   int flag = 0;
   HIPX(hipGetLastError());
   HIPX(hipMemcpy(&flag, bad, 4, hipMemcpyDeviceToHost));
-  if (flag == 0) m->pw = std::move(pw);
+  if (flag == 0) m->pw.set(std::move(pw), m->device);
 }
 
 namespace {
@@ -1254,7 +1297,7 @@ rtg_result build_model(const rtg_config* cfg, Lookup& lk, rtg_storage storage, r
   bool own_staging = false;
   std::unique_ptr<PrefillWeights> pw;
   try {
-    HIPX(hipMalloc(&m->arena, cur));
+    HIPX(device_malloc(&m->arena, cur));
     m->arena_bytes = cur;
     char* A = reinterpret_cast<char*>(m->arena);
     // (uploads pass through the memory of the prefill weights, which are made
@@ -1266,7 +1309,7 @@ rtg_result build_model(const rtg_config* cfg, Lookup& lk, rtg_storage storage, r
       if (hipMalloc(&staging, stage_max) != hipSuccess) {
         (void)hipGetLastError();
         pw.reset();  // the load needs the staging, the prefill can do without its copy
-        HIPX(hipMalloc(&staging, stage_max));
+        HIPX(device_malloc(&staging, stage_max));
       }
     } else staging = static_cast<float*>(pw->arena);
     hipStream_t s = nullptr;
@@ -1581,7 +1624,7 @@ rtg_result rtg_forward_cached_noalloc(const rtg_model* model, rtg_cache* cache, 
   const size_t pv = align_up(n * V, 64);
   // the split-k partial tiles the pass's GEMMs use at n rows (as much as the
   // cache's own workspace would hold for them, so the same kernels run)
-  size_t pw = prefill_ws_floats(model, n, model->pw != nullptr);
+  size_t pw = prefill_ws_floats(model, n, model->pw.get() != nullptr);
   pw = align_up(pw, 64);
   const size_t need = 3 * pd + p3 + p4 + pv;
   if (need > kScratchFloats)
@@ -1733,8 +1776,8 @@ rtg_result rtg_generate(const rtg_model* model, const uint32_t* prompt, size_t n
     PoolLease lease(model, 1);
     rtg_cache* c = lease.c;
     hipStream_t s = c->stream;
-    HIPX(hipMalloc(&toks, total * 4));
-    HIPX(hipMalloc(&steps, max_new * 4));
+    HIPX(device_malloc(&toks, total * 4));
+    HIPX(device_malloc(&steps, max_new * 4));
     std::vector<int> step_no(max_new);
     for (size_t i = 0; i < max_new; ++i) step_no[i] = (int)(i + 1);  // the sampler's generation index + 1
     HIPX(hipMemcpyAsync(toks, prompt, n * 4, hipMemcpyHostToDevice, s));
