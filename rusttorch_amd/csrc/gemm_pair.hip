@@ -14,7 +14,7 @@
 // reaches on this card (8192^3: 1.09); the f32-MFMA kernel it replaced ran at
 // 126 (157 peak) and was further from 64 bits (6.6e-7 against 3.9e-7 relative
 // at K = 1280, 1.24e-6 against 8.0e-7 at 5120). At a few hundred rows the
-// launch, the first loads and the chain of k-tiles bound it (choose() below).
+// launch, the first loads and the chain of k-tiles bound it (gemm_pair_choice.h).
 //
 // A workgroup computes BM x BN outputs from k-tiles of 32: LDS rows of 128
 // bytes [32 hi][32 lo] (64 bytes for one-plane weights), filled by LDS-direct
@@ -31,6 +31,7 @@
 
 #include "f16_pair.h"
 #include "gelu.h"
+#include "gemm_pair_choice.h"
 
 namespace rtg {
 
@@ -442,67 +443,7 @@ __global__ __launch_bounds__(256) void pair_reduce_kernel(const float* __restric
   }
 }
 
-// The tiles, and their times per k-tile of 32 with two planes (us): alone on a
-// CU, and per workgroup where a CU has several to run. Fitted to a sweep of
-// every tile and split over the GPT-2 widths' GEMMs at 48 to 16368 rows: the
-// choice below is within 2% of each shape's fastest in the mean, 8-28% at
-// worst (333 x 3072 x 768: 17.3 against 13.5 us).
-// What each is for (us, f32 weights, M x N x K, tile against the next best):
-//   256 x 256: 16368 x 5120 x 1280: 567 (378 TFLOP/s) against 642
-//   128 x 128, two per CU: 16368 x 1280 x 5120: 630 against 702
-//   128 x 128 on 8 waves: 701 x 4096 x 1024: 28.2 against 31.9
-//   64 x 128: 3000 x 1280 x 1280: 40.0, 701 x 3072 x 1024: 27.6 against 30.0
-//   64 x 64: 333 x 3072 x 768: 13.5 against 17.3
-//   32 x 64: 77 x 5120 x 1280: 14.3 against 16.4
-// (f32-MFMA kernels before: 16368 x 5120 x 1280 1704-1926 us, 701 x 4096 x
-// 1024 74, 77 x 5120 x 1280 49.)
-struct TileTime {
-  int bm, bn;
-  float alone, shared;
-};
-constexpr TileTime kTiles[] = {
-    {256, 256, 2.30f, 2.60f},  // 0: 8 waves of 128 x 64, 2 stages
-    {128, 128, 1.00f, 0.72f},  // 1: 4 waves of 64 x 64, 2 stages, two workgroups per CU
-    {128, 128, 0.69f, 0.78f},  // 2: 8 waves of 64 x 32, 3 stages
-    {64, 128, 0.40f, 0.44f},   // 3: 4 waves of 64 x 32, 3 stages
-    {64, 64, 0.28f, 0.27f},    // 4: 8 waves of 32 x 32 (KW = 2), 4 stages
-    {32, 64, 0.20f, 0.20f},    // 5: 4 waves of 32 x 32 (KW = 2), 6 stages
-};
-constexpr int kSplitMaxRows = 2048;                   // more rows fill the GPU without a split
-constexpr size_t kSplitMaxFloats = (size_t)16 << 20;  // and no larger workspace than this
-
 constexpr int kGroupRows = 8;  // row blocks per group of the block order (4 and 16 measured the same)
-
-struct Choice {
-  int tile, ks;
-};
-
-// Tile and k split with the least estimated time: the k-tiles of a workgroup
-// times the time of one with the workgroups its CU holds, over 256 CUs, plus
-// the split's reduction (a launch, and its partials' way through memory).
-// Depends on M through its blocks of 32 rows only.
-Choice choose(int M, int N, int K, int planes, size_t ws_floats) {
-  const int mr = (M + 31) / 32 * 32, nk = K / 32;
-  Choice best{5, 1};
-  float least = 1e30f;
-  for (int c = 0; c < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++c) {
-    const TileTime& t = kTiles[c];
-    const long tiles = (long)((mr + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-    for (int ks = 1; ks <= 10; ++ks) {
-      const size_t floats = (size_t)ks * mr * N;
-      if (nk % ks != 0) continue;
-      if (ks > 1 && (mr > kSplitMaxRows || floats > kSplitMaxFloats || (size_t)ks * M * N > ws_floats)) break;
-      const long per_cu = (tiles * ks + 255) / 256;
-      const float step = (planes == 2 ? 1.f : 0.7f) * std::max(t.alone, per_cu * t.shared);
-      const float us = nk / ks * step + (ks > 1 ? 2.f + floats * 4 / 3.6e6f : 0.f);
-      if (us < least) {
-        least = us;
-        best = {c, ks};
-      }
-    }
-  }
-  return best;
-}
 
 template <int PW, int WM, int WN, int MI, int NJ, int NS, int KW = 1, bool DUAL = false>
 void launch_tile(hipStream_t s, const PairWeights& w, const PairGemmArgs& a, int ks) {
@@ -519,7 +460,7 @@ void launch_tile(hipStream_t s, const PairWeights& w, const PairGemmArgs& a, int
 
 template <int PW>
 void launch_planes(hipStream_t s, const PairWeights& w, const PairGemmArgs& a) {
-  const Choice c = choose(a.M, w.N, w.K, PW, a.ws ? a.ws_floats : 0);
+  const PairChoice c = pair_choose(a.M, w.N, w.K, PW, a.ws ? a.ws_floats : 0);
   switch (c.tile) {
     case 0: launch_tile<PW, 2, 4, 4, 2, 2>(s, w, a, c.ks); break;
     case 1: launch_tile<PW, 2, 2, 2, 2, 2>(s, w, a, c.ks); break;
@@ -548,7 +489,7 @@ void launch_pair_weights(hipStream_t s, const void* W, int wtype, const float* i
 }
 
 size_t pair_gemm_ws_floats(int M, int N, int K, int planes) {
-  const int ks = choose(M, N, K, planes, kSplitMaxFloats).ks;
+  const int ks = pair_choose(M, N, K, planes, kSplitMaxFloats).ks;
   return ks > 1 ? (size_t)ks * M * N : 0;
 }
 

@@ -6,9 +6,9 @@ ids (f32 throughout, sums in k order): the library may be at most twice as far
 in the 2-norm, plus 2e-7 (3 ulp of f32) where the oracle happens to be closer.
 bf16 storage is compared on weights that are bf16 values already.
 
-Shapes: one layer, chosen so that every tile of the dispatch and the k split
-occur (short and long M against wide and narrow N), with ragged M and V and
-head dims 64 and 32; a second chunk behind cached rows; widths above 2048
+Shapes: one layer, chosen so that every tile of the dispatch occurs with and
+without a k split for both kinds of weights (tests/test_pair_choice.py checks
+that on the CPU), with ragged M and V and head dims 64 and 32; a second chunk behind cached rows; widths above 2048
 (the block-per-row LayerNorm); weights and gains whose magnitudes spread over
 many powers of two; and weights for which the path is not taken at all.
 """
@@ -53,8 +53,8 @@ def check(oracle_lib, sh, sd, m, chunks, batch=1):
     c.close()
 
 
-@pytest.mark.parametrize("storage", ["f32", "bf16"])
-@pytest.mark.parametrize("d,heads,V,batch,chunks", [
+# width, heads, vocabulary, batch, chunks
+SHAPES = [
     (192, 3, 301, 1, (33,)),          # 32 x 64 tiles, split
     (192, 6, 301, 3, (17,)),          # head_dim 32, 51 rows
     (192, 3, 301, 5, (131, 7)),       # 655 rows, then 35 behind 131 cached
@@ -63,9 +63,24 @@ def check(oracle_lib, sh, sd, m, chunks, batch=1):
     (768, 12, 515, 1, (65,)),
     (768, 12, 515, 2, (161,)),
     (768, 12, 515, 9, (129,)),        # 64 x 64 and 64 x 128 tiles
-    (1600, 25, 258, 16, (65,)),       # 128 x 128 tiles, K = 6400 split
-    (128, 2, 50257, 1, (999,)),       # a wide LM head over many rows: 256 x 256 tiles
-])
+    (768, 12, 515, 10, (65,)),        # 128 x 128 tiles of 8 waves
+    (1024, 16, 258, 1, (40,)),        # 64 x 64 tiles, split
+    (1024, 16, 258, 16, (65,)),       # 128 x 128 tiles, split
+    (1280, 20, 258, 1, (40,)),        # 64 x 128 tiles, split
+    (1600, 25, 258, 1, (40,)),
+    (1600, 25, 258, 3, (65,)),        # 128 x 128 tiles of 8 waves, split
+    (1600, 25, 258, 16, (65,)),       # K = 6400 split
+    (1600, 25, 258, 22, (65,)),       # 256 x 256 tiles, split
+    (128, 2, 50257, 1, (40,)),        # a wide LM head: 64 x 128 tiles,
+    (128, 2, 50257, 1, (70,)),        #   128 x 128 tiles of 4 waves,
+    (128, 2, 50257, 1, (200,)),       #   256 x 256 tiles,
+    (128, 2, 50257, 1, (999,)),       #   and over many rows
+]
+MANY_ROWS = (640, 10, 130, 32, (403,))
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+@pytest.mark.parametrize("d,heads,V,batch,chunks", SHAPES)
 def test_shapes(oracle_lib, storage, d, heads, V, batch, chunks):
     sh = synth.ModelShape(V, 1024, d, 1, heads)
     sd, m = build(sh, storage)
@@ -73,11 +88,13 @@ def test_shapes(oracle_lib, storage, d, heads, V, batch, chunks):
     m.close()
 
 
-def test_many_rows(oracle_lib):
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+def test_many_rows(oracle_lib, storage):
     """Enough rows that the layer GEMMs take the 256 x 256 and 128 x 128 tiles."""
-    sh = synth.ModelShape(130, 512, 640, 1, 10)
-    sd, m = build(sh)
-    check(oracle_lib, sh, sd, m, (403,), batch=32)
+    d, heads, V, batch, chunks = MANY_ROWS
+    sh = synth.ModelShape(V, 512, d, 1, heads)
+    sd, m = build(sh, storage)
+    check(oracle_lib, sh, sd, m, chunks, batch=batch)
     m.close()
 
 
@@ -103,6 +120,24 @@ def test_spread_magnitudes(oracle_lib):
     sh = synth.ModelShape(301, 256, 192, 1, 3)
     sd, m = build(sh, change=change)
     check(oracle_lib, sh, sd, m, (77, 120))
+    m.close()
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+@pytest.mark.parametrize("d,heads,batch,chunks", [
+    (192, 3, 1, (40, 30)),       # at most 64 rows, split; 30 behind 40 cached
+    (192, 6, 3, (27,)),          # head_dim 32, 81 rows
+    (192, 3, 1, (520, 90)),      # 64 x 128 tiles, keys over 8 waves
+    (768, 12, 9, (129,)),        # 128 x 128 tiles, split
+    (192, 3, 90, (33, 34)),      # more than 1024 rows; 64 and 32 queries per attention workgroup
+    (640, 10, 32, (403,)),       # 128 queries per attention workgroup
+])
+def test_f32_kernels(oracle_lib, storage, d, heads, batch, chunks):
+    """The f32-MFMA prefill, which drawn prompts and models without the pair
+    copy run: a negative epsilon keeps a model off the pair GEMMs."""
+    sh = synth.ModelShape(301, 1024, d, 1, heads, -1e-9)
+    sd, m = build(sh, storage)
+    check(oracle_lib, sh, sd, m, chunks, batch)
     m.close()
 
 
