@@ -5,16 +5,18 @@
 
 namespace rtg {
 
-// Power-of-two scales (gemm_pair.h: values times their scale are at most 2^15):
-// of q and k per head, of v per column; v's are also the output's.
+// Power-of-two scales (gemm_pair.h: values times their scale are at most 2^15)
+// per column; v's are also the output's. The products of a head's q and k
+// scales are the same in all of its columns: qk[h], between 2^-100 and 2^110.
 struct AttnScales {
-  const float* q;
-  const float* k;
-  const float* v;
+  const float* q;   // [d]: c_attn's own
+  const float* k;   // [d]
+  const float* qk;  // [H]
+  const float* v;   // [d]: c_attn's own
 };
-// q[h], k[h] from the scales col[2 d] of c_attn's q and k columns, their product
-// between 2^-100 and 2^110; *bad is set nonzero where it would be smaller.
-void launch_head_scale(hipStream_t s, const float* col, int H, float* q, float* k, int* bad);
+// k and qk from the scales col[2 d] of c_attn's q and k columns; *bad is set
+// nonzero where a qk would be below 2^-100.
+void launch_head_scale(hipStream_t s, const float* col, int H, float* k, float* qk, int* bad);
 
 // S sequences of T new tokens at offset past: qkv rows [S * T][3 d] (q columns
 // read), the cache of positions [0, past + T); out: pair matrix [S * T][d]

@@ -12,8 +12,9 @@
 // e % 4, are the lane's own accumulators 8 t .. 8 t + 7: P feeds the MFMA from
 // registers. The running maximum, the sums and O are f32.
 //
-// Operands: q and k scaled per head, v per column (the scales of c_attn's
-// outputs, fixed when the model is loaded), P by 2^14; V's scale is the
+// Operands: q, k and v scaled per column (the scales of c_attn's outputs, fixed
+// when the model is loaded; a head's k scales such that the product with q's is
+// the same in every column), P by 2^14; V's scale is the
 // attention output's own, so O / (2^14 l) is the pair GEMM's input as it is.
 // K and V are read from the f32 cache and split while a block is staged in LDS:
 // K rows of 64 hi + 64 lo (256 bytes), V^T rows (one per dim) of 32 hi + 32 lo
@@ -73,7 +74,7 @@ struct Stage {
       }
     }
   }
-  __device__ __forceinline__ void store(char* Ks, char* Vt, float ak, const float4& av, int tid) const {
+  __device__ __forceinline__ void store(char* Ks, char* Vt, const float4& ak, const float4& av, int tid) const {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int e = tid + u * NT, key = 2 * (e >> 4), d4 = (e & 15) * 4;
@@ -81,8 +82,8 @@ struct Stage {
       for (int r = 0; r < 2; ++r) {
         const int row = key + r;
         uint2 h, l;
-        split2(k[u][r].x * ak, k[u][r].y * ak, &h.x, &l.x);
-        split2(k[u][r].z * ak, k[u][r].w * ak, &h.y, &l.y);
+        split2(k[u][r].x * ak.x, k[u][r].y * ak.y, &h.x, &l.x);
+        split2(k[u][r].z * ak.z, k[u][r].w * ak.w, &h.y, &l.y);
         char* p = Ks + row * 256 + (d4 & 4) * 2;
         *reinterpret_cast<uint2*>(p + (((d4 >> 3) ^ (row & 15)) << 4)) = h;
         *reinterpret_cast<uint2*>(p + (((8 + (d4 >> 3)) ^ (row & 15)) << 4)) = l;
@@ -109,16 +110,18 @@ struct State {
   f16x8 qh[4], ql[4];
   floatx16 o0, o1;
   float m, l;
-  __device__ __forceinline__ void init(const float* qrow, float aq, int hh) {
+  __device__ __forceinline__ void init(const float* qrow, const float* aq, int hh) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const float4 a = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * hh);
       const float4 b = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * hh + 4);
+      const float4 sa = *reinterpret_cast<const float4*>(aq + 16 * s + 8 * hh);
+      const float4 sb = *reinterpret_cast<const float4*>(aq + 16 * s + 8 * hh + 4);
       unsigned h[4], l4[4];
-      split2(a.x * aq, a.y * aq, &h[0], &l4[0]);
-      split2(a.z * aq, a.w * aq, &h[1], &l4[1]);
-      split2(b.x * aq, b.y * aq, &h[2], &l4[2]);
-      split2(b.z * aq, b.w * aq, &h[3], &l4[3]);
+      split2(a.x * sa.x, a.y * sa.y, &h[0], &l4[0]);
+      split2(a.z * sa.z, a.w * sa.w, &h[1], &l4[1]);
+      split2(b.x * sb.x, b.y * sb.y, &h[2], &l4[2]);
+      split2(b.z * sb.z, b.w * sb.w, &h[3], &l4[3]);
       qh[s] = __builtin_bit_cast(f16x8, make_uint4(h[0], h[1], h[2], h[3]));
       ql[s] = __builtin_bit_cast(f16x8, make_uint4(l4[0], l4[1], l4[2], l4[3]));
     }
@@ -192,9 +195,7 @@ struct State {
 
 // score = (K . Q) / 8 (1 / sqrt(64)), in units of log2 e, of the scaled operands;
 // finite and not zero (head_scale_kernel), so that a masked score stays -inf
-__device__ __forceinline__ float score_factor(float aq, float ak) {
-  return 0.125f * 1.4426950408889634f / (aq * ak);
-}
+__device__ __forceinline__ float score_factor(float qk) { return 0.125f * 1.4426950408889634f / qk; }
 
 // FW waves, each with its own 32 queries of one (sequence, head), over the
 // same key blocks: the next block's rows are loaded while this one is used.
@@ -215,9 +216,9 @@ __global__ __launch_bounds__(64 * FW, 2) void attn_pair_kernel(const float* __re
   const int qpos = past + qi;
   const size_t head_off = ((size_t)sidx * H + h) * (size_t)P * 64;
   const float *Kh = kc + head_off, *Vh = vc + head_off;
-  const float aq = sc.q[h], ak = sc.k[h];
+  const float4 ak = *reinterpret_cast<const float4*>(sc.k + h * 64 + (tid & 15) * 4);
   const float4 av = *reinterpret_cast<const float4*>(sc.v + h * 64 + (tid & 15) * 4);
-  const float fac = score_factor(aq, ak);
+  const float fac = score_factor(sc.qk[h]);
   const int kmax = past + min(T, (qb + 1) * AP_Q * FW) - 1;  // last key any query here attends
   const int nkb = kmax / AP_K + 1;
   // (a wave past its own last key block only stages: its queries are earlier)
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(64 * FW, 2) void attn_pair_kernel(const float* __re
   Stage<NT, U> st;
   st.load(Kh, Vh, 0, kmax, tid);
   State q;
-  q.init(qkv + ((size_t)sidx * T + min(qi, T - 1)) * 3 * d + h * 64, aq, hh);
+  q.init(qkv + ((size_t)sidx * T + min(qi, T - 1)) * 3 * d + h * 64, sc.q + h * 64, hh);
   for (int kb = 0; kb < nkb; ++kb) {
     __syncthreads();  // every wave is done with the previous block
     st.store(Ks, Vt, ak, av, tid);
@@ -268,15 +269,15 @@ __global__ __launch_bounds__(64 * KS, 2) void attn_pair_ks_kernel(const float* _
   const size_t head_off = ((size_t)sidx * H + h) * (size_t)P * 64;
   const float *Kh = kc + head_off, *Vh = vc + head_off;
   char *Ks = sm[wave], *Vt = sm[wave] + AP_KB;
-  const float aq = sc.q[h], ak = sc.k[h];
+  const float4 ak = *reinterpret_cast<const float4*>(sc.k + h * 64 + (lane & 15) * 4);
   const float4 av = *reinterpret_cast<const float4*>(sc.v + h * 64 + (lane & 15) * 4);
-  const float fac = score_factor(aq, ak);
+  const float fac = score_factor(sc.qk[h]);
   const int kmax = past + min(T, (qb + 1) * AP_Q) - 1;
   const int nkb = kmax / AP_K + 1;
   Stage<64, 4> st;
   if (wave < nkb) st.load(Kh, Vh, wave, kmax, lane);
   State q;
-  q.init(qkv + ((size_t)sidx * T + min(qi, T - 1)) * 3 * d + h * 64, aq, hh);
+  q.init(qkv + ((size_t)sidx * T + min(qi, T - 1)) * 3 * d + h * 64, sc.q + h * 64, hh);
   for (int kb = wave; kb < nkb; kb += KS) {
     // this wave's region only: LDS accesses of one wave are ordered, the
     // wave's previous reads are complete before its writes below
@@ -330,32 +331,33 @@ __global__ __launch_bounds__(64 * KS, 2) void attn_pair_ks_kernel(const float* _
   }
 }
 
-// A head's scales: the smallest of its 64 columns, for q and for k. Each may be
-// up to 2^80; where their product exceeds 2^110 the head's scores are below
-// 2^-77 (64 products of 2^30 over 2^110, over 8), the softmax is uniform
-// whatever they are, and a smaller q scale keeps the score factor from becoming
-// 0, whose product with a masked score is NaN. A product below 2^-100 (scores
-// that may pass f32's range) is left to the f32 attention.
-__global__ __launch_bounds__(64) void head_scale_kernel(const float* __restrict__ col, int H, float* __restrict__ q,
-                                                        float* __restrict__ k, int* bad) {
-  const int h = blockIdx.x;
-  float a = col[h * 64 + threadIdx.x], b = col[(H + h) * 64 + threadIdx.x];
+// A head's k scales and the product qk: the smallest product of a column's q
+// and k scales. A column's k scale is then qk over its q scale, at most its own;
+// what a column of smaller products loses by that is as far below the head's
+// scores as f32's own rounding of them. (One scale for a head's q and one for
+// its k lost 2^-15 of every column beside one that is 2^20 larger.)
+// Above 2^110 the head's scores are below 2^-77 (64 products of 2^30 over 2^110,
+// over 8) and the softmax is uniform whatever they are; a smaller qk keeps the
+// score factor from becoming 0, whose product with a masked score is NaN. A
+// product below 2^-100 (scores that may pass f32's range) is left to the f32
+// attention.
+__global__ __launch_bounds__(64) void head_scale_kernel(const float* __restrict__ col, int H, float* __restrict__ k,
+                                                        float* __restrict__ qk, int* bad) {
+  const int h = blockIdx.x, c = h * 64 + threadIdx.x;
+  const int eq = ilogbf(col[c]), e = eq + ilogbf(col[H * 64 + c]);
+  int least = e;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    a = fminf(a, __shfl_xor(a, o, 64));
-    b = fminf(b, __shfl_xor(b, o, 64));
-  }
-  if (threadIdx.x != 0) return;
-  const int e = ilogbf(a) + ilogbf(b);
-  if (e < -100) *bad = 1;
-  q[h] = ldexpf(a, min(110 - e, 0));
-  k[h] = b;
+  for (int o = 32; o > 0; o >>= 1) least = min(least, __shfl_xor(least, o, 64));
+  if (least < -100) *bad = 1;
+  least = min(least, 110);
+  k[c] = ldexpf(1.f, least - eq);
+  if (threadIdx.x == 0) qk[h] = ldexpf(1.f, least);
 }
 
 }  // namespace
 
-void launch_head_scale(hipStream_t s, const float* col, int H, float* q, float* k, int* bad) {
-  head_scale_kernel<<<H, 64, 0, s>>>(col, H, q, k, bad);
+void launch_head_scale(hipStream_t s, const float* col, int H, float* k, float* qk, int* bad) {
+  head_scale_kernel<<<H, 64, 0, s>>>(col, H, k, qk, bad);
 }
 
 void launch_attn_pair(hipStream_t s, const float* qkv, int S, int T, int past, const float* kc, const float* vc,

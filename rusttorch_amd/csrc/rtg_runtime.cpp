@@ -1133,7 +1133,7 @@ static std::unique_ptr<PrefillWeights> alloc_prefill_weights(const rtg_model* m)
   size_t total = 256;  // the flag
   for (const Shape& x : sh) total += L * (align_up(pair_weight_bytes(x.N, x.K, wt), 256) + align_up(x.N * 4, 256));
   const int H = (int)m->cfg.n_head;
-  total += L * (2 * align_up(d * 4, 256) + align_up(3 * d * 4, 256) + align_up(4 * d * 4, 256) + align_up(2 * H * 4, 256));
+  total += L * (3 * align_up(d * 4, 256) + align_up(3 * d * 4, 256) + align_up(4 * d * 4, 256) + align_up(H * 4, 256));
   total += align_up(pair_weight_bytes(V, d, wt), 256) + align_up((size_t)V * 4, 256) + align_up(d * 4, 256);
   if (hipMalloc(&pw->arena, total) != hipSuccess) {
     (void)hipGetLastError();
@@ -1170,13 +1170,14 @@ static void build_prefill_weights(rtg_model* m, std::unique_ptr<PrefillWeights> 
   };
   for (const LayerW& W : m->layers) {
     PrefillWeights::Layer l;
-    float *s1 = floats(d), *sqkv = floats(3 * d), *s2 = floats(d), *sh4 = floats(4 * d), *heads = floats(2 * H);
+    float *s1 = floats(d), *sqkv = floats(3 * d), *s2 = floats(d), *sh4 = floats(4 * d), *sk = floats(d),
+          *qk = floats(H);
     launch_pair_ln_scale(s, W.ln1w, W.ln1b, d, s1, bad);
     launch_pair_ln_scale(s, W.ln2w, W.ln2b, d, s2, bad);
     // attention averages value rows, so its output has the bound of c_attn's v
     launch_pair_row_scale(s, W.wqkv, wt, 3 * d, d, W.ln1w, W.ln1b, W.bqkv, sqkv, bad);
-    if (m->hd == 64) launch_head_scale(s, sqkv, H, heads, heads + H, bad);
-    l.att = AttnScales{heads, heads + H, sqkv + 2 * d};
+    if (m->hd == 64) launch_head_scale(s, sqkv, H, sk, qk, bad);
+    l.att = AttnScales{sqkv, sk, qk, sqkv + 2 * d};
     launch_pair_row_scale(s, W.wfc, wt, 4 * d, d, W.ln2w, W.ln2b, W.bfc, sh4, bad);
     l.s1 = s1;
     l.s2 = s2;

@@ -142,13 +142,21 @@ def test_f32_kernels(oracle_lib, storage, d, heads, batch, chunks):
 
 
 @pytest.mark.parametrize("chunks", [(77,), (200,)])  # a wave of keys per workgroup, and the keys split over waves
-@pytest.mark.parametrize("what", ["collapsed head", "collapsed keys", "large value"])
+@pytest.mark.parametrize("what", ["collapsed head", "collapsed keys", "large value", "uneven columns"])
 def test_score_range(oracle_lib, what, chunks):
     """A head whose queries and keys are 1e-20 (its scores are 0: uniform
-    attention), one whose keys alone are, and a value column of 1e29 that c_proj
-    brings back to 1 (past the bounds: the f32 kernels run)."""
+    attention), one whose keys alone are, a value column of 1e29 that c_proj
+    brings back to 1 (past the bounds: the f32 kernels run), and a head with a
+    query column 2^24 times the others whose keys are that much smaller, and the
+    other way round."""
     def change(sd):
         w, b = sd["h.0.attn.c_attn.weight"], sd["h.0.attn.c_attn.bias"]
+        if what == "uneven columns":
+            for c, f in ((64, 2.0 ** 24), (70, 2.0 ** -24)):
+                for col, g in ((c, f), (192 + c, 1 / f)):
+                    w[:, col] *= g
+                    b[col] *= g
+            return
         if what == "large value":
             b[2 * 192 + 64] = 1e29
             sd["h.0.attn.c_proj.weight"][64] *= 1e-29
