@@ -109,12 +109,11 @@ def cpu_baseline(sd, sh, prompt, n_decode, all_threads, what):
     return out
 
 
-MFMA_FP32_PEAK_TFLOPS = 157.3
-# dense bf16 MFMA peak; a GEMM with bf16 weights runs each f32 product as
-# three exact bf16 MFMA products (the activation split into three bf16
-# parts), so its peak in f32 flops is a third of it
-MFMA_BF16_PEAK_TFLOPS = 2500.0
-BF16X3_PEAK_TFLOPS = MFMA_BF16_PEAK_TFLOPS / 3
+# dense 16-bit MFMA peak; the prefill's GEMMs run each f32 product as f16
+# products of pairs, three with f32 weights and two with bf16 weights, so their
+# peak in f32 flops is a third or a half of it
+MFMA_F16_PEAK_TFLOPS = 2500.0
+PAIR_PRODUCTS = {4: 3, 2: 2}  # by bytes per weight
 PREFILL_WORKLOADS = {
     # name: (shape, batch, tokens): forward_cached on an empty cache, prompts read without their logits
     "c4": ("large", 32, 1024),
@@ -158,6 +157,7 @@ def run_prefill(a):
     step_s = float(np.mean(times))
     flops = prefill_flops(sh, B, T, 0)
     achieved = flops / step_s / 1e12
+    peak = MFMA_F16_PEAK_TFLOPS / PAIR_PRODUCTS[4]
     out = {
         "metric": f"prefill tokens/s (GPT-2 {shape_name} b={B}, {T} tokens)",
         "value": round(B * T / step_s, 1),
@@ -169,10 +169,9 @@ def run_prefill(a):
         "data": "synthetic: seeded N(0,0.02) random-init weights, uniform random token ids",
         "config": {"workload": f"{a.workload}: GPT-2 {shape_name}, batch {B}, prefill {T} tokens, no logits",
                    "batch": B, "tokens": T, "weights": "f32"},
-        "roofline": {"bound": "mfma", "kernel": "whole prefill (pair_gemm_kernel dominant: f32 products as three f16 MFMA products; "
-                               "frac is of the f32 MFMA peak)",
-                     "achieved": round(achieved, 2), "peak": MFMA_FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(achieved / MFMA_FP32_PEAK_TFLOPS, 4), "flops_per_step": flops,
+        "roofline": {"bound": "mfma", "mfma": "f16x3", "kernel": "whole prefill (pair_gemm_kernel dominant)",
+                     "achieved": round(achieved, 2), "peak": round(peak, 1), "unit": "TFLOP/s",
+                     "frac": round(achieved / peak, 4), "flops_per_step": flops,
                      "traffic": None},
     }
     if not a.no_cpu:
@@ -213,22 +212,20 @@ def prefill_bytes(sh, B, T, wbytes, head_rows=None):
 
 def prefill_roofline(sh, B, T, wbytes, ms, head_rows=None):
     """Roofline of the prefill leg: HBM when its arithmetic intensity is
-    below the MFMA ridge (peak / 8 TB/s), MFMA otherwise. The peak is fp32
-    MFMA for f32 weights and a third of the dense bf16 MFMA rate for bf16
-    weights (three 16-bit products per f32 product, mfma "bf16x3"). The
-    GEMMs run on f16 pairs, three (bf16 weights: two) f16 products per f32
-    product, so long f32 prompts exceed the fp32 MFMA peak."""
+    below the MFMA ridge (peak / 8 TB/s), MFMA otherwise. The peak is that of
+    the f16-pair GEMMs: the dense f16 MFMA rate over the f16 products per f32
+    product (mfma "f16x3" with f32 weights, "f16x2" with bf16 weights)."""
     flops = prefill_flops(sh, B, T, head_rows)
     nbytes = prefill_bytes(sh, B, T, wbytes, head_rows)
     s = ms / 1e3
-    bf16 = wbytes == 2
-    peak = BF16X3_PEAK_TFLOPS if bf16 else MFMA_FP32_PEAK_TFLOPS
+    products = PAIR_PRODUCTS[wbytes]
+    peak = MFMA_F16_PEAK_TFLOPS / products
     if flops / nbytes < peak * 1e12 / (HBM_PEAK_GBS * 1e9):
         ach = nbytes / s / 1e9
         return {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(ach / HBM_PEAK_GBS, 4), "bytes": int(nbytes), "ms": round(ms, 4)}
     ach = flops / s / 1e12
-    return {"bound": "mfma", "mfma": "bf16x3" if bf16 else "fp32", "achieved": round(ach, 2),
+    return {"bound": "mfma", "mfma": f"f16x{products}", "achieved": round(ach, 2),
             "peak": round(peak, 1), "unit": "TFLOP/s", "frac": round(ach / peak, 4), "flops": int(flops),
             "ms": round(ms, 4)}
 

@@ -99,6 +99,11 @@ __global__ __launch_bounds__(256) void pair_row_scale_kernel(const void* __restr
   if (lane == 0) scale[n] = scale_of(sqrt((double)K * sq) + fabs(c + (double)bias[n]), bad);
 }
 
+// The k-tiles (of 32) whose weights are stored negated, of a row's nkt: the two
+// middle quarters (see pair_gemm_kernel).
+__device__ __forceinline__ int flip_begin(int nkt) { return nkt / 4; }
+__device__ __forceinline__ int flip_end(int nkt) { return nkt - nkt / 4; }
+
 // One wave per row: the row's largest |W / in_scale|, then the scaled pairs.
 // Scales are powers of two, so the products are exact; a row whose largest
 // entry is outside [2^-90, 2^90] sets *bad.
@@ -133,7 +138,8 @@ __global__ __launch_bounds__(256) void pair_weights_kernel(const void* __restric
   if (lane == 0) out_scale[n] = ldexpf(1.f, e - 15);
   for (int k = lane * 4; k < K; k += 256) {
     const float4 v = load(k);
-    const float4 y = make_float4(v.x * r, v.y * r, v.z * r, v.w * r);
+    const float f = (k >> 5) >= flip_begin(K >> 5) && (k >> 5) < flip_end(K >> 5) ? -r : r;
+    const float4 y = make_float4(v.x * f, v.y * f, v.z * f, v.w * f);
     if (planes == 2)
       pair_store4(out, n, k, K, y);
     else
@@ -159,6 +165,11 @@ __device__ __forceinline__ void wait_barrier() {
 }
 
 __device__ __forceinline__ f16x8 lds_frag(const char* p) { return *reinterpret_cast<const f16x8*>(p); }
+// v with every element's sign bit flipped where sign is 0x80008000.
+__device__ __forceinline__ f16x8 signed_frag(const f16x8& v, unsigned sign) {
+  const uint4 u = __builtin_bit_cast(uint4, v);
+  return __builtin_bit_cast(f16x8, make_uint4(u.x ^ sign, u.y ^ sign, u.z ^ sign, u.w ^ sign));
+}
 
 struct Out {
   const float* bias;
@@ -213,6 +224,18 @@ __device__ __forceinline__ void put(const Out& o, int M, int N, int m, int n, fl
   else *cp = *cp + (v + bv);
 }
 
+// Signs: an MFMA rounds the small terms of its sum towards minus infinity, so
+// cross products accumulated onto a large sum leave every output short by the
+// same amount (16368 x 3840 x 1280: 3.1e-8 of its root mean square, 0.077 of the
+// error's standard deviation), which an average over a thousand keys keeps while
+// it shrinks every other error. The weights of the two middle quarters of k are
+// therefore stored negated and the sum changes sign with them: the bias there
+// takes back that of the outer quarters (the sums grow like the square root of
+// k, so + - - + leaves a twentieth): now below 0.001, for 0.8% of the time (a
+// change of sign every 4 k-tiles: 2.6%; operands negated in registers: 6%).
+// DUAL's cross products meet small sums only (0.004 without this): those tiles
+// take the weights' signs back.
+//
 // WM x WN waves, each MI x NJ blocks of 32 x 32; PW weight planes; NS stages.
 // KW = 2: twice the waves, each pair sharing its blocks and taking one half
 // of every k-tile. DUAL: the cross products hi lo + lo hi have their own
@@ -316,8 +339,19 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void pair_gemm_kernel(const uint
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p)
     if (p < nk) issue(p, p);
+  auto negate = [&]() {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          acc[i][j][e] = -acc[i][j][e];
+        }
+  };
+  const int kt0 = z * nk, neg0 = flip_begin(K / 32) - kt0, neg1 = flip_end(K / 32) - kt0;
   int st = 0;
-  for (int kt = 0; kt < nk; ++kt) {
+  auto tile = [&](int kt) {
     // tile kt has landed once only the loads of the NS - 2 later tiles are
     // outstanding; past the barrier that holds for every wave, and no wave
     // reads the stage that is filled next any more
@@ -325,6 +359,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void pair_gemm_kernel(const uint
     else wait_barrier<0>();
     if (kt + NS - 1 < nk) issue(kt + NS - 1, st == 0 ? NS - 1 : st - 1);
     const char* sp = lds + st * T::STAGE;
+    const unsigned sign = DUAL && kt >= neg0 && kt < neg1 ? 0x80008000u : 0u;
 #pragma unroll
     for (int s0 = 0; s0 < 2; s0 += KW) {
       const int s = KW == 2 ? kz : s0;
@@ -332,7 +367,10 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void pair_gemm_kernel(const uint
 #pragma unroll
       for (int p = 0; p < PW; ++p)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) w[p][j] = lds_frag(sp + (KW == 2 ? wrz[p] : wrd[p][s0]) + j * 32 * 64 * PW);
+        for (int j = 0; j < NJ; ++j) {
+          w[p][j] = lds_frag(sp + (KW == 2 ? wrz[p] : wrd[p][s0]) + j * 32 * 64 * PW);
+          if (DUAL) w[p][j] = signed_frag(w[p][j], sign);
+        }
 #pragma unroll
       for (int p = 0; p < 2; ++p)
 #pragma unroll
@@ -355,6 +393,18 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void pair_gemm_kernel(const uint
       }
     }
     st = st + 1 == NS ? 0 : st + 1;
+  };
+  if constexpr (DUAL) {
+    for (int kt = 0; kt < nk; ++kt) tile(kt);
+  } else {
+    // the three runs of equal sign, as far as this split has k-tiles of them
+    int kt = 0;
+#pragma unroll 1
+    for (int run = 0; run < 3; ++run) {
+      const int end = run == 2 ? nk : min(nk, run == 0 ? neg0 : neg1);
+      for (; kt < end; ++kt) tile(kt);
+      if (run < 2) negate();
+    }
   }
 
   if constexpr (DUAL) {

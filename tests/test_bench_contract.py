@@ -79,10 +79,11 @@ def test_prefill_flops_small_case_by_brute_force():
 def test_prefill_roofline_bound_and_peak():
     sh = synth.SHAPES["large"]
     r = bench.prefill_roofline(sh, 32, 1024, 4, 420.0)
-    assert r["bound"] == "mfma" and r["mfma"] == "fp32" and r["peak"] == bench.MFMA_FP32_PEAK_TFLOPS
+    assert r["bound"] == "mfma" and r["mfma"] == "f16x3"
+    assert r["peak"] == pytest.approx(bench.MFMA_F16_PEAK_TFLOPS / 3, rel=1e-3)
     assert r["frac"] == pytest.approx(bench.prefill_flops(sh, 32, 1024) / 0.42 / 1e12 / r["peak"], rel=1e-3)
     r16 = bench.prefill_roofline(synth.SHAPES["xl"], 16, 64, 2, 16.0)
-    assert r16["mfma"] == "bf16x3" and r16["peak"] == pytest.approx(bench.MFMA_BF16_PEAK_TFLOPS / 3, rel=1e-3)
+    assert r16["mfma"] == "f16x2" and r16["peak"] == pytest.approx(bench.MFMA_F16_PEAK_TFLOPS / 2, rel=1e-3)
     small = bench.prefill_roofline(synth.SHAPES["small"], 1, 4, 4, 0.5)
     assert small["bound"] == "hbm" and small["peak"] == bench.HBM_PEAK_GBS
 
