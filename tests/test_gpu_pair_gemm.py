@@ -190,3 +190,34 @@ def test_models_outside_the_bounds(oracle_lib, what):
     fine = np.isfinite(ref)
     assert np.all(np.abs(got[fine] - ref[fine]) <= 1e-3 + 1e-4 * np.abs(ref[fine]))
     m.close()
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+def test_no_bias(storage):
+    """The largest tiles' rounding errors have no common part (small terms are
+    rounded towards minus infinity when an MFMA adds them to a large sum): the
+    mean error of the first layer's keys and values, in units of the errors'
+    deviation, is what the mean of as many independent errors shows, 6 standard
+    deviations of it, plus 0.01 (without the weights' signs: -0.042 and -0.059)."""
+    d, heads, V, batch, (n,) = MANY_ROWS
+    sh = synth.ModelShape(V, 512, d, 1, heads)
+    sd, m = build(sh, storage)
+    ids = np.stack([synth.make_tokens(n, V, stream=40 + b) for b in range(batch)])
+    c = m.new_cache(batch)
+    print(f"[gpu] pair gemm bias {storage}", flush=True)
+    m.forward_cached_batched(ids, c, want_logits=False)
+    errors = []
+    for b in (0, batch // 2, batch - 1):
+        x = sd["wte.weight"].astype(np.float64)[ids[b]] + sd["wpe.weight"].astype(np.float64)[:n]
+        x = ref64.layer_norm(x, sd["h.0.ln_1.weight"].astype(np.float64), sd["h.0.ln_1.bias"].astype(np.float64),
+                             sh.layer_norm_epsilon)
+        kv = x @ sd["h.0.attn.c_attn.weight"].astype(np.float64) + sd["h.0.attn.c_attn.bias"].astype(np.float64)
+        for h in range(heads):
+            for values in (False, True):
+                col = d * (1 + values) + 64 * h
+                errors.append(c.read(0, h, b, values=values) - kv[:, col:col + 64])
+    e = np.stack(errors)
+    print(f"  mean {e.mean() / e.std():.4f} of the deviation, {e.size} errors", flush=True)
+    assert abs(e.mean()) / e.std() <= 6 / np.sqrt(e.size) + 0.01
+    c.close()
+    m.close()
