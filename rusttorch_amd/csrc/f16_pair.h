@@ -1,6 +1,7 @@
 // f32 values as pairs of f16 (hi + lo) scaled by powers of two, for f16 MFMAs
 // that compute f32 products: hi = f16(v), lo = f16(v - hi), so hi + lo is v to
-// 2^-23 or better wherever |v| >= 2^-2, and to an absolute 2^-25 below.
+// 2^-23 or better (one bit short of f32 for a quarter of the values) wherever
+// |v| >= 2^-2, and to an absolute 2^-25 below.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

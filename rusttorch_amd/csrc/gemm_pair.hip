@@ -4,15 +4,16 @@
 // of f16, hi + lo, scaled by powers of two (f16_pair.h), and a product is
 // hi hi + hi lo + lo hi: three f16 MFMAs per f32 product, each exact in the
 // f32 accumulator's input (11 x 11 bits), so the rounding left is the pair's
-// own (2^-24 of a value in the mean) and the accumulator's, which takes 16
+// own (2^-24 of a value in the mean, 2^-23 at worst; the dropped lo lo 2^-24 and
+// 2^-22 of a product) and the accumulator's, which takes 16
 // products per rounding instead of 2. bf16 weights fit one f16: two MFMAs.
 // The scales are fixed when the model is loaded, from bounds that hold for
 // every input (gemm_pair.h), so no value overflows f16.
 //
 // What bounds it: at 16368 x 5120 x 1280 the 256 x 256 tile runs at 378-385
 // TFLOP/s of f32 products, 1.15 PFLOP/s of f16 MFMA, what a library f16 GEMM
-// reaches on this card (8192^3: 1.09); the f32-MFMA kernel it replaced ran at
-// 126 (157 peak) and was further from 64 bits (6.6e-7 against 3.9e-7 relative
+// reaches on this card (8192^3: 1.09); the f32-MFMA kernel runs at
+// 126 (157 peak) and is further from 64 bits (6.6e-7 against 3.9e-7 relative
 // at K = 1280, 1.24e-6 against 8.0e-7 at 5120). At a few hundred rows the
 // launch, the first loads and the chain of k-tiles bound it (gemm_pair_choice.h).
 //
@@ -23,7 +24,8 @@
 // rows span them, so the swizzle is row / 2 (row / 4 for 64-byte rows). By the
 // row itself every read took twice its cycles (SQ_LDS_BANK_CONFLICT 6.9e7 per
 // dispatch of 32768 x 1280 x 3840-5120, now 0): 1.66e7 -> 1.64e7 cycles, the
-// 128 x 128 tiles 1.28e7 -> 1.26e7; the MFMAs' power sets the time.
+// 128 x 128 tiles 1.28e7 -> 1.26e7. By the counters the MFMAs are busy half of
+// the cycles, at about 1.9 GHz; what takes the other half is not pinned down.
 #include "gemm_pair.h"
 
 #include <algorithm>

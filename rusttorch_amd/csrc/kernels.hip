@@ -1,6 +1,7 @@
 // gfx950 kernels for the GPT-2 token loop: embedding, LayerNorm, decode GEMV
 // with fused epilogues, attention over the KV cache (decode and causal
-// prefill), argmax, and an fp32 MFMA GEMM for prefill.
+// prefill), argmax, and fp32 MFMA GEMMs for prefill (gemm_pair.hip and
+// attn_pair.hip hold the f16-pair forms that most prompts run).
 //
 // Each kernel states the reference function it computes (file:line in
 // rusttorch-core/src/nn/gpt2.rs). Arithmetic is fp32 throughout; weights may
