@@ -110,6 +110,8 @@ struct HostStages {
   static constexpr size_t kKeep = 4;
   std::mutex mu;
   std::vector<std::pair<int, std::unique_ptr<HostStage>>> idle;  // by device
+  // Null where there is no page-locked memory to be had (test hook
+  // RTG_TEST_PINNED_FAIL=1).
   std::unique_ptr<HostStage> take(int device) {
     {
       std::lock_guard<std::mutex> g(mu);
@@ -121,7 +123,13 @@ struct HostStages {
         }
     }
     std::unique_ptr<HostStage> s(new HostStage());
-    HIPX(hipHostMalloc(reinterpret_cast<void**>(&s->mem), 2 * HostStage::kChunk + 256, hipHostMallocDefault));
+    const char* t = getenv("RTG_TEST_PINNED_FAIL");
+    if ((t && t[0] == '1') || hipHostMalloc(reinterpret_cast<void**>(&s->mem), 2 * HostStage::kChunk + 256,
+                                            hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      s->mem = nullptr;
+      return nullptr;
+    }
     for (auto& e : s->ev) HIPX(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     return s;
   }
@@ -144,8 +152,14 @@ unsigned copy_out(hipStream_t s, int device, void* dst, const void* src, size_t 
     return 0;
   }
   std::unique_ptr<HostStage> st = host_stages().take(device);
-  uint32_t* word = reinterpret_cast<uint32_t*>(st->mem + 2 * HostStage::kChunk);
   unsigned e = 0;
+  if (!st) {  // through the runtime's own staging
+    if (bytes) HIPX(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+    HIPX(hipStreamSynchronize(s));
+    if (err) HIPX(hipMemcpy(&e, err, 4, hipMemcpyDeviceToHost));
+    return e;
+  }
+  uint32_t* word = reinterpret_cast<uint32_t*>(st->mem + 2 * HostStage::kChunk);
   if (bytes <= HostStage::kChunk) {
     launch_copy_out(s, static_cast<const uint32_t*>(src), bytes / 4, err, reinterpret_cast<uint32_t*>(st->mem));
     HIPX(hipGetLastError());

@@ -9,7 +9,7 @@ import threading
 import numpy as np
 import pytest
 
-from rusttorch_amd import synth
+from rusttorch_amd import _lib, synth
 from rusttorch_amd.gpt2 import Gpt2Config, Gpt2Model
 from tests.test_zz_no_alloc import call
 
@@ -34,6 +34,19 @@ def test_every_chunk_arrives(model, n):
     assert np.array_equal(m.forward_cached(ids, a), call("rtg_forward_cached_noalloc", m, b, ids, sh.vocab_size))
     a.close()
     b.close()
+
+
+def test_no_page_locked_memory(model, monkeypatch):
+    """Results still arrive, through the runtime's own staging: one token (the
+    persistent step and its error word), the multi-row forward, several chunks."""
+    sh, m = model
+    texts = [synth.make_tokens(n, sh.vocab_size, stream=930 + n) for n in (1, 9, 50)]
+    want = [m.forward(t) for t in texts]
+    print("[gpu] host copies without page-locked memory", flush=True)
+    _lib.load().rtg_cleanup()  # the stages that calls so far left behind
+    monkeypatch.setenv("RTG_TEST_PINNED_FAIL", "1")
+    for t, w in zip(texts, want):
+        assert np.array_equal(m.forward(t), w)
 
 
 def test_threads_have_their_own_stages(model):
